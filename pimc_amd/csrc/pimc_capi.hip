@@ -389,10 +389,7 @@ bool pimc_ctx::stream_quiet() {
 
 pimc_ctx::~pimc_ctx() {
     if (stream) (void)hipStreamSynchronize(stream);
-    if (copy_stream) {
-        (void)hipStreamSynchronize(copy_stream);
-        (void)hipStreamDestroy(copy_stream);
-    }
+    pimc::dma_close(&dma);
     for (auto& e : chunk_ev)
         if (e) (void)hipEventDestroy(e);
     pimc::direct_ring_release(&dring);
@@ -661,14 +658,16 @@ int pimc_ctx_create(const pimc_desc* d, pimc_ctx** out) {
     if ((r = ctx_dalloc(c.get(), &c->d_slices, M))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_walker, 1))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_vslice, M))) return r;
-    if ((r = ctx_dalloc(c.get(), &c->d_out, 16))) return r;
+    if ((r = ctx_dalloc(c.get(), &c->d_out, 32))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_hist, 64))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_kin_partials, 1024))) return r;
-    if ((r = ctx_halloc(c.get(), &c->h_stage, std::max<size_t>(3 * (size_t)M * N, 256)))) return r;
+    c->cap_stage = std::max<size_t>(3 * (size_t)M * N, 256);
+    if ((r = ctx_halloc(c.get(), &c->h_stage, c->cap_stage))) return r;
     if ((r = ctx_halloc(c.get(), &c->h_out, 64))) return r;
     {
         // small results are written by the kernels straight into host memory
-        hipError_t e = hipHostMalloc((void**)&c->h_map, sizeof(double) * 64,
+        hipError_t e = hipHostMalloc((void**)&c->h_map,
+                                     sizeof(double) * (pimc_ctx::kSqSlot + pimc_ctx::kMappedSq),
                                      hipHostMallocMapped | hipHostMallocCoherent);
         if (e != hipSuccess) return fail(nullptr, PIMC_E_NOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
         c->host_allocs.push_back((void*)c->h_map);
@@ -685,6 +684,7 @@ int pimc_ctx_create(const pimc_desc* d, pimc_ctx** out) {
     }
     HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_hash, 0xff, sizeof(int) * (size_t)cells * M * N, c->stream));
     HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_numlab, 0, sizeof(int) * (size_t)cells * M, c->stream));
+    HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_out, 0, sizeof(double) * 32, c->stream));
     build_grid_nn(c.get());
     HIP_OR_FAIL(c.get(), hipMemcpyAsync(c->d_grid_nn, c->grid_nn.data(), sizeof(int) * c->grid_nn.size(),
                                         hipMemcpyHostToDevice, c->stream));

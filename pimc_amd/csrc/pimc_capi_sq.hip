@@ -3,10 +3,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <string>
 #include <memory>
+#include <utility>
 #include <vector>
 
 #include "pimc_host.hpp"
@@ -51,84 +53,140 @@ int true_num_particles(pimc_ctx* c) {
     return (int)(on / c->desc.num_slices);
 }
 
-// rho_q(m) for a group of q-vectors into c->d_rho ([M][nq][2])
-// Room for nq q-vectors in both device q lists.
+// Room for nq q-vectors in the device list of the general (non-lattice) forms.
 int ensure_q(pimc_ctx* c, int nq) {
+    size_t cap = (size_t)c->cap_q;
+    const int r = grow(c, &c->d_q, &cap, (size_t)nq * 3);
+    if (!r) c->cap_q = (int)cap;
+    return r;
+}
+
+// The plan of a lattice q list on the device, one copy from pinned memory.
+struct DevPlan {
+    const int* dst = nullptr;    // [nu][2] list rows of each mode, for F
+    RhoMatrixArgs mat{};         // matrix form
+    RhoArgs lane{};              // one lane per mode
+};
+
+int upload_plan(pimc_ctx* c, const RhoPlan& P, const std::vector<int>& n3, bool want_dst, DevPlan* D) {
+    const size_t n_rows = 2 * P.rows.size(), n_jobs = 2 * P.jobs.size(), n_slot = P.slot.size();
+    const size_t n_dst = want_dst ? 2 * (size_t)P.nu : 0, n_list = P.matrix ? 0 : 3 * (size_t)P.nu;
+    const size_t need = n_rows + n_jobs + n_slot + n_dst + n_list;
     int r;
-    size_t capq = (size_t)c->cap_q;
-    if ((size_t)nq * 3 > capq) {
-        size_t cq = capq, cn = capq;
-        if ((r = grow(c, &c->d_q, &cq, (size_t)nq * 3))) return r;
-        if ((r = grow(c, &c->d_qn, &cn, (size_t)nq * 3))) return r;
-        c->cap_q = (int)std::min(cq, cn);
+    if ((r = grow(c, &c->d_plan, &c->cap_plan, std::max<size_t>(need, 16384)))) return r;
+    // packed in the context's pinned staging block where it fits (the block holds
+    // the path, 24 M N bytes; nothing else uses it during the call)
+    std::vector<int> unpinned;
+    int* h = reinterpret_cast<int*>(c->h_stage);
+    if (sizeof(int) * need > sizeof(double) * c->cap_stage) {
+        unpinned.resize(need);
+        h = unpinned.data();
+    }
+    int* d = c->d_plan;
+    // the jobs and rows first: 8-byte records at an aligned start
+    size_t o = 0;
+    const size_t o_jobs = o;
+    if (n_jobs) std::memcpy(h + o, P.jobs.data(), sizeof(int) * n_jobs);
+    o += n_jobs;
+    const size_t o_rows = o;
+    if (n_rows) std::memcpy(h + o, P.rows.data(), sizeof(int) * n_rows);
+    o += n_rows;
+    const size_t o_slot = o;
+    if (n_slot) std::memcpy(h + o, P.slot.data(), sizeof(int) * n_slot);
+    o += n_slot;
+    const size_t o_dst = o;
+    for (int u = 0; u < (int)(n_dst / 2); ++u) {
+        h[o + 2 * (size_t)u] = P.first[u];
+        h[o + 2 * (size_t)u + 1] = P.second[u];
+    }
+    o += n_dst;
+    const size_t o_list = o;
+    for (int u = 0; u < (int)(n_list / 3); ++u)
+        for (int k = 0; k < 3; ++k) h[o + 3 * (size_t)u + k] = n3[3 * (size_t)P.first[u] + k];
+    SHIP(c, hipMemcpyAsync(d, h, sizeof(int) * need, hipMemcpyHostToDevice, c->stream));
+    if (!unpinned.empty()) SHIP(c, hipStreamSynchronize(c->stream));
+    D->dst = want_dst ? d + o_dst : nullptr;
+    if (P.matrix) {
+        RhoMatrixArgs& A = D->mat;
+        A.pos = c->d_pos;
+        A.plane = c->plane;
+        A.nalloc = c->desc.num_alloc;
+        A.num_slices = c->desc.num_slices;
+        A.nbs = c->d_nbs;
+        A.invL = 1.0 / c->desc.side;
+        for (int k = 0; k < 3; ++k) A.nmax[k] = P.nmax[k];
+        A.rows = reinterpret_cast<const int2*>(d + o_rows);
+        A.jobs = reinterpret_cast<const RhoJob*>(d + o_jobs);
+        A.job0 = 0;
+        A.job_end = (int)P.jobs.size();
+        A.slot = d + o_slot;
+        A.width = P.width;
+        A.nu = P.nu;
+        A.rho = c->d_rho;
+    } else {
+        RhoArgs& A = D->lane;
+        A.pos = c->d_pos;
+        A.plane = c->plane;
+        A.nalloc = c->desc.num_alloc;
+        A.num_slices = c->desc.num_slices;
+        A.nbs = c->d_nbs;
+        A.invL = 1.0 / c->desc.side;
+        A.nq = P.nu;
+        A.qn = d + o_list;
+        for (int k = 0; k < 3; ++k) A.nmax[k] = P.nmax[k];
+        A.rho = c->d_rho;
     }
     return PIMC_OK;
 }
 
-// The density-mode arguments of the context's worldlines for nq q-vectors,
-// modes into c->d_rho; for lattice q, qn (host, nq x 3) sets the phasor ranges.
-RhoArgs rho_args(pimc_ctx* c, int nq, const int* qn) {
-    RhoArgs A{};
-    A.pos = c->d_pos;
-    A.plane = c->plane;
-    A.nalloc = c->desc.num_alloc;
-    A.num_slices = c->desc.num_slices;
-    A.nbs = c->d_nbs;
-    A.invL = 1.0 / c->desc.side;
-    A.nq = nq;
-    A.rho = c->d_rho;
-    if (qn) {
-        int nm[3] = {0, 0, 0};
-        for (int k = 0; k < nq; ++k)
-            for (int d = 0; d < 3; ++d) nm[d] = std::max(nm[d], std::abs(qn[3 * k + d]));
-        for (int d = 0; d < 3; ++d) A.nmax[d] = nm[d];
-    }
-    return A;
+// rho_u(m) of the plan's modes into c->d_rho [M][nu][2]
+int lattice_rho(pimc_ctx* c, const RhoPlan& P, const std::vector<int>& n3, bool want_dst, DevPlan* D) {
+    int r;
+    if ((r = grow(c, &c->d_rho, &c->cap_rho, (size_t)c->desc.num_slices * P.nu * 2))) return r;
+    if ((r = upload_plan(c, P, n3, want_dst, D))) return r;
+    c->timed_begin(2);
+    SHIP(c, P.matrix ? launch_rho_matrix(c->stream, D->mat) : launch_rho(true, c->stream, D->lane));
+    c->timed_end();
+    return PIMC_OK;
 }
 
-int compute_rho(pimc_ctx* c, bool lattice, const std::vector<int>& qn, const std::vector<double>& qv, int nq) {
+// rho_q(m) of general q into c->d_rho [M][nq][2]
+int general_rho(pimc_ctx* c, const std::vector<double>& qv, int nq) {
     const int M = c->desc.num_slices;
     int r;
     if ((r = ensure_q(c, nq))) return r;
     if ((r = grow(c, &c->d_rho, &c->cap_rho, (size_t)M * nq * 2))) return r;
-    RhoArgs A = rho_args(c, nq, lattice ? qn.data() : nullptr);
-    if (lattice) {
-        SHIP(c, hipMemcpyAsync(c->d_qn, qn.data(), sizeof(int) * 3 * nq, hipMemcpyHostToDevice, c->stream));
-        A.qn = c->d_qn;
-    } else {
-        SHIP(c, hipMemcpyAsync(c->d_q, qv.data(), sizeof(double) * 3 * nq, hipMemcpyHostToDevice, c->stream));
-        A.q = c->d_q;
-    }
+    RhoArgs A{};
+    A.pos = c->d_pos;
+    A.plane = c->plane;
+    A.nalloc = c->desc.num_alloc;
+    A.num_slices = M;
+    A.nbs = c->d_nbs;
+    A.invL = 1.0 / c->desc.side;
+    A.nq = nq;
+    A.q = c->d_q;
+    A.rho = c->d_rho;
+    SHIP(c, hipMemcpyAsync(c->d_q, qv.data(), sizeof(double) * 3 * nq, hipMemcpyHostToDevice, c->stream));
     c->timed_begin(2);
-    SHIP(c, launch_rho(lattice, c->stream, A));
+    SHIP(c, launch_rho(false, c->stream, A));
     c->timed_end();
     return PIMC_OK;
 }
 
 // F(q, tau) of a long lattice q list written straight into page-locked memory:
-// the list runs in chunks, each chunk's density modes and lags on the context's
-// stream, and each chunk's rows are copied out on a second stream while the
-// next chunk computes (100 401 q x 250 lags make a 200 MB result whose copy
-// takes ~6 ms after ~18 ms of kernels).  A q's modes and lags come from the same
-// expressions whatever q share its launch, so the values are those of the
-// one-launch path bit for bit.
-// q per chunk: at 100 401 q x 250 lags, chunks of 34 000 / 25 600 / 18 432 q
-// took 22.0 / 22.2 / 22.6 ms against 23.9 ms in one launch (interleaved), and
-// 14 400 (4 q per lane in k_rho_lattice) 28.5 ms; chunks on two alternating
-// streams with a mode buffer each were no faster (22.2 / 22.5 / 22.8 ms)
-constexpr int kIsfChunkQ = 34000;                  // 8 q per lane in k_rho_lattice from M = 121 on
-constexpr int kIsfChunkMinQ = 1024;                // shorter lists: one launch per kernel
-constexpr size_t kIsfChunkMinBytes = 4u << 20;     // smaller results: one launch per kernel
-constexpr int kIsfChunksMax = 64;
+// the modes run in pieces of row tiles, each piece's modes and lags on the
+// context's stream, and the list rows it completes are copied out while the next
+// piece computes.  A mode's sums do not depend on what
+// shares its launch, so the values are those of the one-launch path bit for bit.
+// 100 401 q x 250 lags are 200 MB, 3.5 ms at the 57 GB/s the link gives, beside
+// 2.8 ms of kernels; S(q) and F of that list took 39.6 ms together and now take
+// 7.6 ms, F of 5377 q x 167 (one piece) 392 us and now 256 us.
+constexpr int kIsfPieceMinQ = 2048;                // shorter lists: one copy
+constexpr size_t kIsfPieceMinBytes = 4u << 20;     // smaller results: one copy
+constexpr int kIsfPiecesMax = 16;
 
-// q per chunk: lists of up to two chunks of kIsfChunkQ run as two halves
-// (5377 q x 167 lags: 7.2 MB, whose copy is half the one-launch wall)
-int isf_chunk_q(int n) {
-    return n > 2 * kIsfChunkQ ? std::max(kIsfChunkQ, (n + kIsfChunksMax - 1) / kIsfChunksMax) : (n + 1) / 2;
-}
-
-bool isf_chunks_pay(pimc_ctx* c, int n, int M, const double* fqt) {
-    if (n < 2 * kIsfChunkMinQ || (size_t)n * M * sizeof(double) < kIsfChunkMinBytes) return false;
+bool isf_pieces_pay(pimc_ctx* c, int n, int M, const double* fqt) {
+    if (n < kIsfPieceMinQ || (size_t)n * M * sizeof(double) < kIsfPieceMinBytes) return false;
     // a timed call keeps one launch per kernel, so its durations stay per call
     if (c->timing && (c->timing_kinds & ((1u << 2) | (1u << 4)))) return false;
     // a pageable destination is copied through staging with the host waiting
@@ -138,42 +196,111 @@ bool isf_chunks_pay(pimc_ctx* c, int n, int M, const double* fqt) {
     return e == hipSuccess && at.type == hipMemoryTypeHost;
 }
 
-int isf_lattice_chunked(pimc_ctx* c, const std::vector<int>& qn, int n, int M, double inv_n, double* fqt) {
-    const int per = isf_chunk_q(n);
-    const int chunks = (n + per - 1) / per;
+// What pimc_kernel_time counts as "isf_chunks": the q of such a call in parts of
+// 34 000, at least two.
+int isf_parts(int n) { return std::max(2, (n + 33999) / 34000); }
+
+// The list rows of modes [u0, u_end) as at most two runs {first row, rows}: their
+// first q and their second q (those of -q), each a run when the rows named are
+// consecutive (in either direction), which a list in the reference's order
+// gives.  False when they are not.
+bool isf_runs(const RhoPlan& P, int u0, int u_end, std::pair<int, int> run[2]) {
+    const std::vector<int>* by[2] = {&P.first, &P.second};
+    for (int s = 0; s < 2; ++s) {
+        int lo = INT_MAX, hi = -1, cnt = 0;
+        for (int u = u0; u < u_end; ++u) {
+            const int k = (*by[s])[u];
+            if (k < 0) continue;
+            lo = std::min(lo, k);
+            hi = std::max(hi, k);
+            ++cnt;
+        }
+        if (cnt && hi - lo + 1 != cnt) return false;   // the rows of distinct modes are distinct
+        run[s] = {cnt ? lo : 0, cnt};
+    }
+    return true;
+}
+
+int isf_lattice_pieces(pimc_ctx* c, const RhoPlan& P, const std::vector<int>& n3, int n, int M, double inv_n,
+                        double* fqt) {
     int r;
-    if ((r = ensure_q(c, n))) return r;
-    if ((r = grow(c, &c->d_rho, &c->cap_rho, (size_t)M * per * 2))) return r;
+    if ((r = grow(c, &c->d_rho, &c->cap_rho, (size_t)M * P.nu * 2))) return r;
     if ((r = grow(c, &c->d_fqt, &c->cap_fqt, (size_t)n * M))) return r;
-    if (!c->copy_stream) SHIP(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
-    while ((int)c->chunk_ev.size() < chunks) {
+    DevPlan D;
+    if ((r = upload_plan(c, P, n3, true, &D))) return r;
+    const int pieces = (int)P.piece_modes.size();
+    while ((int)c->chunk_ev.size() < pieces) {
         hipEvent_t ev = nullptr;
         SHIP(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         c->chunk_ev.push_back(ev);
     }
-    SHIP(c, hipMemcpyAsync(c->d_qn, qn.data(), sizeof(int) * 3 * (size_t)n, hipMemcpyHostToDevice, c->stream));
     hipError_t e = hipSuccess;
-    for (int k = 0; k < chunks && e == hipSuccess; ++k) {
-        const int off = k * per, nc = std::min(per, n - off);
-        RhoArgs A = rho_args(c, nc, qn.data() + 3 * (size_t)off);
-        A.qn = c->d_qn + 3 * (size_t)off;
-        double* rows = c->d_fqt + (size_t)off * M;
-        // the chunk's modes overwrite d_rho after the previous chunk's lags (one stream)
-        e = launch_rho(true, c->stream, A);
-        if (e == hipSuccess) e = launch_isf(c->stream, c->d_rho, nc, M, inv_n, rows, 0);
+    int u0 = 0;
+    std::vector<std::pair<int, int>> runs;   // two per piece
+    bool late = false;                       // rows left for one copy at the end
+    for (int k = 0; k < pieces && e == hipSuccess; ++k) {
+        RhoMatrixArgs A = D.mat;
+        A.job0 = P.piece_job[k];
+        A.job_end = P.piece_job[k + 1];
+        e = launch_rho_matrix(c->stream, A);
+        const int u1 = P.piece_modes[k];
+        if (e == hipSuccess) e = launch_isf(c->stream, c->d_rho, P.nu, u0, u1, M, inv_n, D.dst, c->d_fqt);
         if (e == hipSuccess) e = hipEventRecord(c->chunk_ev[k], c->stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(c->copy_stream, c->chunk_ev[k], 0);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(fqt + (size_t)off * M, rows, sizeof(double) * (size_t)nc * M, hipMemcpyDeviceToHost,
-                               c->copy_stream);
-        if (e == hipSuccess) ++c->isf_chunks;
+        std::pair<int, int> run[2];
+        late = late || !isf_runs(P, u0, u1, run);
+        runs.insert(runs.end(), run, run + 2);
+        u0 = u1;
     }
-    // both streams end quiet, after an error too (no copy may land later)
-    const hipError_t e1 = hipStreamSynchronize(c->copy_stream);
-    const hipError_t e2 = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = e1 != hipSuccess ? e1 : e2;
-    if (e != hipSuccess) return sfail(c, PIMC_E_HIP, std::string("F(q,tau) in chunks: ") + hipGetErrorString(e));
+    // the copies go to the DMA engines, which leave the compute units to the next
+    // piece (copy kernels on a second stream slowed the pieces 1.7 times at 100 401
+    // q); the host, which would only wait, starts each piece's once the piece's
+    // event has passed
+    const bool dma = e == hipSuccess && !late && dma_open(&c->dma, c->d_fqt, fqt);
+    bool moved = dma;
+    if (dma) {
+        for (int k = 0; k < pieces && moved && e == hipSuccess; ++k) {
+            while ((e = hipEventQuery(c->chunk_ev[k])) == hipErrorNotReady) __builtin_ia32_pause();
+            for (int s = 0; s < 2 && moved && e == hipSuccess; ++s) {
+                const std::pair<int, int>& r2 = runs[2 * k + s];
+                if (r2.second)
+                    moved = dma_start(&c->dma, fqt + (size_t)r2.first * M, c->d_fqt + (size_t)r2.first * M,
+                                      sizeof(double) * (size_t)r2.second * M);
+            }
+        }
+        (void)hipGetLastError();   // hipErrorNotReady is no error
+        moved = dma_wait(&c->dma) && moved;
+    }
+    if (e == hipSuccess && !moved)
+        e = hipMemcpyAsync(fqt, c->d_fqt, sizeof(double) * (size_t)n * M, hipMemcpyDeviceToHost, c->stream);
+    // the stream ends quiet, after an error too (no copy may land later)
+    const hipError_t e1 = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = e1;
+    if (e != hipSuccess) return sfail(c, PIMC_E_HIP, std::string("F(q,tau) in pieces: ") + hipGetErrorString(e));
+    c->isf_chunks += isf_parts(n);
     return PIMC_OK;
+}
+
+// The rows of a list's repeated q, from the rows of the modes' first q.
+void isf_repeats(const RhoPlan& P, int M, double* rows) {
+    for (int k : P.repeat)
+        std::memcpy(rows + (size_t)k * M, rows + (size_t)P.first[P.mode[k]] * M, sizeof(double) * M);
+}
+
+// A list with nl lattice q among its nq, split: an all-lattice list keeps its
+// order (idx_l empty, n3 as it is); otherwise the lattice q's components move to
+// the front of n3 and idx_l / idx_g list both kinds' places.
+void split_list(const double* q, int nq, int nl, const std::vector<uint8_t>& lat, std::vector<int>& n3,
+                std::vector<int>& idx_l, std::vector<int>& idx_g, std::vector<double>& qg) {
+    if (nl == nq) return;
+    for (int k = 0; k < nq; ++k) {
+        if (lat[k]) {
+            for (int d = 0; d < 3; ++d) n3[3 * idx_l.size() + d] = n3[3 * (size_t)k + d];
+            idx_l.push_back(k);
+        } else {
+            idx_g.push_back(k);
+            qg.insert(qg.end(), q + 3 * (size_t)k, q + 3 * (size_t)k + 3);
+        }
+    }
 }
 
 }  // namespace
@@ -185,12 +312,169 @@ bool lattice_q(const double* q, double L, int* n3) {
     for (int d = 0; d < 3; ++d) {
         const double x = q[d] * f;
         const double r = std::nearbyint(x);
-        if (std::fabs(r) > rho_max_nmax()) return false;
+        if (!(std::fabs(r) <= rho_max_nmax())) return false;
         const double back = r * 2.0 * M_PI / L;
         if (std::fabs(back - q[d]) > 1e-9 * std::max(1.0, std::fabs(q[d]))) return false;
         n3[d] = (int)r;
     }
     return true;
+}
+
+int lattice_qs(const double* q, int nq, double L, std::vector<int>& n3, std::vector<uint8_t>& lat) {
+    // blocks whose components all lie well inside lattice_q's tolerance (straight
+    // arithmetic the compiler vectorises: round to nearest by adding and taking
+    // away 1.5 2^52, no division) need no second look
+    constexpr int kBlock = 64;
+    n3.resize(3 * (size_t)nq);
+    lat.resize(nq);
+    std::memset(lat.data(), 1, (size_t)nq);
+    const double f = L / (2.0 * M_PI), g = 2.0 * M_PI / L, top = rho_max_nmax();
+    constexpr double kRound = 6755399441055744.0;
+    int count = 0;
+    for (int k0 = 0; k0 < nq; k0 += kBlock) {
+        const int n = 3 * std::min(kBlock, nq - k0);
+        const double* s = q + 3 * (size_t)k0;
+        int* o = n3.data() + 3 * (size_t)k0;
+        double rr[3 * kBlock];
+        int sure = 1;
+        for (int t = 0; t < n; ++t) {
+            const double r = (s[t] * f + kRound) - kRound;
+            rr[t] = r;
+            // NaN fails both
+            sure &= (int)(std::fabs(r) <= top) & (int)(std::fabs(r * g - s[t]) <= 0.5e-9);
+        }
+        if (sure) {
+            for (int t = 0; t < n; ++t) o[t] = (int)rr[t];
+            count += n / 3;
+            continue;
+        }
+        for (int k = 0; k < n / 3; ++k) {
+            const bool ok = lattice_q(s + 3 * k, L, o + 3 * k);
+            lat[k0 + k] = ok;
+            count += ok;
+        }
+    }
+    return count;
+}
+
+// A 16 x 16 block of the matrix form takes the same time whatever it holds (up to
+// 512 modes, both signs of n_z), a mode of the lane form always its own.  Random
+// parts of the 100 401 q at N = 2048 x 250: at 160 modes a block the matrix form
+// took 2.01 ms against 3.68 ms, at 73 2.01 against 1.73, at 25 1.16 against 0.83
+// ms; of the 5377 q at N = 256 x 167: at 97 31.7 against 41.0 us, at 47 29.7
+// against 29.8, at 28 29.9 against 24.8 us.  With a few blocks both are a chain of
+// stages, shorter in the matrix form (one block, 14 modes: 17.7 against 19.4 us).
+constexpr int kModesPerBlock = 72, kFewBlocks = 4;
+
+// Jobs of a launch that fill the workgroups of one round: 16 waves each, one
+// workgroup per slice (k_rho_matrix), and most chips' worth of slices.
+constexpr int kPieceJobs = 16;
+
+void make_rho_plan(const int* n3, int nq, int max_pieces, RhoPlan* P) {
+    int h[3] = {0, 0, 0};
+    for (int k = 0; k < nq; ++k)
+        for (int d = 0; d < 3; ++d) h[d] = std::max(h[d], std::abs(n3[3 * (size_t)k + d]));
+    for (int d = 0; d < 3; ++d) P->nmax[d] = h[d];
+    const int wy = 2 * h[1] + 1, wz = 2 * h[2] + 1;
+    const int width = 16 * (h[2] / 16 + 1), blocks = width / 16;
+    P->width = width;
+    // modes by (n_x, n_y, n_z) of the half space, rows by (n_x, n_y)
+    P->mode_at.assign((size_t)(h[0] + 1) * wy * wz, -1);
+    P->row_at.assign((size_t)(h[0] + 1) * wy, -1);
+    P->mode.resize(nq);
+    P->first.resize(nq);
+    P->second.resize(nq);
+    P->mode_row.resize(nq);
+    P->mode_nz.resize(nq);
+    P->repeat.clear();
+    P->list_rows.clear();
+    P->row_mode.clear();   // a row's first mode
+    P->row_cols.clear();   // the 16-column blocks a row uses
+    int nu = 0;
+    for (int k = 0; k < nq; ++k) {
+        int nx = n3[3 * (size_t)k], ny = n3[3 * (size_t)k + 1], nz = n3[3 * (size_t)k + 2];
+        if (nx < 0 || (nx == 0 && (ny < 0 || (ny == 0 && nz < 0)))) {
+            nx = -nx;
+            ny = -ny;
+            nz = -nz;
+        }
+        const size_t rk = (size_t)nx * wy + (ny + h[1]);
+        int& u = P->mode_at[rk * wz + (nz + h[2])];
+        if (u < 0) {
+            u = nu++;
+            P->first[u] = k;
+            P->second[u] = -1;
+            int& r = P->row_at[rk];
+            if (r < 0) {
+                r = (int)P->list_rows.size();
+                P->list_rows.push_back(make_int2(nx, ny));
+                P->row_mode.push_back(u);
+                P->row_cols.push_back(0);
+            }
+            P->row_cols[r] |= 1 << (std::abs(nz) >> 4);
+            P->mode_row[u] = r;
+            P->mode_nz[u] = nz;
+        } else if (P->second[u] < 0) {
+            P->second[u] = k;
+        } else {
+            P->repeat.push_back(k);
+        }
+        P->mode[k] = u;
+    }
+    P->nu = nu;
+    // the pieces' rows, sorted by their blocks (stable: then in the list's order),
+    // 16 to a tile; a tile's jobs are the blocks its rows use
+    const int n_rows = (int)P->list_rows.size();
+    std::vector<int>& order = P->order;   // tile places -> rows (-1: unused)
+    int pieces = 1;
+    for (int pass = 0; pass < 2; ++pass) {
+        order.clear();
+        P->jobs.clear();
+        P->piece_job.assign(1, 0);
+        P->piece_modes.clear();
+        for (int k = 0; k < pieces; ++k) {
+            const int r0 = (int)((int64_t)n_rows * k / pieces), r1 = (int)((int64_t)n_rows * (k + 1) / pieces);
+            const size_t o0 = order.size();
+            for (int mask = (1 << blocks) - 1; mask > 0; --mask)
+                for (int r = r0; r < r1; ++r)
+                    if (P->row_cols[r] == mask) order.push_back(r);
+            while (order.size() % 16) order.push_back(-1);
+            for (size_t t = o0; t < order.size(); t += 16) {
+                int mask = 0;
+                for (int i = 0; i < 16; ++i)
+                    if (order[t + i] >= 0) mask |= P->row_cols[order[t + i]];
+                for (int c = 0; c < blocks; ++c)
+                    if (mask & (1 << c)) P->jobs.push_back({(int)(t / 16), 16 * c});
+            }
+            P->piece_job.push_back((int)P->jobs.size());
+            // the modes of the rows still to run start at the smallest first mode among them
+            int least = nu;
+            for (int r = r1; r < n_rows; ++r) least = std::min(least, P->row_mode[r]);
+            P->piece_modes.push_back(least);
+        }
+        const int want = std::min(max_pieces, ((int)P->jobs.size() + kPieceJobs - 1) / kPieceJobs);
+        if (pass || want <= 1) break;
+        pieces = want;
+    }
+    P->matrix = (int)P->jobs.size() <= kFewBlocks || (int64_t)nu >= (int64_t)kModesPerBlock * (int64_t)P->jobs.size();
+    if (!P->matrix) {
+        P->jobs.clear();
+        P->rows.clear();
+        P->slot.clear();
+        return;
+    }
+    P->rows.assign(order.size(), make_int2(0, 0));
+    P->at.resize(n_rows);
+    for (size_t t = 0; t < order.size(); ++t)
+        if (order[t] >= 0) {
+            P->rows[t] = P->list_rows[order[t]];
+            P->at[order[t]] = (int)t;
+        }
+    P->slot.assign(order.size() * 2 * width, -1);
+    for (int u = 0; u < nu; ++u) {
+        const int nz = P->mode_nz[u];
+        P->slot[((size_t)P->at[P->mode_row[u]] * 2 + (nz < 0 ? 1 : 0)) * width + std::abs(nz)] = u;
+    }
 }
 
 }  // namespace pimc
@@ -206,41 +490,53 @@ int pimc_ssf(pimc_ctx* c, const double* q, int nq, double* sq) {
     const int Np = true_num_particles(c);
     if (Np <= 0) return sfail(c, PIMC_E_STATE, "no active particles");
     const double inv_n = 1.0 / Np;
-    std::vector<int> idx_l, idx_g, qn;
+    std::vector<int>& n3 = c->q_n3;
+    std::vector<uint8_t>& lat = c->q_lat;
+    std::vector<int> idx_l, idx_g;
     std::vector<double> qg;
-    for (int k = 0; k < nq; ++k) {
-        int n3[3];
-        if (lattice_q(q + 3 * k, c->desc.side, n3)) {
-            idx_l.push_back(k);
-            qn.insert(qn.end(), n3, n3 + 3);
-        } else {
-            idx_g.push_back(k);
-            qg.insert(qg.end(), q + 3 * k, q + 3 * k + 3);
-        }
-    }
+    const int nl = lattice_qs(q, nq, c->desc.side, n3, lat);
+    split_list(q, nq, nl, lat, n3, idx_l, idx_g, qg);
     int r;
-    std::vector<double> host;
-    if (!idx_l.empty()) {
-        const int nl = (int)idx_l.size();
-        if ((r = compute_rho(c, true, qn, qg, nl))) return r;
-        if ((r = grow(c, &c->d_fqt, &c->cap_fqt, (size_t)nl))) return r;
+    if (nl) {
+        RhoPlan& P = c->plan;
+        make_rho_plan(n3.data(), nl, 1, &P);
+        DevPlan D;
+        if ((r = lattice_rho(c, P, n3, false, &D))) return r;
+        // a few thousand values go straight into mapped memory and the host spins
+        // on the kernel's completion word; more are copied
+        const bool mapped = P.nu <= pimc_ctx::kMappedSq;
+        if (!mapped && (r = grow(c, &c->d_fqt, &c->cap_fqt, (size_t)P.nu))) return r;
+        const unsigned long long seq = ++c->seq;
         c->timed_begin(3);
-        SHIP(c, launch_isf(c->stream, c->d_rho, nl, M, inv_n, c->d_fqt, 1));
+        SHIP(c, launch_ssf(c->stream, c->d_rho, P.nu, M, inv_n, mapped ? c->d_map + pimc_ctx::kSqSlot : c->d_fqt, c->d_ticket(),
+                           mapped ? c->d_done() : nullptr, seq));
         c->timed_end();
-        host.resize(nl);
-        SHIP(c, hipMemcpyAsync(host.data(), c->d_fqt, sizeof(double) * nl, hipMemcpyDeviceToHost, c->stream));
-        SHIP(c, hipStreamSynchronize(c->stream));
-        for (int k = 0; k < nl; ++k) sq[idx_l[k]] = host[k];
+        const double* got = c->h_map + pimc_ctx::kSqSlot;
+        std::vector<double> host;
+        if (mapped) {
+            if (c->wait_done(seq) != 0) {
+                // the arrival counter may have been left part-way
+                (void)hipMemsetAsync(c->d_ticket(), 0, sizeof(unsigned), c->stream);
+                return sfail(c, PIMC_E_HIP, "S(q): completion not published");
+            }
+        } else {
+            double* to = c->h_stage;
+            if ((size_t)P.nu > c->cap_stage) {
+                host.resize(P.nu);
+                to = host.data();
+            }
+            SHIP(c, hipMemcpyAsync(to, c->d_fqt, sizeof(double) * P.nu, hipMemcpyDeviceToHost, c->stream));
+            SHIP(c, hipStreamSynchronize(c->stream));
+            got = to;
+        }
+        if (idx_l.empty())
+            for (int k = 0; k < nl; ++k) sq[k] = got[P.mode[k]];
+        else
+            for (int k = 0; k < nl; ++k) sq[idx_l[k]] = got[P.mode[k]];
     }
     if (!idx_g.empty()) {
         const int ng = (int)idx_g.size();
-        size_t capq = (size_t)c->cap_q;
-        if ((size_t)ng * 3 > capq) {
-            size_t cq = capq, cn = capq;
-            if ((r = grow(c, &c->d_q, &cq, (size_t)ng * 3))) return r;
-            if ((r = grow(c, &c->d_qn, &cn, (size_t)ng * 3))) return r;
-            c->cap_q = (int)std::min(cq, cn);
-        }
+        if ((r = ensure_q(c, ng))) return r;
         if ((r = grow(c, &c->d_rho, &c->cap_rho, (size_t)ng * M))) return r;
         if ((r = grow(c, &c->d_fqt, &c->cap_fqt, (size_t)ng))) return r;
         SHIP(c, hipMemcpyAsync(c->d_q, qg.data(), sizeof(double) * 3 * ng, hipMemcpyHostToDevice, c->stream));
@@ -248,7 +544,7 @@ int pimc_ssf(pimc_ctx* c, const double* q, int nq, double* sq) {
         SHIP(c, launch_ssf_pairs(c->stream, c->d_pos, c->plane, c->desc.num_alloc, M, c->d_nbs, c->d_q, ng, c->box,
                                  c->d_rho, inv_n, c->d_fqt));
         c->timed_end();
-        host.resize(ng);
+        std::vector<double> host(ng);
         SHIP(c, hipMemcpyAsync(host.data(), c->d_fqt, sizeof(double) * ng, hipMemcpyDeviceToHost, c->stream));
         SHIP(c, hipStreamSynchronize(c->stream));
         for (int k = 0; k < ng; ++k) sq[idx_g[k]] = host[k];
@@ -265,38 +561,48 @@ int pimc_isf(pimc_ctx* c, const double* q, int nq, double* fqt) {
     const int Np = true_num_particles(c);
     if (Np <= 0) return sfail(c, PIMC_E_STATE, "no active particles");
     const double inv_n = 1.0 / Np;
+    std::vector<int>& n3 = c->q_n3;
+    std::vector<uint8_t>& lat = c->q_lat;
+    std::vector<int> idx_l, idx_g;
+    std::vector<double> qg;
+    const int nl = lattice_qs(q, nq, c->desc.side, n3, lat);
+    split_list(q, nq, nl, lat, n3, idx_l, idx_g, qg);
     for (int pass = 0; pass < 2; ++pass) {
-        std::vector<int> idx, qn;
-        std::vector<double> qg;
-        for (int k = 0; k < nq; ++k) {
-            int n3[3];
-            const bool lat = lattice_q(q + 3 * k, c->desc.side, n3);
-            if (lat != (pass == 0)) continue;
-            idx.push_back(k);
-            if (lat) qn.insert(qn.end(), n3, n3 + 3);
-            else qg.insert(qg.end(), q + 3 * k, q + 3 * k + 3);
-        }
-        if (idx.empty()) continue;
-        const int n = (int)idx.size();
+        const int n = pass == 0 ? nl : nq - nl;
+        if (n == 0) continue;
         int r;
-        if (pass == 0 && n == nq && isf_chunks_pay(c, n, M, fqt)) {
-            if ((r = isf_lattice_chunked(c, qn, n, M, inv_n, fqt))) return r;
-            continue;
+        RhoPlan& P = c->plan;
+        DevPlan D;
+        if (pass == 0) {
+            const bool pieces = n == nq && isf_pieces_pay(c, n, M, fqt);
+            make_rho_plan(n3.data(), nl, pieces ? kIsfPiecesMax : 1, &P);
+            if (pieces && P.matrix) {
+                if ((r = isf_lattice_pieces(c, P, n3, n, M, inv_n, fqt))) return r;
+                isf_repeats(P, M, fqt);
+                continue;
+            }
+            if ((r = lattice_rho(c, P, n3, true, &D))) return r;
+        } else if ((r = general_rho(c, qg, n))) {
+            return r;
         }
-        if ((r = compute_rho(c, pass == 0, qn, qg, n))) return r;
+        const int nu = pass == 0 ? P.nu : n;
+        if (pass == 1) P.repeat.clear();
         if ((r = grow(c, &c->d_fqt, &c->cap_fqt, (size_t)n * M))) return r;
         c->timed_begin(4);
-        SHIP(c, launch_isf(c->stream, c->d_rho, n, M, inv_n, c->d_fqt, 0));
+        SHIP(c, launch_isf(c->stream, c->d_rho, nu, 0, nu, M, inv_n, D.dst, c->d_fqt));
         c->timed_end();
         if (n == nq) {
             // every q in this pass, in order: straight into the caller's array
             SHIP(c, hipMemcpyAsync(fqt, c->d_fqt, sizeof(double) * n * M, hipMemcpyDeviceToHost, c->stream));
             SHIP(c, hipStreamSynchronize(c->stream));
+            isf_repeats(P, M, fqt);
             continue;
         }
         std::unique_ptr<double[]> host(new double[(size_t)n * M]);
         SHIP(c, hipMemcpyAsync(host.get(), c->d_fqt, sizeof(double) * n * M, hipMemcpyDeviceToHost, c->stream));
         SHIP(c, hipStreamSynchronize(c->stream));
+        isf_repeats(P, M, host.get());
+        const std::vector<int>& idx = pass == 0 ? idx_l : idx_g;
         for (int k = 0; k < n; ++k) std::memcpy(fqt + (size_t)idx[k] * M, host.get() + (size_t)k * M, sizeof(double) * M);
     }
     return PIMC_OK;

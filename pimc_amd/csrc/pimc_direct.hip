@@ -427,4 +427,65 @@ void direct_dispatch(DirectRing* r, const DirectKernel& k, const ArgPiece* piece
     direct_submit(r, k, slot, grid_x, block_x);
 }
 
+namespace {
+// The agent that owns the allocation p lies in, when host and device address it
+// alike (not registered or foreign memory); the agent must be of type t.
+bool plain_owner(const void* p, hsa_device_type_t t, hsa_agent_t* a) {
+    hsa_amd_pointer_info_t i{};
+    i.size = sizeof(i);
+    if (hsa_amd_pointer_info(const_cast<void*>(p), &i, nullptr, nullptr, nullptr) != HSA_STATUS_SUCCESS ||
+        i.type != HSA_EXT_POINTER_TYPE_HSA)
+        return false;
+    hsa_device_type_t got;
+    if (hsa_agent_get_info(i.agentOwner, HSA_AGENT_INFO_DEVICE, &got) != HSA_STATUS_SUCCESS || got != t) return false;
+    *a = i.agentOwner;
+    return true;
+}
+}  // namespace
+
+bool dma_open(DmaCopies* d, const void* src, const void* dst) {
+    hsa_agent_t g{}, c{};
+    if (!plain_owner(src, HSA_DEVICE_TYPE_GPU, &g) || !plain_owner(dst, HSA_DEVICE_TYPE_CPU, &c)) return false;
+    d->gpu = g.handle;
+    d->cpu = c.handle;
+    if (!d->signal) {
+        // HIP has initialised the runtime; this takes one more reference on it
+        if (hsa_init() != HSA_STATUS_SUCCESS) return false;
+        hsa_signal_t s{};
+        if (hsa_signal_create(0, 0, nullptr, &s) != HSA_STATUS_SUCCESS) {
+            (void)hsa_shut_down();
+            return false;
+        }
+        d->signal = s.handle;
+    }
+    hsa_signal_store_relaxed(hsa_signal_t{d->signal}, 0);
+    return true;
+}
+
+bool dma_start(DmaCopies* d, void* dst, const void* src, size_t bytes) {
+    const hsa_signal_t s{d->signal};
+    hsa_signal_add_relaxed(s, 1);
+    if (hsa_amd_memory_async_copy(dst, hsa_agent_t{d->cpu}, src, hsa_agent_t{d->gpu}, bytes, 0, nullptr, s) ==
+        HSA_STATUS_SUCCESS)
+        return true;
+    hsa_signal_subtract_relaxed(s, 1);
+    return false;
+}
+
+bool dma_wait(DmaCopies* d) {
+    const hsa_signal_t s{d->signal};
+    // an error sets the signal negative
+    hsa_signal_value_t v;
+    while ((v = hsa_signal_wait_scacquire(s, HSA_SIGNAL_CONDITION_LT, 1, UINT64_MAX, HSA_WAIT_STATE_ACTIVE)) > 0) {
+    }
+    return v == 0;
+}
+
+void dma_close(DmaCopies* d) {
+    if (!d->signal) return;
+    (void)hsa_signal_destroy(hsa_signal_t{d->signal});
+    (void)hsa_shut_down();
+    d->signal = 0;
+}
+
 }  // namespace pimc

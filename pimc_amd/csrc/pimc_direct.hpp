@@ -75,4 +75,19 @@ char* direct_stage(DirectRing* r, const ArgPiece* pieces, int n_pieces);
 void direct_flush(int device);
 void direct_submit(DirectRing* r, const DirectKernel& k, const char* kernargs, uint32_t grid_x, uint32_t block_x);
 
+// Copies from device to page-locked host memory on the DMA engines, outside any
+// HIP stream: the caller starts one when the data is complete (after an event or a
+// synchronisation that releases the device's caches to the system) and waits for
+// all of them before the memory is used, freed or written again.
+struct DmaCopies {
+    uint64_t signal = 0;          // hsa_signal_t: copies still running
+    uint64_t gpu = 0, cpu = 0;    // hsa_agent_t of the source and the destination
+};
+// False when src and dst are not plain HIP allocations of a GPU and of the host.
+bool dma_open(DmaCopies* d, const void* src, const void* dst);
+bool dma_start(DmaCopies* d, void* dst, const void* src, size_t bytes);
+// Waits for every copy started; false if one failed.
+bool dma_wait(DmaCopies* d);
+void dma_close(DmaCopies* d);
+
 }  // namespace pimc

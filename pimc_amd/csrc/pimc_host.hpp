@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <string>
 #include <vector>
 
@@ -24,6 +25,36 @@ double aziz_tail(const AzizParams& p, double rc);
 // q = (2 pi / L) n with integer n, |n_d| <= rho_max_nmax(): the lattice
 // wavevectors whose S(q) and F(q,tau) use the density-mode kernels.
 bool lattice_q(const double* q, double L, int* n3);
+// lattice_q of a whole list: n3 [nq][3] (where lattice), lat [nq]; returns the
+// number of lattice q.
+int lattice_qs(const double* q, int nq, double L, std::vector<int>& n3, std::vector<uint8_t>& lat);
+
+// The density modes a list of lattice q needs.  rho_{-q} is the conjugate of
+// rho_q, so q and -q (and repeats of either) share one mode; modes are numbered
+// in the order the list first names them.  With matrix set, rows, jobs and slot
+// describe the matrix form (RhoMatrixArgs).  Its rows (n_x, n_y), in the list's
+// order, run in pieces of equal shares of them; within a piece the rows are sorted
+// by the 16-column blocks of |n_z| they use, so that the tiles of 16 rows multiply
+// few columns no row of theirs has.  Piece k takes the jobs [piece_job[k],
+// piece_job[k + 1]), after which the modes [0, piece_modes[k]) are complete.
+// A plan is made anew for each call; only its storage is kept.
+struct RhoPlan {
+    int nu = 0;
+    int nmax[3] = {0, 0, 0};
+    std::vector<int> mode;          // [nq] the mode of each q of the list
+    std::vector<int> first, second; // [nu] the list's first and second q of each mode (-1: none)
+    std::vector<int> repeat;        // q of the list beyond those two, rows to be copied from `first`
+    bool matrix = false;
+    std::vector<int2> rows;
+    std::vector<RhoJob> jobs;
+    std::vector<int> piece_job, piece_modes, slot;
+    int width = 0;
+    // scratch of make_rho_plan
+    std::vector<int> mode_at, row_at, row_mode, row_cols, mode_row, mode_nz, order, at;
+    std::vector<int2> list_rows;
+};
+// max_pieces: 1 for one launch; more: as many as fill the chip, at most that many
+void make_rho_plan(const int* n3, int nq, int max_pieces, RhoPlan* P);
 
 struct TableCache;
 TableCache& table_cache();
@@ -65,13 +96,18 @@ struct pimc_ctx {
     int device = 0;               // the HIP device current when the context was created
     double* d_vslice = nullptr;
     double* d_out = nullptr;
-    double* h_map = nullptr;      // 64 doubles of mapped, coherent pinned host memory
+    // mapped, coherent pinned host memory: 64 doubles of small results, then from
+    // kSqSlot room for kMappedSq S(q) values
+    static constexpr int kSqSlot = 64, kMappedSq = 8192;
+    double* h_map = nullptr;
     double* d_map = nullptr;      // its device address
     // completion word (slot kDoneSlot of the mapped block): the last kernel of a
     // call publishes the call's sequence number there
     static constexpr int kDoneSlot = 63;
     unsigned long long seq = 0;
     unsigned long long* d_done() { return reinterpret_cast<unsigned long long*>(d_map + kDoneSlot); }
+    // the arrival counter of the S(q) kernel (zero between calls): past d_out's 16
+    unsigned* d_ticket() { return reinterpret_cast<unsigned*>(d_out + 16); }
     int wait_done(unsigned long long s);   // spin, then fall back to a stream sync
     // the direct Delta V form's per-bead results (mapped, coherent pinned block)
     pimc::VnnDirectOut* h_vdir = nullptr;
@@ -151,18 +187,24 @@ struct pimc_ctx {
     // structure factors
     int cap_q = 0;
     double* d_q = nullptr;
-    int* d_qn = nullptr;
     double* d_rho = nullptr;
     size_t cap_rho = 0;
     double* d_fqt = nullptr;
     size_t cap_fqt = 0;
-    // F(q,tau) of long lattice q lists into page-locked memory: a second stream
-    // copies each chunk's rows out while the next chunk computes
-    hipStream_t copy_stream = nullptr;
+    // a call's q list: lattice components, kinds and plan (storage kept)
+    std::vector<int> q_n3;
+    std::vector<uint8_t> q_lat;
+    pimc::RhoPlan plan;
+    int* d_plan = nullptr;             // the plan on the device
+    size_t cap_plan = 0;
+    // F(q,tau) of long lattice q lists into page-locked memory: the DMA engines
+    // copy each chunk's rows out while the next chunk computes
+    pimc::DmaCopies dma;
     std::vector<hipEvent_t> chunk_ev;
     long isf_chunks = 0;               // chunks computed that way (pimc_kernel_time "isf_chunks")
     // staging
-    double* h_stage = nullptr;    // >= 3*M*N doubles, pinned
+    double* h_stage = nullptr;    // cap_stage >= 3*M*N doubles, pinned
+    size_t cap_stage = 0;
     double* h_out = nullptr;      // 64 doubles, pinned
     // host mirrors
     std::vector<int> h_nbs;

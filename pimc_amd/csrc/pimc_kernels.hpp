@@ -168,6 +168,27 @@ struct RhoArgs {
     double* rho;           // [M][nq][2] FP64
 };
 
+// A wave's job of the matrix form of rho_q(m) (k_rho_matrix): the 16 rows
+// (n_x, n_y) of a tile against the 16 columns |n_z| from col0.
+struct RhoJob {
+    int tile, col0;
+};
+struct RhoMatrixArgs {
+    const double* pos;   // SoA planes [3][M][nalloc]
+    int64_t plane;
+    int nalloc, num_slices;
+    const int* nbs;
+    double invL;
+    int nmax[3];
+    const int2* rows;    // [tiles][16] (n_x, n_y), n_x >= 0; unused rows (0, 0)
+    const RhoJob* jobs;
+    int job0, job_end;   // the launch's jobs
+    const int* slot;     // [16 tiles][2][width]: the mode of +n_z and of -n_z, or -1
+    int width;           // columns, a multiple of 16
+    int nu;              // modes
+    double* rho;         // [M][nu][2] FP64
+};
+
 // Publishes seq to a host-mapped completion word after the calling thread's
 // earlier writes (the host spins on it instead of a stream synchronisation).
 __device__ __forceinline__ void publish_done(unsigned long long* done, unsigned long long seq) {
@@ -281,7 +302,15 @@ hipError_t launch_kinetic(hipStream_t st, const double* pos, int64_t plane, int 
 hipError_t launch_aziz_batch(int mode, hipStream_t st, const double* sep, int n, const AzizDev& az, const double* d1,
                              const double* d2, int what, double* out);
 hipError_t launch_rho(bool lattice, hipStream_t st, const RhoArgs& A);
-hipError_t launch_isf(hipStream_t st, const double* rho, int nq, int M, double inv_n, double* fqt, int only_tau0);
+hipError_t launch_rho_matrix(hipStream_t st, const RhoMatrixArgs& A);
+// F of modes [u0, u_end) of rho [M][nu]: mode u to rows dst[2 u], dst[2 u + 1] of
+// fqt (-1: none), or to row u without dst.
+hipError_t launch_isf(hipStream_t st, const double* rho, int nu, int u0, int u_end, int M, double inv_n,
+                      const int* dst, double* fqt);
+// S of nq modes; done (or null): published with seq once sq (mapped) is written,
+// ticket a zeroed counter.
+hipError_t launch_ssf(hipStream_t st, const double* rho, int nq, int M, double inv_n, double* sq,
+                      unsigned* ticket = nullptr, unsigned long long* done = nullptr, unsigned long long seq = 0);
 hipError_t launch_ssf_pairs(hipStream_t st, const double* pos, int64_t plane, int nalloc, int M, const int* nbs,
                             const double* q, int nq, const BoxDev& box, double* partial, double inv_n, double* sq);
 int rho_max_nmax();

@@ -111,7 +111,7 @@ int ssf_run(pimc_ctx* c, char* base, bool lattice, const double* q, int n, const
         A.rho = d_rho;
         for (int d = 0; d < 3; ++d) A.nmax[d] = nmax[d];
         NA_HIP(c, launch_rho(true, c->stream, A));
-        NA_HIP(c, launch_isf(c->stream, d_rho, n, M, inv_n, d_out, 1));
+        NA_HIP(c, launch_ssf(c->stream, d_rho, n, M, inv_n, d_out));
     } else {
         NA_HIP(c, launch_ssf_pairs(c->stream, c->d_pos, c->plane, c->desc.num_alloc, M, c->d_nbs, d_q, n, c->box,
                                    d_rho, inv_n, d_out));

@@ -821,7 +821,7 @@ hipError_t pimc_server::fire_ssf(const BatchLaunch& L) {
         for (int k = k0; k < k0 + n; ++k)
             for (int d = 0; d < 3; ++d) A.nmax[d] = std::max(A.nmax[d], std::abs(h_qn[3 * k + d]));
         e = launch_rho(true, S.stream, A);
-        if (e == hipSuccess) e = launch_isf(S.stream, S.d_rho, n, M, L.inv_n, S.m_sq + k0, 1);
+        if (e == hipSuccess) e = launch_ssf(S.stream, S.d_rho, n, M, L.inv_n, S.m_sq + k0);
     }
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_serve_publish, dim3(1), dim3(64), 0, S.stream, S.d_done, S.seq);

@@ -11,15 +11,16 @@
 // (O(n_q M^2)) instead of O(n_q M^2 N^2) trigonometric pair terms.
 //
 // Lattice q = (2 pi / L) n: exp(i q.r) = prod_d exp(2 pi i n_d s_d), s_d = x_d / L.
-// Each workgroup stages per-bead axis phasors exp(2 pi i n s_d) for -nmax <= n <=
-// nmax in LDS (phase reduced in FP64, FP32 sincospi; the negative n are the
-// conjugates), then each lane accumulates a run of q-vectors with FP32 complex
-// products and FP64 per-chunk sums; the X Y product of a row of q sharing
-// (n_x, n_y) is formed once per bead (k_rho_lattice).
+// Each workgroup stages per-bead axis phasors exp(2 pi i n s_d) in LDS (phase
+// reduced in FP64, FP32 sincospi) and sums X Y Z over the beads with FP32 products
+// and FP64 sums every 32 beads: as real matrix products on the matrix cores for a
+// list of q (k_rho_matrix), or one lane per q (k_rho_lattice).  q and -q have
+// conjugate modes and equal S and F, so a list's modes are formed once per pair.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "pimc_kernels.hpp"
 
@@ -28,45 +29,134 @@ namespace pimc {
 constexpr int kRhoThreads = 256;
 constexpr int kRhoBeadChunk = 32;  // beads per LDS phasor stage
 constexpr int kMaxNmax = 40;       // largest |n_d| of a lattice q
-constexpr int kReseed = 4;         // exact sincospi every kReseed powers, products in between
 
-// rho_q(m) for lattice q.  Lane t of a workgroup takes q = base + t + 256 k
-// (k < QPT), so a wave walks consecutive q: mostly one (n_x, n_y) and consecutive
-// n_z, which makes the x/y phasor reads LDS broadcasts and the z reads
-// consecutive words.  Tables are bead-major: ph[axis][bead][n + nmax].
-//
-// Rows: consecutive q of the list that share (n_x, n_y) -- in the reference's
-// order a q set is runs of n_z -- share the product X(n_x) Y(n_y) of each bead.
-// A workgroup first numbers the rows its q touch (a block scan over the q
-// range); when they fit the launch's row capacity (rows_cap, at most
-// kRhoRowsMax, sized with the q per workgroup), each bead chunk forms every row's product
-// once into LDS and a lane's term per (q, bead) is one complex product with
-// Z(n_z), 4 FMA instead of 8.  The products are formed by the same FP32
-// expressions as in the per-lane form, and the FP32 partial of every 32 beads
-// is added into the FP64 sum either way, so both forms give the same bits.
-constexpr int kRhoRowsMax = 128;   // rows of one workgroup's q range that share products
+// Per-bead axis phasors E(n) = exp(2 pi i n s), s = x_d / L, of one stage of
+// kRhoBeadChunk beads (beads past the slice's last are zero), bead-major in LDS:
+// x and z for 0 <= n <= H, y for -H <= n <= H, up to the list's own nmax[d] <= H.
+// H is fixed at compile time, so a bead's rows are an immediate offset apart, and
+// even, so the row lengths are odd and the beads start on distinct LDS banks.
+// n < 4 and the multiples of four are evaluated (seeds(): the phase in quarter
+// turns reduced in FP64, sine and cosine of the remainder in FP32), the others are
+// one complex product E(4 a) E(b) of those (products(), after a barrier): no entry
+// is more than one product away from an evaluated one.  Each pass walks (entry,
+// bead), bead fastest, over the whole workgroup, the entries through descriptors
+// made once.  Both kernels below read tables made here.
+template <int H>
+struct Phasors {
+    static constexpr int WX = H + 1, WY = 2 * H + 1, WZ = H + 1;
+    static constexpr int X = 0, Y = kRhoBeadChunk * WX, Z = Y + kRhoBeadChunk * WY;
+    // and 16 more: the matrix form reads columns up to 15 past a row's end (unused)
+    static constexpr int kEntries = Z + kRhoBeadChunk * WZ + 16;
+    static constexpr int kSeeds = 3 * (4 + H / 4), kProducts = 3 * (H - 3 - H / 4);
+    struct Entries {
+        int4 seed[kSeeds];       // place, row length | (place of -n, + 1) << 8, 4 n, 32 axis
+        int4 product[kProducts]; // place, row length | (place of -n, + 1) << 8, places of the factors
+        int n_seeds, n_products;
+    };
+    static __device__ __forceinline__ int count_seeds(int h) { return h < 4 ? h + 1 : 4 + h / 4; }
+    // by every lane, before a barrier
+    static __device__ __forceinline__ void make_entries(Entries& E, const int nmax[3]) {
+        const int base[3] = {X, Y + H, Z}, width[3] = {WX, WY, WZ};
+        int s0 = 0, p0 = 0;
+#pragma unroll
+        for (int axis = 0; axis < 3; ++axis) {
+            const int h = nmax[axis], ns = count_seeds(h), np = h + 1 - ns;
+            for (int e = threadIdx.x; e < ns; e += (int)blockDim.x) {
+                const int n = e < 4 ? e : 4 * (e - 3);
+                const int back = axis == 1 && n ? base[1] - n + 1 : 0;
+                E.seed[s0 + e] = make_int4(base[axis] + n, width[axis] | back << 8, 4 * n, kRhoBeadChunk * axis);
+            }
+            for (int e = threadIdx.x; e < np; e += (int)blockDim.x) {
+                const int n4 = 4 * (1 + e / 3), n1 = 1 + e % 3, n = n4 + n1;
+                const int back = axis == 1 ? base[1] - n + 1 : 0;
+                E.product[p0 + e] = make_int4(base[axis] + n, width[axis] | back << 8, base[axis] + n4, base[axis] + n1);
+            }
+            s0 += ns;
+            p0 += np;
+        }
+        if (threadIdx.x == 0) {
+            E.n_seeds = s0;
+            E.n_products = p0;
+        }
+    }
+    // at: the beads' positions in box units, |at| <= 1/2, [3][kRhoBeadChunk] in LDS
+    static __device__ __forceinline__ void seeds(float2* t, const Entries& E, const double* at, int nb) {
+        const int bb = threadIdx.x & (kRhoBeadChunk - 1);
+        for (int e = threadIdx.x / kRhoBeadChunk; e < E.n_seeds; e += (int)blockDim.x / kRhoBeadChunk) {
+            const int4 d = E.seed[e];
+            // quarter turns: the nearest whole number k and the rest, |r| <= 1/2,
+            // whose FP32 rounding is under 2.4e-8 of a radian
+            const double v = (double)d.z * at[d.w + bb];
+            const double k = rint(v);
+            const float r = (float)(v - k) * 1.57079632679489662f;
+            const int quad = (int)k;
+            // sine and cosine by their series, |r| <= pi/4 (last terms r^9/9!, r^10/10!)
+            const float r2 = r * r;
+            float sn = fmaf(r2, 2.7557319e-6f, -1.9841270e-4f);
+            sn = fmaf(r2, sn, 8.3333333e-3f);
+            sn = fmaf(r2, sn, -1.6666667e-1f);
+            sn = fmaf(r2 * r, sn, r);
+            float cs = fmaf(r2, -2.7557319e-7f, 2.4801587e-5f);
+            cs = fmaf(r2, cs, -1.3888889e-3f);
+            cs = fmaf(r2, cs, 4.1666667e-2f);
+            cs = fmaf(r2, cs, -0.5f);
+            cs = fmaf(r2, cs, 1.0f);
+            const bool odd = quad & 1;
+            float c = odd ? sn : cs, s = odd ? cs : sn;
+            // E rotates by i every quarter turn: (c, s) -> (-s, c)
+            c = ((quad + 1) & 2) ? -c : c;
+            s = (quad & 2) ? -s : s;
+            if (bb >= nb) c = s = 0.f;
+            const int w = d.y & 255, back = d.y >> 8;
+            t[d.x + bb * w] = make_float2(c, s);
+            if (back) t[back - 1 + bb * w] = make_float2(c, -s);
+        }
+    }
+    static __device__ __forceinline__ void products(float2* t, const Entries& E) {
+        const int bb = threadIdx.x & (kRhoBeadChunk - 1);
+        for (int e = threadIdx.x / kRhoBeadChunk; e < E.n_products; e += (int)blockDim.x / kRhoBeadChunk) {
+            const int4 d = E.product[e];
+            const int w = d.y & 255, back = d.y >> 8;
+            const float2 p = t[d.z + bb * w], q = t[d.w + bb * w];
+            const float c = fmaf(p.x, q.x, -p.y * q.y);
+            const float s = fmaf(p.x, q.y, p.y * q.x);
+            t[d.x + bb * w] = make_float2(c, s);
+            if (back) t[back - 1 + bb * w] = make_float2(c, -s);
+        }
+    }
+};
+static_assert(kMaxNmax <= 40 && 2 * 40 + 1 < 256, "row lengths take 8 bits");
 
-template <int QPT>
-__global__ __launch_bounds__(kRhoThreads) void k_rho_lattice(RhoArgs A, int rows_cap) {
-    extern __shared__ float2 ph[];
+// A coordinate in box units, less its whole boxes (they drop out of lattice phases).
+__device__ __forceinline__ double box_fraction(double x, double invL) {
+    const double s = x * invL;
+    return s - rint(s);
+}
+
+// rho at +n_z (sg = +1) or -n_z (sg = -1) of a row (n_x, n_y) from its four real
+// sums over the beads, with X Y = xr + i xi and Z(|n_z|) = c + i s:
+//   rc = sum xr c, rs = sum xr s, ic = sum xi c, is = sum xi s.
+__device__ __forceinline__ double2 rho_of_sums(double rc, double rs, double ic, double is, double sg) {
+    return make_double2(rc - sg * is, ic + sg * rs);
+}
+
+// rho_q(m) for lattice q, one lane per q (lane t of a workgroup takes q = base +
+// t + 256 k, k < QPT): the form for short runs and for q lists too sparse for
+// the matrix form below.  q and -q are conjugates, so a q is first turned into
+// the half space n_x > 0, or n_x = 0 and n_y > 0, ...: the sums, their order
+// (32 beads in FP32, then FP64) and so the bits are those of the matrix form.
+template <int QPT, int H>
+__global__ __launch_bounds__(kRhoThreads) void k_rho_lattice(RhoArgs A) {
+    using T = Phasors<H>;
+    __shared__ float2 ph[T::kEntries];
+    __shared__ typename T::Entries E;
+    __shared__ double at[3 * kRhoBeadChunk];
     const int m = blockIdx.y;
     const int n_beads = A.nbs[m];
-    const int h0 = A.nmax[0], h1 = A.nmax[1], h2 = A.nmax[2];
-    const int w0 = 2 * h0 + 1, w1 = 2 * h1 + 1, w2 = 2 * h2 + 1;
-    float2* phx = ph;
-    float2* phy = phx + w0 * kRhoBeadChunk;
-    float2* phz = phy + w1 * kRhoBeadChunk;
-    float2* xy = phz + w2 * kRhoBeadChunk;                                // [rows_cap][kRhoBeadChunk]
-    int2* rows = reinterpret_cast<int2*>(xy + rows_cap * kRhoBeadChunk);  // [rows_cap] (n_x, n_y)
-    int* scan = reinterpret_cast<int*>(xy);                                // [kRhoThreads * QPT], before xy is used
-    __shared__ int wave_tot[kRhoThreads / 64];
     const double* px = A.pos + (int64_t)m * A.nalloc;
-    const double* py = px + A.plane;
-    const double* pz = py + A.plane;
-
-    const int q0 = blockIdx.x * kRhoThreads * QPT;
-    const int qbase = q0 + threadIdx.x;
-    int ix[QPT], iy[QPT], iz[QPT], ro[QPT];
+    const int qbase = blockIdx.x * kRhoThreads * QPT + threadIdx.x;
+    int ix[QPT], iy[QPT], iz[QPT];
+    double sg[QPT], cj[QPT];
 #pragma unroll
     for (int k = 0; k < QPT; ++k) {
         const int qi = qbase + k * kRhoThreads;
@@ -76,154 +166,184 @@ __global__ __launch_bounds__(kRhoThreads) void k_rho_lattice(RhoArgs A, int rows
             ny = A.qn[3 * qi + 1];
             nz = A.qn[3 * qi + 2];
         }
-        ix[k] = nx + h0;
-        iy[k] = ny + h1;
-        iz[k] = nz + h2;
-        ro[k] = 0;
+        const bool flip = nx < 0 || (nx == 0 && (ny < 0 || (ny == 0 && nz < 0)));
+        cj[k] = flip ? -1.0 : 1.0;
+        ix[k] = flip ? -nx : nx;
+        iy[k] = H + (flip ? -ny : ny);
+        iz[k] = nz < 0 ? -nz : nz;
+        sg[k] = (flip ? -nz : nz) < 0 ? -1.0 : 1.0;
     }
-    bool use_rows = false;
-    int n_rows = 0;
-    if (rows_cap > 0) {
+    double rc[QPT], rs[QPT], ic[QPT], is[QPT];
 #pragma unroll
-        for (int k = 0; k < QPT; ++k) {
-            const int qi = qbase + k * kRhoThreads;
-            const int start = qi < A.nq &&
-                              (qi == q0 || ix[k] - h0 != A.qn[3 * qi - 3] || iy[k] - h1 != A.qn[3 * qi - 2]);
-            scan[threadIdx.x + k * kRhoThreads] = start;
-        }
-        __syncthreads();
-        // inclusive prefix of the row starts over the workgroup's q range: lane t
-        // owns entries [t QPT, (t + 1) QPT), then a wave scan and the waves in order
-        int own[QPT];
-        int run = 0;
-#pragma unroll
-        for (int k = 0; k < QPT; ++k) {
-            run += scan[threadIdx.x * QPT + k];
-            own[k] = run;
-        }
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        int incl = run;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int v = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += v;
-        }
-        if (lane == 63) wave_tot[wave] = incl;
-        __syncthreads();
-        int before = incl - run;
-        for (int w = 0; w < wave; ++w) before += wave_tot[w];
-        n_rows = wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
-        __syncthreads();   // every lane has read its entries
-#pragma unroll
-        for (int k = 0; k < QPT; ++k) scan[threadIdx.x * QPT + k] = before + own[k];
-        __syncthreads();
-        use_rows = n_rows <= rows_cap;
-#pragma unroll
-        for (int k = 0; k < QPT; ++k) {
-            const int l = threadIdx.x + k * kRhoThreads;
-            const int r = scan[l] - 1;   // the row of q_l (starts counted up to and with it)
-            const bool first = l == 0 || scan[l - 1] != scan[l];
-            ro[k] = (use_rows && r >= 0 && r < rows_cap) ? r : 0;
-            if (use_rows && first && qbase + k * kRhoThreads < A.nq && r >= 0 && r < rows_cap)
-                rows[r] = make_int2(ix[k] - h0, iy[k] - h1);
-        }
-    }
-    double are[QPT], aim[QPT];
-#pragma unroll
-    for (int k = 0; k < QPT; ++k) are[k] = aim[k] = 0.0;
-
+    for (int k = 0; k < QPT; ++k) rc[k] = rs[k] = ic[k] = is[k] = 0.0;
+    T::make_entries(E, A.nmax);
     for (int b0 = 0; b0 < n_beads; b0 += kRhoBeadChunk) {
         const int nb = min(kRhoBeadChunk, n_beads - b0);
         __syncthreads();
-        // one lane per (axis, bead) row: exp(2 pi i n s) for n = 0..nmax, and the
-        // conjugates at -n
-        for (int r = threadIdx.x; r < 3 * kRhoBeadChunk; r += kRhoThreads) {
-            const int axis = r / kRhoBeadChunk, bb = r % kRhoBeadChunk;
-            const int h = axis == 0 ? h0 : (axis == 1 ? h1 : h2);
-            float2* row = (axis == 0 ? phx : (axis == 1 ? phy : phz)) + bb * (2 * h + 1) + h;
-            if (bb >= nb) {
-                for (int n = -h; n <= h; ++n) row[n] = make_float2(0.f, 0.f);
-                continue;
-            }
-            const double x = (axis == 0 ? px : (axis == 1 ? py : pz))[b0 + bb];
-            const double sfrac = x * A.invL;           // position in box units
-            float s1, c1;
-            {
-                const double red = sfrac - rint(sfrac);
-                sincospif((float)(2.0 * red), &s1, &c1);
-            }
-            float cr = 1.f, ci = 0.f;
-            for (int n = 0; n <= h; ++n) {
-                if (n % kReseed == 0) {
-                    const double t = (double)n * sfrac;
-                    const double red = t - rint(t);
-                    sincospif((float)(2.0 * red), &ci, &cr);
-                } else {
-                    const float nr = fmaf(cr, c1, -ci * s1);
-                    const float ni = fmaf(cr, s1, ci * c1);
-                    cr = nr;
-                    ci = ni;
-                }
-                row[n] = make_float2(cr, ci);
-                row[-n] = make_float2(cr, -ci);
-            }
+        if (threadIdx.x < 3 * kRhoBeadChunk) {
+            const int axis = threadIdx.x / kRhoBeadChunk, bb = threadIdx.x % kRhoBeadChunk;
+            at[threadIdx.x] = bb < nb ? box_fraction(px[axis * A.plane + b0 + bb], A.invL) : 0.0;
         }
         __syncthreads();
-        float sre[QPT], sim[QPT];
+        T::seeds(ph, E, at, nb);
+        __syncthreads();
+        T::products(ph, E);
+        __syncthreads();
+        float frc[QPT], frs[QPT], fic[QPT], fis[QPT];
 #pragma unroll
-        for (int k = 0; k < QPT; ++k) sre[k] = sim[k] = 0.f;
-        if (use_rows) {
-            // every row's X Y product of the chunk's beads, once
-            for (int t = threadIdx.x; t < n_rows * kRhoBeadChunk; t += kRhoThreads) {
-                const int r = t / kRhoBeadChunk, bb = t % kRhoBeadChunk;
-                const int2 rn = rows[r];
-                const float2 ex = phx[bb * w0 + rn.x + h0];
-                const float2 ey = phy[bb * w1 + rn.y + h1];
+        for (int k = 0; k < QPT; ++k) frc[k] = frs[k] = fic[k] = fis[k] = 0.f;
+        for (int bb = 0; bb < nb; ++bb) {
+#pragma unroll
+            for (int k = 0; k < QPT; ++k) {
+                const float2 ex = ph[T::X + bb * T::WX + ix[k]];
+                const float2 ey = ph[T::Y + bb * T::WY + iy[k]];
+                const float2 ez = ph[T::Z + bb * T::WZ + iz[k]];
                 const float xr = fmaf(ex.x, ey.x, -ex.y * ey.y);
                 const float xi = fmaf(ex.x, ey.y, ex.y * ey.x);
-                xy[t] = make_float2(xr, xi);
-            }
-            __syncthreads();
-            for (int bb = 0; bb < nb; ++bb) {
-#pragma unroll
-                for (int k = 0; k < QPT; ++k) {
-                    const float2 p = xy[ro[k] * kRhoBeadChunk + bb];
-                    const float2 ez = phz[bb * w2 + iz[k]];
-                    sre[k] = fmaf(p.x, ez.x, sre[k]);
-                    sre[k] = fmaf(-p.y, ez.y, sre[k]);
-                    sim[k] = fmaf(p.x, ez.y, sim[k]);
-                    sim[k] = fmaf(p.y, ez.x, sim[k]);
-                }
-            }
-        } else {
-            for (int bb = 0; bb < nb; ++bb) {
-#pragma unroll
-                for (int k = 0; k < QPT; ++k) {
-                    const float2 ex = phx[bb * w0 + ix[k]];
-                    const float2 ey = phy[bb * w1 + iy[k]];
-                    const float2 ez = phz[bb * w2 + iz[k]];
-                    const float xr = fmaf(ex.x, ey.x, -ex.y * ey.y);
-                    const float xi = fmaf(ex.x, ey.y, ex.y * ey.x);
-                    sre[k] = fmaf(xr, ez.x, sre[k]);
-                    sre[k] = fmaf(-xi, ez.y, sre[k]);
-                    sim[k] = fmaf(xr, ez.y, sim[k]);
-                    sim[k] = fmaf(xi, ez.x, sim[k]);
-                }
+                frc[k] = fmaf(xr, ez.x, frc[k]);
+                frs[k] = fmaf(xr, ez.y, frs[k]);
+                fic[k] = fmaf(xi, ez.x, fic[k]);
+                fis[k] = fmaf(xi, ez.y, fis[k]);
             }
         }
 #pragma unroll
         for (int k = 0; k < QPT; ++k) {
-            are[k] += (double)sre[k];
-            aim[k] += (double)sim[k];
+            rc[k] += (double)frc[k];
+            rs[k] += (double)frs[k];
+            ic[k] += (double)fic[k];
+            is[k] += (double)fis[k];
         }
     }
 #pragma unroll
     for (int k = 0; k < QPT; ++k) {
         const int qi = qbase + k * kRhoThreads;
         if (qi < A.nq) {
-            A.rho[((int64_t)m * A.nq + qi) * 2 + 0] = are[k];
-            A.rho[((int64_t)m * A.nq + qi) * 2 + 1] = aim[k];
+            const double2 v = rho_of_sums(rc[k], rs[k], ic[k], is[k], sg[k]);
+            reinterpret_cast<double2*>(A.rho)[(int64_t)m * A.nq + qi] = make_double2(v.x, cj[k] * v.y);
         }
+    }
+}
+
+// rho_q(m) of a whole list of lattice q as real matrix products.  For a slice the
+// rows (n_x, n_y) of the list's half space and the columns |n_z| make
+//   rho(n_x, n_y, +-n_z) = sum_b X Y(row, b) Z(n_z, b)^(+-1),
+// four real products (Re or Im of X Y against cos or sin of Z) whose sums give
+// both signs of n_z (rho_of_sums).  A wave takes a job of 16 rows by 16 columns:
+// four accumulators of v_mfma_f32_16x16x4_f32 (lane l: row and column l % 16,
+// bead l / 16 of the four of a step; the unit adds the four products in bead
+// order with one rounding each, as the chain of FP32 FMA it replaces).  The X Y
+// operand is formed in registers from the phasor tables, four FMA per step, so
+// nothing but the tables is staged; up to 16 waves of a workgroup share them.
+// Every 32 beads the FP32 sums go into FP64 ones, as in k_rho_lattice.  Three
+// table buffers: while stage c is summed, stage c + 1 gets its products and
+// stage c + 2 its seeds, one barrier per stage.
+// Bound: the FP32 matrix rate (126 TFLOP/s measured here), 128 SIMD cycles per job
+// and four beads; the unit shares the vector unit's multipliers, so the tables, the
+// X Y operands and the FP64 sums (about a third of the time) add to it.  At N = 2048
+// x 250 the 50 201 modes of 100 401 q take 2.0 ms (one lane per q, every q: 17.8
+// ms; one lane per mode 7.8 ms), at N = 256 x 167 the 2689 modes of 5377 q 32 us
+// (103 us; 72 us).  Waves that only make tables beside waves that only sum were
+// slower (2.8 ms), as were 8 waves to a workgroup (2.9 ms).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kRhoWaves = 16;
+
+template <int H>
+__global__ __launch_bounds__(64 * kRhoWaves) void k_rho_matrix(RhoMatrixArgs A) {
+    using T = Phasors<H>;
+    extern __shared__ float2 ph[];                 // [3][T::kEntries]
+    __shared__ typename T::Entries E;
+    __shared__ double at[2][3 * kRhoBeadChunk];   // positions in box units, two stages
+    const int m = blockIdx.y;
+    const int n_beads = A.nbs[m];
+    const int stages = (n_beads + kRhoBeadChunk - 1) / kRhoBeadChunk;
+    const double* px = A.pos + (int64_t)m * A.nalloc;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int j = A.job0 + blockIdx.x * ((int)blockDim.x >> 6) + wave;
+    const bool work = j < A.job_end;
+    const RhoJob job = work ? A.jobs[j] : RhoJob{0, 0};
+    const int l16 = lane & 15, l4 = lane >> 4;
+    const int2 row = work ? A.rows[16 * job.tile + l16] : make_int2(0, 0);
+    const int ix = T::X + l4 * T::WX + row.x;
+    const int iy = T::Y + l4 * T::WY + H + row.y;
+    const int iz = T::Z + l4 * T::WZ + job.col0 + l16;
+    double sum[4][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[k][r] = 0.0;
+    auto make_seeds = [&](int c) {
+        if (c < stages)
+            T::seeds(ph + (c % 3) * T::kEntries, E, at[c & 1], min(kRhoBeadChunk, n_beads - c * kRhoBeadChunk));
+    };
+    auto make_products = [&](int c) {
+        if (c < stages) T::products(ph + (c % 3) * T::kEntries, E);
+    };
+    // a stage's positions: lanes 0 .. 95 load them one stage before they are put
+    // into LDS, so no pass waits for memory
+    const int p_axis = threadIdx.x / kRhoBeadChunk, p_bead = threadIdx.x % kRhoBeadChunk;
+    auto load_pos = [&](int c) {
+        const int b = c * kRhoBeadChunk + p_bead;
+        return p_axis < 3 && b < n_beads ? box_fraction(px[p_axis * A.plane + b], A.invL) : 0.0;
+    };
+    auto put_pos = [&](int c, double v) {
+        if (p_axis < 3) at[c & 1][threadIdx.x] = v;
+    };
+    auto sum_stage = [&](int c) {
+        if (!work) return;
+        const float2* t = ph + (c % 3) * T::kEntries;
+        const float2 *bx = t + ix, *by = t + iy, *bz = t + iz;
+        const int steps = (min(kRhoBeadChunk, n_beads - c * kRhoBeadChunk) + 3) >> 2;
+        f32x4 acc[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto step = [&](int k) {
+            const float2 ex = bx[4 * k * T::WX], ey = by[4 * k * T::WY], ez = bz[4 * k * T::WZ];
+            const float xr = fmaf(ex.x, ey.x, -ex.y * ey.y);
+            const float xi = fmaf(ex.x, ey.y, ex.y * ey.x);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr, ez.x, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xr, ez.y, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(xi, ez.x, acc[2], 0, 0, 0);
+            acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(xi, ez.y, acc[3], 0, 0, 0);
+        };
+        if (steps == kRhoBeadChunk / 4) {
+#pragma unroll
+            for (int k = 0; k < kRhoBeadChunk / 4; ++k) step(k);
+        } else {
+            for (int k = 0; k < steps; ++k) step(k);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[k][r] += (double)acc[k][r];
+    };
+    T::make_entries(E, A.nmax);
+    put_pos(0, load_pos(0));
+    put_pos(1, load_pos(1));
+    __syncthreads();
+    double ahead = load_pos(2);
+    make_seeds(0);
+    make_seeds(1);
+    __syncthreads();
+    make_products(0);
+    put_pos(2, ahead);
+    __syncthreads();
+    for (int c = 0; c < stages; ++c) {
+        ahead = load_pos(c + 3);
+        make_products(c + 1);
+        make_seeds(c + 2);
+        sum_stage(c);
+        put_pos(c + 3, ahead);   // the other of the two: seeds of stage c + 1 are done
+        __syncthreads();
+    }
+    if (!work) return;
+    // lane l, register r: row 4 (l / 16) + r, column l % 16
+    double2* out = reinterpret_cast<double2*>(A.rho) + (int64_t)m * A.nu;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int* slot = A.slot + (int64_t)(16 * job.tile + 4 * l4 + r) * 2 * A.width + job.col0 + l16;
+        const int up = slot[0], un = slot[A.width];
+        if (up >= 0) out[up] = rho_of_sums(sum[0][r], sum[1][r], sum[2][r], sum[3][r], 1.0);
+        if (un >= 0) out[un] = rho_of_sums(sum[0][r], sum[1][r], sum[2][r], sum[3][r], -1.0);
     }
 }
 
@@ -259,22 +379,26 @@ __global__ __launch_bounds__(kRhoThreads) void k_rho_general(RhoArgs A) {
 }
 
 // F(q,tau) = sum_m Re rho(m) conj(rho(m+tau)).  A workgroup of 4 waves takes
-// kIsfQ = 4 q-vectors, one per wave; rho_q(m) is staged twice over (m and
-// m + M) so lag tau reads row[m + tau] with no wrap test: rho(m) is an LDS
-// broadcast, rho(m + tau) consecutive words, each lag at a fixed offset.  Rows
-// are 2M + 64 long: lanes past the last lag read the zero padding.
+// kIsfQ = 4 modes, one per wave; rho(m) is staged twice over (m and m + M) so lag
+// tau reads row[m + tau] with no wrap test: rho(m) is an LDS broadcast,
+// rho(m + tau) consecutive words, each lag at a fixed offset.  Rows are 2M + 64
+// long: lanes past the last lag read the zero padding.  The sum over the closed
+// path makes F(M - tau) = F(tau), so only the lags up to M / 2 are formed.  With
+// dst, mode u's lags go to the rows dst[2 u] and dst[2 u + 1] (those of q and -q;
+// -1: none), else to row u.
 constexpr int kIsfQ = 4;
-constexpr int kIsfLagsPerLane = 8;   // M <= 512
-__global__ __launch_bounds__(256) void k_isf_from_rho(const double* __restrict__ rho, int nq, int M,
-                                                     double inv_n, double* __restrict__ fqt) {
+constexpr int kIsfLagsPerLane = 5;   // M / 2 + 1 <= 257
+__global__ __launch_bounds__(256) void k_isf_from_rho(const double* __restrict__ rho, int nu, int u0, int u_end, int M,
+                                                     double inv_n, const int* __restrict__ dst,
+                                                     double* __restrict__ fqt) {
     extern __shared__ double2 sr[];  // [kIsfQ][2M + 64]
     const int R = 2 * M + 64;
-    const int qb = blockIdx.x * kIsfQ;
-    const int nql = min(kIsfQ, nq - qb);
+    const int qb = u0 + blockIdx.x * kIsfQ;
+    const int nql = min(kIsfQ, u_end - qb);
     for (int t = threadIdx.x; t < M * kIsfQ; t += 256) {
         const int m = t / kIsfQ, k = t % kIsfQ;
         double2 v = make_double2(0.0, 0.0);
-        if (k < nql) v = make_double2(rho[((int64_t)m * nq + qb + k) * 2], rho[((int64_t)m * nq + qb + k) * 2 + 1]);
+        if (k < nql) v = reinterpret_cast<const double2*>(rho)[(int64_t)m * nu + qb + k];
         sr[(int64_t)k * R + m] = v;
         sr[(int64_t)k * R + m + M] = v;
     }
@@ -286,57 +410,97 @@ __global__ __launch_bounds__(256) void k_isf_from_rho(const double* __restrict__
     double acc[kIsfLagsPerLane];
 #pragma unroll
     for (int u = 0; u < kIsfLagsPerLane; ++u) acc[u] = 0.0;
-    const int nu = (M + 63) / 64;
+    const int half = M / 2 + 1;   // lags 0 .. M/2
+    const int nl = (half + 63) / 64;
     const double2* b = row + lane;
     for (int m = 0; m < M; ++m, ++b) {
         const double2 a = row[m];
 #pragma unroll
         for (int u = 0; u < kIsfLagsPerLane; ++u) {
-            if (u < nu) {
+            if (u < nl) {
                 const double2 c = b[64 * u];
                 acc[u] = fma(a.x, c.x, acc[u]);
                 acc[u] = fma(a.y, c.y, acc[u]);
             }
         }
     }
+    const int r0 = dst ? dst[2 * (qb + k)] : qb + k, r1 = dst ? dst[2 * (qb + k) + 1] : -1;
 #pragma unroll
     for (int u = 0; u < kIsfLagsPerLane; ++u) {
         const int tau = lane + 64 * u;
-        if (u < nu && tau < M) fqt[(int64_t)(qb + k) * M + tau] = acc[u] * inv_n;
+        if (u < nl && tau < half) {
+            const double v = acc[u] * inv_n;
+            const int back = tau ? M - tau : 0;
+            if (r0 >= 0) {
+                fqt[(int64_t)r0 * M + tau] = v;
+                fqt[(int64_t)r0 * M + back] = v;
+            }
+            if (r1 >= 0) {
+                fqt[(int64_t)r1 * M + tau] = v;
+                fqt[(int64_t)r1 * M + back] = v;
+            }
+        }
     }
 }
 
-// S(q) contribution = sum_m |rho_q(m)|^2 / N, one lane per q (coalesced over q),
-// slices added in order.  Eight slices' rho are read before their terms are
-// added, so a lane has eight loads in flight instead of one: with a few hundred
-// q the kernel is that chain of loads (257 q x 512 slices, a served S(q)
-// request: 132 -> 28 us; 5377 q x 167: 48 -> 14 us; 100 401 q x 250: 134 -> 79
-// us, ~5 TB/s; sixteen in flight gained nothing), and the order of the additions
-// is unchanged.
-__global__ void k_ssf_from_rho(const double* __restrict__ rho, int nq, int M, double inv_n,
-                               double* __restrict__ sq) {
-    const int qi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (qi >= nq) return;
-    const double2* r = reinterpret_cast<const double2*>(rho) + qi;   // rho_q(m) at r[m nq]
-    constexpr int U = 8;
+// S(q) contribution = sum_m |rho_q(m)|^2 / N.  A workgroup takes 32 q (32
+// consecutive entries of rho, coalesced) with 8 lanes each: lane g adds the
+// slices [g seg, (g + 1) seg), seg = ceil(M / 8), in order, eight loads in flight,
+// and the eight parts are added in order, so a value depends on M and rho alone.
+// With a few hundred q the kernel is a chain of loads, which the 8 lanes cut to
+// an eighth; with many it is bound by reading rho
+// (50 201 modes x 250: 38 us, 5.3 TB/s).
+// done (or null): the last workgroup to finish publishes seq there (ticket: the
+// arrival counter, zero between calls); sq is then mapped host memory.
+constexpr int kSsfQ = 32, kSsfParts = 8;
+__global__ __launch_bounds__(kSsfQ* kSsfParts) void k_ssf_from_rho(const double* __restrict__ rho, int nq, int M,
+                                                                  double inv_n, double* __restrict__ sq,
+                                                                  unsigned* ticket, unsigned long long* done,
+                                                                  unsigned long long seq) {
+    __shared__ double part[kSsfParts][kSsfQ];
+    const int g = threadIdx.x / kSsfQ, k = threadIdx.x % kSsfQ;
+    const int qi = blockIdx.x * kSsfQ + k;
+    const int seg = (M + kSsfParts - 1) / kSsfParts;
     double acc = 0.0;
-    int m = 0;
-    for (; m + U <= M; m += U) {
-        double2 v[U];
+    if (qi < nq) {
+        const double2* r = reinterpret_cast<const double2*>(rho) + qi;   // rho_q(m) at r[m nq]
+        constexpr int U = 8;
+        int m = g * seg;
+        const int m_end = min(M, m + seg);
+        for (; m + U <= m_end; m += U) {
+            double2 v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = r[(int64_t)(m + u) * nq];
+            for (int u = 0; u < U; ++u) v[u] = r[(int64_t)(m + u) * nq];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            acc = fma(v[u].x, v[u].x, acc);
-            acc = fma(v[u].y, v[u].y, acc);
+            for (int u = 0; u < U; ++u) {
+                acc = fma(v[u].x, v[u].x, acc);
+                acc = fma(v[u].y, v[u].y, acc);
+            }
+        }
+        for (; m < m_end; ++m) {
+            const double2 v = r[(int64_t)m * nq];
+            acc = fma(v.x, v.x, acc);
+            acc = fma(v.y, v.y, acc);
         }
     }
-    for (; m < M; ++m) {
-        const double2 v = r[(int64_t)m * nq];
-        acc = fma(v.x, v.x, acc);
-        acc = fma(v.y, v.y, acc);
+    part[g][k] = acc;
+    __syncthreads();
+    if (g == 0 && qi < nq) {
+        double s = part[0][k];
+#pragma unroll
+        for (int u = 1; u < kSsfParts; ++u) s += part[u][k];
+        sq[qi] = s * inv_n;
+        if (done) __threadfence_system();
     }
-    sq[qi] = acc * inv_n;
+    if (!done) return;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        if (t + 1 == gridDim.x) {
+            __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            publish_done(done, seq);
+        }
+    }
 }
 
 // Direct minimum-image S(q) pair sum for general q: one block per (q, slice).
@@ -377,40 +541,33 @@ __global__ void k_ssf_finish(const double* __restrict__ partial, int nq, int M, 
     sq[qi] = s * inv_n;
 }
 
+// The smallest table size that holds nmax: f(std::integral_constant<int, H>).
+template <typename F>
+static hipError_t for_table_size(const int nmax[3], F f) {
+    const int h = std::max(nmax[0], std::max(nmax[1], nmax[2]));
+    if (h <= 4) return f(std::integral_constant<int, 4>{});
+    if (h <= 8) return f(std::integral_constant<int, 8>{});
+    if (h <= 16) return f(std::integral_constant<int, 16>{});
+    if (h <= 32) return f(std::integral_constant<int, 32>{});
+    return f(std::integral_constant<int, 40>{});
+}
+
 hipError_t launch_rho(bool lattice, hipStream_t st, const RhoArgs& A) {
     (void)hipGetLastError();  // drop any stale error of an earlier call
     if (A.nq <= 0) return hipSuccess;
     if (lattice) {
-        const size_t tables = sizeof(float2) * (2 * (A.nmax[0] + A.nmax[1] + A.nmax[2]) + 3) * kRhoBeadChunk;
         // the most q per lane that still leaves >= 2048 workgroups
         auto blocks = [&](int qpt) { return (int64_t)((A.nq + kRhoThreads * qpt - 1) / (kRhoThreads * qpt)) * A.num_slices; };
-        int qpt = 8;
+        int qpt = 4;
         while (qpt > 1 && blocks(qpt) < 2048) qpt >>= 1;
         dim3 g((A.nq + kRhoThreads * qpt - 1) / (kRhoThreads * qpt), A.num_slices), b(kRhoThreads);
-        // row products when a workgroup takes 1024 or more q (up to 128 rows; a
-        // q set in the reference's order has runs of n_z longer than 8, so this
-        // is rarely exceeded, and a workgroup with more rows takes the per-lane
-        // products); with fewer q per workgroup their set-up outweighs them.  The
-        // products' space first holds the row scan (256 QPT ints).
-        const int rows_cap = qpt >= 4 ? kRhoRowsMax : 0;
-        const size_t lds = tables + sizeof(float2) * rows_cap * kRhoBeadChunk + sizeof(int2) * rows_cap;
-        // set once per process (two threads racing here both set the same value)
-        static std::atomic<bool> attr_set{false};
-        if (!attr_set.load(std::memory_order_acquire)) {
-            // up to 63 + 32 + 1 KB at |n_d| <= 40, above the default 64 KB of dynamic LDS
-            // (the kernel's static LDS comes on top, within the 160 KB of a CU)
-            const void* fns[4] = {(const void*)k_rho_lattice<1>, (const void*)k_rho_lattice<2>,
-                                  (const void*)k_rho_lattice<4>, (const void*)k_rho_lattice<8>};
-            for (const void* f : fns) {
-                const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-                if (e != hipSuccess) return e;
-            }
-            attr_set.store(true, std::memory_order_release);
-        }
-        if (qpt == 8) hipLaunchKernelGGL(k_rho_lattice<8>, g, b, lds, st, A, rows_cap);
-        else if (qpt == 4) hipLaunchKernelGGL(k_rho_lattice<4>, g, b, lds, st, A, rows_cap);
-        else if (qpt == 2) hipLaunchKernelGGL(k_rho_lattice<2>, g, b, lds, st, A, rows_cap);
-        else hipLaunchKernelGGL(k_rho_lattice<1>, g, b, lds, st, A, rows_cap);
+        (void)for_table_size(A.nmax, [&](auto h) {
+            constexpr int H = decltype(h)::value;
+            if (qpt == 4) hipLaunchKernelGGL((k_rho_lattice<4, H>), g, b, 0, st, A);
+            else if (qpt == 2) hipLaunchKernelGGL((k_rho_lattice<2, H>), g, b, 0, st, A);
+            else hipLaunchKernelGGL((k_rho_lattice<1, H>), g, b, 0, st, A);
+            return hipSuccess;
+        });
     } else {
         dim3 g((A.nq + kRhoThreads - 1) / kRhoThreads, A.num_slices), b(kRhoThreads);
         hipLaunchKernelGGL(k_rho_general, g, b, 0, st, A);
@@ -418,24 +575,54 @@ hipError_t launch_rho(bool lattice, hipStream_t st, const RhoArgs& A) {
     return hipGetLastError();
 }
 
-hipError_t launch_isf(hipStream_t st, const double* rho, int nq, int M, double inv_n, double* fqt, int only_tau0) {
-    (void)hipGetLastError();  // drop any stale error of an earlier call
-    if (nq <= 0) return hipSuccess;
-    if (only_tau0) {
-        hipLaunchKernelGGL(k_ssf_from_rho, dim3((nq + 255) / 256), dim3(256), 0, st, rho, nq, M, inv_n, fqt);
-    } else {
-        dim3 g((nq + kIsfQ - 1) / kIsfQ), b(256);
-        const size_t lds = sizeof(double2) * kIsfQ * (2 * (size_t)M + 64);
+hipError_t launch_rho_matrix(hipStream_t st, const RhoMatrixArgs& A) {
+    (void)hipGetLastError();
+    const int jobs = A.job_end - A.job0;
+    if (jobs <= 0) return hipSuccess;
+    // the jobs spread evenly over the fewest workgroups of up to 16 waves; at least
+    // four waves, which share the table passes however few jobs there are
+    const int groups = (jobs + kRhoWaves - 1) / kRhoWaves;
+    const int waves = std::max(4, (jobs + groups - 1) / groups);
+    const hipError_t e = for_table_size(A.nmax, [&](auto h) {
+        constexpr int H = decltype(h)::value;
+        const size_t lds = 3 * sizeof(float2) * Phasors<H>::kEntries;   // at most 126 KB
         static std::atomic<bool> attr_set{false};
         if (!attr_set.load(std::memory_order_acquire)) {
-            // rows of M <= 512 slices need up to 68 KB of the 160 KB LDS
-            hipError_t e = hipFuncSetAttribute((const void*)k_isf_from_rho,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            if (e != hipSuccess) return e;
+            const hipError_t e1 = hipFuncSetAttribute((const void*)k_rho_matrix<H>,
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e1 != hipSuccess) return e1;
             attr_set.store(true, std::memory_order_release);
         }
-        hipLaunchKernelGGL(k_isf_from_rho, g, b, lds, st, rho, nq, M, inv_n, fqt);
+        hipLaunchKernelGGL(k_rho_matrix<H>, dim3(groups, A.num_slices), dim3(64 * waves), lds, st, A);
+        return hipSuccess;
+    });
+    return e != hipSuccess ? e : hipGetLastError();
+}
+
+hipError_t launch_isf(hipStream_t st, const double* rho, int nu, int u0, int u_end, int M, double inv_n,
+                      const int* dst, double* fqt) {
+    (void)hipGetLastError();  // drop any stale error of an earlier call
+    if (u_end <= u0) return hipSuccess;
+    dim3 g((u_end - u0 + kIsfQ - 1) / kIsfQ), b(256);
+    const size_t lds = sizeof(double2) * kIsfQ * (2 * (size_t)M + 64);
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set.load(std::memory_order_acquire)) {
+        // rows of M <= 512 slices need up to 68 KB of the 160 KB LDS
+        hipError_t e = hipFuncSetAttribute((const void*)k_isf_from_rho, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           160 * 1024);
+        if (e != hipSuccess) return e;
+        attr_set.store(true, std::memory_order_release);
     }
+    hipLaunchKernelGGL(k_isf_from_rho, g, b, lds, st, rho, nu, u0, u_end, M, inv_n, dst, fqt);
+    return hipGetLastError();
+}
+
+hipError_t launch_ssf(hipStream_t st, const double* rho, int nq, int M, double inv_n, double* sq, unsigned* ticket,
+                      unsigned long long* done, unsigned long long seq) {
+    (void)hipGetLastError();
+    if (nq <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ssf_from_rho, dim3((nq + kSsfQ - 1) / kSsfQ), dim3(kSsfQ * kSsfParts), 0, st, rho, nq, M,
+                       inv_n, sq, ticket, done, seq);
     return hipGetLastError();
 }
 
