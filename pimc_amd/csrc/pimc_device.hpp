@@ -148,21 +148,52 @@ __device__ __forceinline__ double aziz_vmid(double kd, double y, const AzizDev& 
     return rep - aziz_disp_y(kd, y, a);
 }
 
+// valueV of any bin kd >= 1 (an integer in FP64) from y, the reciprocal-root
+// estimate of |w| (kd <= |w| < kd + 1): aziz_vmix without the FP64 reciprocal,
+// which takes four issue slots.  1/kd^2 is y^2 and one Newton step, off by 4/kd^2:
+// under 4e-10 down to x = 0.1, below which the damping factor exp(-(D/x - 1)^2) <
+// e^-120 leaves nothing of the dispersion.  (512 walkers of N = 16 .. 256: 1.85 ->
+// 1.73 ms per batch, with the bin kept as an FP64 whole number.)
+template <bool BETA0 = false>
+__device__ __forceinline__ double aziz_vmix_y(double kd, double y, const AzizDev& a, double k_d) {
+    const double rep = split_exp2(BETA0 ? fma(a.rep_c1, kd, a.rep_c0) : fma(fma(a.rep_c2, kd, a.rep_c1), kd, a.rep_c0));
+    const double q = kd * kd;
+    const double r0 = y * y;
+    const double iq = fma(r0, fma(-q, r0, 1.0), r0);
+    const double disp = (iq * iq * iq) * fma(fma(a.eC10k, iq, a.eC8k), iq, a.eC6k);
+    double v = rep - disp;
+    if (kd < k_d) {
+        // as in aziz_vmix; F underflows to 0 below x = 0.01
+        const double t = fma(a.Ds * kd, iq, -1.0);
+        v = fma(-disp, split_exp2(-1.4426950408889634074 * t * t), rep);
+    }
+    return v;
+}
+
+// 1/x in FP64: the hardware estimate (~2^-23) and two Newton steps, within an ulp
+// or two of the quotient (the IEEE division takes ~10 instructions more).
+__device__ __forceinline__ double recip64(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+
 // valueV at the bin radius, FP64 arithmetic.  Requires k_eps <= k < table_length.
 __device__ __forceinline__ double aziz_v64(int k, const AzizDev& a) {
     const double x = (double)k * a.s;
-    const double rep = a.A * exp(-a.alpha * x + a.beta * x * x);
+    const double ix = recip64(x);
+    const double ix2 = ix * ix;
+    const double disp = (ix2 * ix2 * ix2) * fma(fma(a.C10, ix2, a.C8), ix2, a.C6);
+    // the repulsion is below the rounding of the difference in a wave of far bins
+    double rep = 0.0;
+    if (__builtin_amdgcn_ballot_w64(k < a.k_far)) rep = a.A * exp(-a.alpha * x + a.beta * x * x);
     if (k < a.k_hc) return a.eps * rep;
-    const double ix2 = 1.0 / (x * x);
-    const double ix6 = ix2 * ix2 * ix2;
-    const double ix8 = ix6 * ix2;
-    const double ix10 = ix8 * ix2;
     double F = 1.0;
     if (k < a.k_d) {
-        const double u = a.D / x - 1.0;
+        const double u = fma(a.D, ix, -1.0);
         F = exp(-u * u);
     }
-    return a.eps * (rep - (a.C6 * ix6 + a.C8 * ix8 + a.C10 * ix10) * F);
+    return a.eps * fma(-disp, F, rep);
 }
 
 // valuedVdr at the bin radius (src/potential.cpp:1847-1873): FP64 closed form.

@@ -63,11 +63,6 @@ __device__ __forceinline__ double sep_bins_mixed(const RowMixed& q, double xj, d
     return fma(res * y, 0.5, r0);
 }
 
-__device__ __forceinline__ int bin_mixed(const RowMixed& q, double xj, double yj, double zj) {
-    double y;
-    return (int)sep_bins_mixed(q, xj, yj, zj, &y);
-}
-
 // One lane: row bead i (held in registers) against partners j = (i + d) mod n for
 // d = d, d + G, ... < d_end (0 <= i < n, 1 <= d <= n/2), T iterations, the
 // count of the tile's first lane group (uniform, so the loop runs on a scalar
@@ -103,29 +98,59 @@ constexpr int pair_lds_plane() {
 // The tier tests run on the bin as an FP64 integer (floor of |w|, equal to the
 // truncated int for |w| >= 0), so the far tier needs no integer round trip.
 struct TierBounds {
-    double far_lo, mid_lo, hi;   // k_far, k_d, table_length
+    double far_lo, mid_lo, lo, hi;   // k_far, k_d, k_eps, table_length
 };
+__device__ __forceinline__ TierBounds tier_bounds(const AzizDev& a) {
+    return {(double)a.k_far, (double)a.k_d, (double)a.k_eps, (double)a.table_length};
+}
 template <bool BETA0, bool FAR>
-__device__ __forceinline__ double pair_term_mixed(const RowMixed& q, double x, double y, double z, const AzizDev& a,
-                                                  const AzizDev& av, int lenm1, const TierBounds& tb) {
+__device__ __forceinline__ double pair_term_mixed(const RowMixed& q, double x, double y, double z, const AzizDev& av,
+                                                  const TierBounds& tb) {
     double yr;
-    const double w = sep_bins_mixed(q, x, y, z, &yr);
+    const double kd = floor(sep_bins_mixed(q, x, y, z, &yr));
     if (FAR) {
-        const double kd = floor(w);
         if (__builtin_amdgcn_ballot_w64(!(kd >= tb.far_lo && kd < tb.hi)) == 0) return aziz_vfar(kd, yr, av);
         if (__builtin_amdgcn_ballot_w64(!(kd >= tb.mid_lo && kd < tb.hi)) == 0) return aziz_vmid<BETA0>(kd, yr, av);
     }
-    const int k = (int)w;
-    // k_eps <= k < tableLength, else V = 0 (include/potential.h:252-257): the
-    // clamped bin keeps the arithmetic finite, and only a wave holding such a
-    // pair pays for the select
-    const int kk = min(max(k, a.k_eps), lenm1);
-    double v = aziz_vmix<BETA0>(kk, av);
-    if (__builtin_amdgcn_ballot_w64(k != kk)) {
+    double v = aziz_vmix_y<BETA0>(kd, yr, av, tb.mid_lo);
+    // k_eps <= k < tableLength, else V = 0 (include/potential.h:252-257), whatever the
+    // arithmetic made of such a bin; only a wave holding one pays for the select
+    const bool in = kd >= tb.lo && kd < tb.hi;
+    if (__builtin_amdgcn_ballot_w64(!in)) {
         asm volatile("");
-        v = (k != kk) ? 0.0 : v;
+        v = in ? v : 0.0;
     }
     return v;
+}
+
+// One pair term of the exact modes (FP64 closed form, table), the bin the host's bit
+// for bit.  The mixed mode's |w| is within ~1e-6 bin of |r|/dr (2e-9 from the
+// separation, the rest from the root after one Newton step, below 2^-40 relative at
+// up to 1.5e7 bins), so away from a whole number by kBinGuard its floor is the
+// host's int(sqrt(r2)/dr); a lane nearer than that (2 in 10 000) has its bin
+// evaluated as the host does, with the reference's minimum image, IEEE root and
+// division, which would cost ~35 instructions on every pair (full action in FP64,
+// N = 777 x 61: 179 -> 155 us with the quotients of aziz_v64 as well).
+constexpr double kBinGuard = 1.0e-4;
+template <int MODE>
+__device__ __forceinline__ double pair_term_exact(const RowMixed& q, double xi, double yi, double zi, double x,
+                                                  double y, double z, const BoxDev& box, const AzizDev& a) {
+    double yr;
+    const double w = sep_bins_mixed(q, x, y, z, &yr);
+    const double f = __builtin_amdgcn_fract(w);
+    int k = (int)w;
+    // also where w is no number (coincident beads: 0 times the infinite root estimate)
+    const bool near = !(f >= kBinGuard && f <= 1.0 - kBinGuard);
+    if (__builtin_amdgcn_ballot_w64(near)) {
+        if (near) {
+            double r;
+            k = bin_exact(sep_r2<MODE>(xi, yi, zi, x, y, z, box), a.dr, &r);
+        }
+    }
+    const bool in = (unsigned)(k - a.k_eps) < (unsigned)(a.table_length - a.k_eps);
+    if (MODE == 2) return in ? a.table[k] : 0.0;
+    const double v = aziz_v64(in ? k : a.k_hc, a);
+    return in ? v : 0.0;
 }
 
 template <int MODE, int PS, bool FACTORS, bool BETA0, bool NOWRAP, bool FAR>
@@ -145,16 +170,13 @@ __device__ __forceinline__ double row_loop(const double* px, const double* py, c
     unsigned jc = (unsigned)j0 * kW;
     const int skip_d = (mask && i >= (n >> 1)) ? (n >> 1) : -1;
     RowMixed q;
-    if (MODE == 0) {
-        q.invL = box.invL;
-        q.cx = fma(-xi, box.invL, 0.5);
-        q.cy = fma(-yi, box.invL, 0.5);
-        q.cz = fma(-zi, box.invL, 0.5);
-        q.S = box.L * inv_dr;
-        q.Sh = in_vgpr(-0.5 * q.S);
-    }
-    const int lenm1 = in_vgpr(a.table_length - 1);
-    const TierBounds tb{(double)a.k_far, (double)a.k_d, (double)a.table_length};
+    q.invL = box.invL;
+    q.cx = fma(-xi, box.invL, 0.5);
+    q.cy = fma(-yi, box.invL, 0.5);
+    q.cz = fma(-zi, box.invL, 0.5);
+    q.S = box.L * inv_dr;
+    q.Sh = in_vgpr(-0.5 * q.S);
+    const TierBounds tb = tier_bounds(a);
     AzizDev av = a;
     if (MODE == 0) {
         av.rep_c1 = in_vgpr(a.rep_c1);
@@ -185,10 +207,9 @@ __device__ __forceinline__ double row_loop(const double* px, const double* py, c
     auto eval = [&](const Pos& p) -> double {
         double v;
         if (MODE == 0) {
-            v = pair_term_mixed<BETA0, FAR>(q, p.x, p.y, p.z, a, av, lenm1, tb);
+            v = pair_term_mixed<BETA0, FAR>(q, p.x, p.y, p.z, av, tb);
         } else {
-            const double r2 = sep_r2<MODE>(xi, yi, zi, p.x, p.y, p.z, box);
-            v = pair_value_from_r2<MODE>(r2, a, inv_dr);
+            v = pair_term_exact<MODE>(q, xi, yi, zi, p.x, p.y, p.z, box, a);
         }
         if (FACTORS) {
             int j = (int)(p.c / kW);
@@ -448,8 +469,7 @@ __device__ __forceinline__ double row_loop_win(const double* lw, double xi, doub
     q.cz = fma(-zi, box.invL, 0.5);
     q.S = box.L * inv_dr;
     q.Sh = in_vgpr(-0.5 * q.S);
-    const int lenm1 = in_vgpr(a.table_length - 1);
-    const TierBounds tb{(double)a.k_far, (double)a.k_d, (double)a.table_length};
+    const TierBounds tb = tier_bounds(a);
     AzizDev av = a;
     av.rep_c1 = in_vgpr(a.rep_c1);
     av.eC8k = in_vgpr(a.eC8k);
@@ -468,7 +488,7 @@ __device__ __forceinline__ double row_loop_win(const double* lw, double xi, doub
         return p;
     };
     auto eval = [&](const Pos& p) -> double {
-        double v = pair_term_mixed<BETA0, true>(q, p.x, p.y, p.z, a, av, lenm1, tb);
+        double v = pair_term_mixed<BETA0, true>(q, p.x, p.y, p.z, av, tb);
         if (FACTORS) {
             int j = w0 + (int)(p.c >> 3);
             if (j >= n) j -= n;
