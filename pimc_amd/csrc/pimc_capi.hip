@@ -571,8 +571,9 @@ static void fill_walker(pimc_ctx* c, WalkerDesc* w, int shift, const double vf[2
     w->worm = c->worm;
 }
 
-// gradVSquared(slice) for every slice into c->d_g2part (partials per slice).
-static int run_gradv2(pimc_ctx* c, const AzizDev& az) {
+// gradVSquared(slice) into c->d_g2part (partials per slice) of the even (need bit
+// 0) and odd (bit 1) slices; 0 for the others.
+static int run_gradv2(pimc_ctx* c, const AzizDev& az, int need) {
     const int M = c->desc.num_slices, N = c->desc.num_alloc;
     if (c->desc.v_mode == PIMC_V_TABLE && !az.dtable)
         return fail(c, PIMC_E_STATE, "gradVSquared in the table mode needs the dV/dr table");
@@ -582,7 +583,8 @@ static int run_gradv2(pimc_ctx* c, const AzizDev& az) {
         if ((r = ctx_dalloc(c, &c->d_g2part, (size_t)M * B))) return r;
         if (!c->d_g2slice && (r = ctx_dalloc(c, &c->d_g2slice, (size_t)M))) return r;
     }
-    const int C = gradv2_chunks(N, M, c->num_cus);
+    const int active = (need & 1 ? (M + 1) / 2 : 0) + (need & 2 ? M / 2 : 0);
+    const int C = gradv2_chunks(N, std::max(1, active), c->num_cus);
     if (C > 1 && c->cap_g2f < (size_t)M * C * N * 3) {
         int r;
         free_dev(c, c->d_g2f);
@@ -593,7 +595,7 @@ static int run_gradv2(pimc_ctx* c, const AzizDev& az) {
     int blocks = 0;
     c->timed_begin(5);
     HIP_OR_FAIL(c, launch_gradv2(c->desc.v_mode, c->stream, c->d_pos, c->plane, N, M, c->d_nbs, c->box, az,
-                                 c->lds_beads, c->d_g2part, &blocks, C, c->d_g2f));
+                                 c->lds_beads, c->d_g2part, &blocks, C, c->d_g2f, need));
     c->timed_end();
     c->g2_blocks = blocks;
     return PIMC_OK;
@@ -842,7 +844,7 @@ int pimc_gradv_squared(pimc_ctx* c, double* g2) {
         az.dtable = table_cache().get(c->desc.aziz_year, 1, az.table_length, &err);
         if (!az.dtable) return fail(c, PIMC_E_NOMEM, err);
     }
-    if ((r = run_gradv2(c, az))) return r;
+    if ((r = run_gradv2(c, az, 3))) return r;
     // the per-block partials of every slice, summed in block order as the
     // pair kernel's finalisation sums them into the corrected action
     const int B = c->g2_blocks;
@@ -876,7 +878,13 @@ int pimc_potential_slices(pimc_ctx* c, double* v_slices, int32_t* sep_hist) {
     return PIMC_OK;
 }
 
-int pimc_total_action(pimc_ctx* c, int shift, const double vfactor[2], double* action, double* v_slices) {
+}  // extern "C"
+
+// pimc_total_action; g2 (or null, with v_slices): gradVSquared of the slices whose
+// gradVFactor is finite (the context's action carries the correction).  Without
+// with_correction the action leaves the correction out and only V(slice) is asked for.
+static int total_action(pimc_ctx* c, int shift, const double vfactor[2], double* action, double* v_slices, double* g2,
+                        bool with_correction = true) {
     if (!c || !action) return fail(c, PIMC_E_ARG, "null argument");
     if (!c->have_path) return fail(c, PIMC_E_STATE, "no path uploaded");
     if (shift < 1) return fail(c, PIMC_E_ARG, "shift must be >= 1");
@@ -893,8 +901,8 @@ int pimc_total_action(pimc_ctx* c, int shift, const double vfactor[2], double* a
         c->walker_valid = true;
     }
     if (c->n_tiles > 0) {
-        const bool cor = c->correction();
-        if (cor && (r = run_gradv2(c, az))) return r;
+        const bool cor = with_correction && c->correction();
+        if (cor && (r = run_gradv2(c, az, (c->gvf[0] > kCorrEps ? 1 : 0) | (c->gvf[1] > kCorrEps ? 2 : 0)))) return r;
         const bool spatial = c->pair_spatial && c->desc.v_mode == PIMC_V_MIXED;
         if (spatial && c->perm_version != c->path_version) {
             HIP_OR_FAIL(c, launch_slice_order(c->stream, c->d_slices, M, c->d_pos, c->box.invL, c->d_perm));
@@ -902,12 +910,17 @@ int pimc_total_action(pimc_ctx* c, int shift, const double vfactor[2], double* a
         }
         const KernelTimer kt = c->kernel_timer(0);
         const unsigned long long seq = ++c->seq;
+        // the slice values go straight into mapped memory beside the action, so one
+        // spin on the completion word covers both (a copy and a stream
+        // synchronisation took ~10 us more)
+        const bool mapped = v_slices && 2 * M <= pimc_ctx::kMappedSq;
         HIP_OR_FAIL(c, launch_pair_action(c->desc.v_mode, c->stream, c->d_tiles, c->n_tiles, c->d_ranges, c->n_groups,
                                           c->d_slices, M, c->d_walker, 1, c->d_pos, az, c->pair_lds, c->d_partials,
                                           c->d_vslice, c->d_map, &kt, true, c->d_done(), seq,
                                           cor ? c->d_g2part : nullptr, c->g2_blocks, c->d_g2slice,
-                                          spatial ? c->d_perm : nullptr));
-        if (v_slices) {
+                                          spatial ? c->d_perm : nullptr,
+                                          mapped ? c->d_map + pimc_ctx::kSqSlot : nullptr));
+        if (v_slices && !mapped) {
             HIP_OR_FAIL(c, hipMemcpyAsync(c->h_stage, c->d_vslice, sizeof(double) * M, hipMemcpyDeviceToHost,
                                           c->stream));
             HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
@@ -915,11 +928,19 @@ int pimc_total_action(pimc_ctx* c, int shift, const double vfactor[2], double* a
             return fail(c, PIMC_E_HIP, "pair action: completion not published");
         }
         *action = c->h_map[0];
-        if (v_slices)
+        if (v_slices) {
+            const double* v = mapped ? c->h_map + pimc_ctx::kSqSlot : c->h_stage;
             for (int m = 0; m < M; ++m) {
                 v_slices[2 * m] = 0.0;
-                v_slices[2 * m + 1] = c->h_stage[m];
+                v_slices[2 * m + 1] = v[m];
             }
+            if (g2) {
+                if (mapped)
+                    std::memcpy(g2, v + M, sizeof(double) * M);
+                else
+                    HIP_OR_FAIL(c, hipMemcpy(g2, c->d_g2slice, sizeof(double) * M, hipMemcpyDeviceToHost));
+            }
+        }
     } else {
         *action = 0.0;
         if (v_slices)
@@ -928,9 +949,21 @@ int pimc_total_action(pimc_ctx* c, int shift, const double vfactor[2], double* a
     return PIMC_OK;
 }
 
-// Per-slice virial sums (pimc_virial.hip), summed over each slice's workgroups
-// in order: S [M][kVirialTerms].
-static int run_virial(pimc_ctx* c, const int32_t* next_links, int window, std::vector<double>& S) {
+extern "C" {
+
+int pimc_total_action(pimc_ctx* c, int shift, const double vfactor[2], double* action, double* v_slices) {
+    return total_action(c, shift, vfactor, action, v_slices, nullptr);
+}
+
+// The per-workgroup virial sums on their way (pimc_virial.hip): in mapped memory
+// once a later kernel of the stream has published, or on the device.
+struct VirialPending {
+    int blocks = 0;
+    const double* mapped = nullptr;
+};
+
+// Launches the virial kernels.
+static int launch_virial_terms(pimc_ctx* c, const int32_t* next_links, int window, VirialPending* V) {
     const int M = c->desc.num_slices, N = c->desc.num_alloc;
     if (window < 1) return fail(c, PIMC_E_ARG, "virial window must be >= 1");
     int r;
@@ -1003,7 +1036,11 @@ static int run_virial(pimc_ctx* c, const int32_t* next_links, int window, std::v
     A.t_odd = c->gvf[1] > kCorrEps;
     A.lds_beads = N <= kLdsBeads ? N : 0;
     A.box = c->box;
-    A.part = c->d_virial;
+    // a few thousand sums go straight into mapped memory, past the slice values
+    const bool mapped = 2 * (size_t)M + need <= (size_t)pimc_ctx::kMappedSq;
+    V->mapped = mapped ? c->h_map + pimc_ctx::kSqSlot + 2 * M : nullptr;
+    A.part = mapped ? c->d_map + pimc_ctx::kSqSlot + 2 * M : c->d_virial;
+    A.part_on_host = mapped;
     A.chunks = gradv2_chunks(N, M, c->num_cus);
     A.fpart = nullptr;
     if (A.chunks > 1) {
@@ -1016,14 +1053,26 @@ static int run_virial(pimc_ctx* c, const int32_t* next_links, int window, std::v
         }
         A.fpart = c->d_vf;
     }
-    int blocks = 0;
     c->timed_begin(7);
-    HIP_OR_FAIL(c, launch_virial(c->desc.v_mode, c->stream, A, az, &blocks));
+    HIP_OR_FAIL(c, launch_virial(c->desc.v_mode, c->stream, A, az, &V->blocks));
     c->timed_end();
-    std::vector<double> part(need);
-    HIP_OR_FAIL(c, hipMemcpyAsync(part.data(), c->d_virial, sizeof(double) * need, hipMemcpyDeviceToHost,
-                                  c->stream));
-    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    return PIMC_OK;
+}
+
+// Per-slice virial sums S [M][kVirialTerms], each slice's workgroups in order.
+// published: a later kernel's publication has been waited for.
+static int collect_virial(pimc_ctx* c, const VirialPending& V, bool published, std::vector<double>& S) {
+    const int M = c->desc.num_slices, blocks = V.blocks;
+    const size_t need = (size_t)M * blocks * kVirialTerms;
+    std::vector<double> copy;
+    const double* part = V.mapped;
+    if (!part) {
+        copy.resize(need);
+        HIP_OR_FAIL(c, hipMemcpyAsync(copy.data(), c->d_virial, sizeof(double) * need, hipMemcpyDeviceToHost,
+                                      c->stream));
+        part = copy.data();
+    }
+    if (!V.mapped || !published) HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     S.assign((size_t)M * kVirialTerms, 0.0);
     for (int m = 0; m < M; ++m)
         for (int b = 0; b < blocks; ++b)
@@ -1055,8 +1104,10 @@ int pimc_virial_terms(pimc_ctx* c, const int32_t* next_links, int window, double
     if (!c || !out6) return fail(c, PIMC_E_ARG, "null argument");
     if (!c->have_path) return fail(c, PIMC_E_STATE, "no path uploaded");
     std::vector<double> S;
-    int r = run_virial(c, next_links, window, S);
+    VirialPending V;
+    int r = launch_virial_terms(c, next_links, window, &V);
     if (r) return r;
+    if ((r = collect_virial(c, V, false, S))) return r;
     virial_slice_terms(c, S, out6);
     return PIMC_OK;
 }
@@ -1066,9 +1117,14 @@ int pimc_virial_energy(pimc_ctx* c, const int32_t* next_links, int window, doubl
     if (!c->have_path) return fail(c, PIMC_E_STATE, "no path uploaded");
     const int M = c->desc.num_slices;
     std::vector<double> vs(2 * (size_t)M), terms(6 * (size_t)M), S;
-    int r = pimc_potential_slices(c, vs.data(), nullptr);
+    // the virial kernels, then the pair kernel, one wait for both
+    VirialPending V;
+    const double vf1[2] = {1.0, 1.0};
+    double act = 0.0;
+    int r = launch_virial_terms(c, next_links, window, &V);
     if (r) return r;
-    if ((r = run_virial(c, next_links, window, S))) return r;
+    if ((r = total_action(c, 1, vf1, &act, vs.data(), nullptr, false))) return r;
+    if ((r = collect_virial(c, V, c->n_tiles > 0, S))) return r;
     virial_slice_terms(c, S, terms.data());
     // VirialEnergyEstimator::accumulate (src/estimator.cpp:1086-1251), one call
     long on = 0;
@@ -1217,8 +1273,7 @@ int pimc_energy(pimc_ctx* c, const int32_t* next_links, double mu, double* out9)
     if (!c->have_path) return fail(c, PIMC_E_STATE, "no path uploaded");
     const int M = c->desc.num_slices, N = c->desc.num_alloc;
     std::vector<double> vs(2 * (size_t)M);
-    int r = pimc_potential_slices(c, vs.data(), nullptr);
-    if (r) return r;
+    int r;
     int* d_next = nullptr;
     if (next_links) {
         // the last call's links stay on the device: the same links again are
@@ -1246,11 +1301,17 @@ int pimc_energy(pimc_ctx* c, const int32_t* next_links, double mu, double* out9)
         }
         d_next = c->d_enext;
     }
+    // the link sum, then the slice values and (where the action carries the
+    // correction) gradVSquared(slice): one wait for all of them
+    constexpr int kKineticSlot = 40;
     HIP_OR_FAIL(c, launch_kinetic(c->stream, c->d_pos, c->plane, N, M, c->d_nbs, d_next, c->box, c->d_kin_partials,
-                                  1024, c->d_out + 8));
-    HIP_OR_FAIL(c, hipMemcpyAsync(c->h_out, c->d_out + 8, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    const double link_sum = c->h_out[0];
+                                  1024, c->d_map + kKineticSlot));
+    std::vector<double> g2(M, 0.0);
+    const double vf1[2] = {1.0, 1.0};
+    double act = 0.0;
+    if ((r = total_action(c, 1, vf1, &act, vs.data(), c->correction() ? g2.data() : nullptr))) return r;
+    if (c->n_tiles == 0) HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    const double link_sum = c->h_map[kKineticSlot];
     // EnergyEstimator::accumulate (src/estimator.cpp:940-1029) with the context's action factors
     long on = 0;
     for (auto v : c->h_on) on += v;
@@ -1261,11 +1322,6 @@ int pimc_energy(pimc_ctx* c, const int32_t* next_links, double mu, double* out9)
     const double kinNorm = (1.0 / (4.0 * lambda * tau)) / (tau * M);
     const double classical = (0.5 * 3 / tau) * Np;
     double totK = -link_sum * kinNorm;
-    // gradVSquared(slice) from the same pass when the action carries the correction
-    std::vector<double> g2(M, 0.0);
-    if (c->correction()) {
-        HIP_OR_FAIL(c, hipMemcpy(g2.data(), c->d_g2slice, sizeof(double) * M, hipMemcpyDeviceToHost));
-    }
     // derivPotentialActionLambda / Tau (src/action.cpp:751-802) and the operator
     // V on every period-th slice
     double t1 = 0.0, t2 = 0.0, vop0 = 0.0, vop1 = 0.0;
@@ -1337,6 +1393,8 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
     A.gvf0 = c->gvf[0];
     A.gvf1 = c->gvf[1];
     A.lambda = c->desc.lambda;
+    // no separation exceeds sqrt(3)/2 L: every bead is in the list of either position
+    A.gnn_shared = c->box.ngrid < 4 && c->box.rc2 > 0.76 * c->box.L * c->box.L;
     if (cor) {
         const size_t need = (size_t)c->cap_req * 2 * A.gnn_chunks * 4;
         if ((size_t)c->cap_gnn < need) {

@@ -88,6 +88,7 @@ struct VirialArgs {
     int lds_beads;       // slices with at most this many beads are staged in LDS
     BoxDev box;
     double* part;        // [M][blocks][kVirialTerms]
+    int part_on_host;    // part is mapped host memory, read after a later kernel's publication
     int chunks;          // partner chunks (1: one pass per row block)
     double* fpart;       // chunk partials [M][chunks][nalloc][9] = F, T (chunks > 1)
 };
@@ -130,6 +131,7 @@ struct VnnArgs {
     // gradient correction: gradVnnSquared partials [n_beads][2][gnn_chunks][4] (null: none)
     const double* gnn_part;
     int gnn_chunks;
+    int gnn_shared;        // one workgroup serves both positions (their lists are the same)
     double gvf0, gvf1, lambda;
     int cor_any_shift;     // evaluate the correction at any shift (potentialActionCorrection)
     double* per_bead_cor;  // [n_beads][2] corrections at the old / new position, or null
@@ -214,7 +216,8 @@ __device__ __forceinline__ int xcd_contiguous_item(int b, int G) {
 // ---- launchers (defined in pimc_pair.hip / pimc_sq.hip) ----
 // The persistent row-tile pair kernel over G workgroups, then (finalize != 0)
 // the single-workgroup slice and walker sums.
-// done (host-mapped, or null) is set to seq after action has been written.
+// done (host-mapped, or null) is set to seq after action has been written, and
+// v_host (host-mapped, or null) receives the slice sums before it.
 // g2_part (or null): gradVSquared partials [n_slices][g2_blocks] whose slice sums
 // (written to g2_slice) enter the walkers' actions with the gradient correction.
 // perm (or null): mixed mode, the window form (k_pair_window, tiles from
@@ -226,7 +229,7 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
                               double* action, const KernelTimer* timer = nullptr, bool finalize = true,
                               unsigned long long* done = nullptr, unsigned long long seq = 0,
                               const double* g2_part = nullptr, int g2_blocks = 0, double* g2_slice = nullptr,
-                              const int* perm = nullptr);
+                              const int* perm = nullptr, double* v_host = nullptr);
 // Spatial order of every slice (slices of at most kLdsBeads beads, one box):
 // perm[slices[s].pos + t], t < slices[s].n, lists slice s's beads by the index of
 // their cell along a Hilbert curve through a 32^3 grid over the box, ties by
@@ -250,10 +253,11 @@ constexpr uint32_t kVdirOffReq = karg_align(sizeof(VnnArgs), alignof(VnnInline))
 constexpr uint32_t kVdirOffAz = karg_align(kVdirOffReq + sizeof(VnnInline), alignof(AzizDev));
 constexpr uint32_t kVdirOffOut = karg_align(kVdirOffAz + sizeof(AzizDev), alignof(VnnDirectOut*));
 constexpr uint32_t kVdirBytes = kVdirOffOut + sizeof(VnnDirectOut*);
-// gradVSquared(slice) partials [M][blocks_per_slice] for every slice.
+// gradVSquared(slice) partials [M][blocks_per_slice] for the even (need bit 0) and
+// odd (bit 1) slices, 0 for the others.
 hipError_t launch_gradv2(int mode, hipStream_t st, const double* pos, int64_t plane, int nalloc, int num_slices,
                          const int* nbs, const BoxDev& box, const AzizDev& az, int lds_beads, double* part,
-                         int* blocks_per_slice, int chunks = 1, double* fpart = nullptr);
+                         int* blocks_per_slice, int chunks = 1, double* fpart = nullptr, int need = 3);
 // Partner chunks of the gradVSquared sum that fill the CUs (1: one pass).
 int gradv2_chunks(int nalloc, int num_slices, int num_cus);
 // Device-resident chain (pimc_dchain.hip): one workgroup runs n_moves moves.

@@ -636,7 +636,9 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_window(const RowTile* __r
 // 1024 lanes: the partials and the slices' item ranges are first pulled into LDS
 // with every load in flight; then each lane sums the items of one slice in item
 // order, and one wave per walker sums its slices (lanes strided, fixed shuffle
-// tree), so the result depends only on the work list, never on timing.
+// tree), so the result depends only on the work list, never on timing.  v_host (or
+// null): mapped host memory, also receives the slice sums and, after them, the
+// slices' gradVSquared.
 constexpr int kFinThreads = 1024;
 constexpr int kFinLds = 5120;      // partials staged in LDS (beyond: read from HBM)
 constexpr int kFinSlices = 1024;   // slice ranges / sums staged in LDS (beyond: HBM)
@@ -647,7 +649,8 @@ __global__ __launch_bounds__(kFinThreads) void k_pair_finalize(int n_items, cons
                                                               double* __restrict__ action,
                                                               unsigned long long* done, unsigned long long seq,
                                                               const double* __restrict__ g2_part, int g2_blocks,
-                                                              double* __restrict__ g2_slice) {
+                                                              double* __restrict__ g2_slice,
+                                                              double* __restrict__ v_host) {
     __shared__ double sp[kFinLds];
     __shared__ double vs[kFinSlices];
     __shared__ double gs[kFinSlices];
@@ -669,13 +672,16 @@ __global__ __launch_bounds__(kFinThreads) void k_pair_finalize(int n_items, cons
         for (int k = b; k < e; ++k) v += src[k];
         v_slice[sl] = v;
         if (small) vs[sl] = v;
+        if (v_host) v_host[sl] = v;
         if (g2_part) {
             double g = 0.0;
             for (int b2 = 0; b2 < g2_blocks; ++b2) g += g2_part[(int64_t)sl * g2_blocks + b2];
             g2_slice[sl] = g;
             if (small) gs[sl] = g;
+            if (v_host) v_host[n_slices + sl] = g;
         }
     }
+    if (v_host) __threadfence_system();
     __threadfence_block();   // v_slice is re-read below when the slices do not fit in LDS
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -871,16 +877,24 @@ __device__ __forceinline__ double force2(P px, P py, P pz, int n, int i, const B
 
 // gradVSquared(slice) (src/action.cpp:1188-1223): block (b, m) takes rows
 // 256 b .. 256 b + 255 of slice m; one partial per block, summed in block order.
+// need (here and in the kernels below): bit m % 2, the slices to evaluate.  An
+// action weights only those with a finite gradVFactor (GSF: the odd ones), so the
+// others' partials are 0 (with gnn_shared below, the full GSF action and three moves
+// at N = 256 x 166: 132 -> 115 us).
 template <int MODE>
 __global__ __launch_bounds__(256) void k_gradv2(const double* __restrict__ pos, int64_t plane, int nalloc,
                                                 const int* __restrict__ nbs, BoxDev box, AzizDev az, int lds_beads,
-                                                double* __restrict__ part) {
+                                                int need, double* __restrict__ part) {
     extern __shared__ double lds[];
     __shared__ double red[4];
     double* lx = lds;
     double* ly = lds + lds_beads;
     double* lz = lds + 2 * lds_beads;
     const int m = blockIdx.y, b = blockIdx.x;
+    if (!((need >> (m & 1)) & 1)) {
+        if (threadIdx.x == 0) part[(int64_t)m * gridDim.x + b] = 0.0;
+        return;
+    }
     const int n = nbs[m];
     const double* px = pos + (int64_t)m * nalloc;
     const double* py = px + plane;
@@ -909,12 +923,14 @@ __global__ __launch_bounds__(256) void k_gradv2(const double* __restrict__ pos, 
 template <int MODE>
 __global__ __launch_bounds__(256) void k_gradv2_chunk(const double* __restrict__ pos, int64_t plane, int nalloc,
                                                       const int* __restrict__ nbs, BoxDev box, AzizDev az,
-                                                      int lds_beads, int C, double* __restrict__ fpart) {
+                                                      int lds_beads, int C, int need,
+                                                      double* __restrict__ fpart) {
     extern __shared__ double lds[];
     double* lx = lds;
     double* ly = lds + lds_beads;
     double* lz = lds + 2 * lds_beads;
     const int m = blockIdx.y, b = blockIdx.x / C, c = blockIdx.x - b * C;
+    if (!((need >> (m & 1)) & 1)) return;
     const int n = nbs[m];
     const double* px = pos + (int64_t)m * nalloc;
     const double* py = px + plane;
@@ -969,10 +985,11 @@ __global__ __launch_bounds__(256) void k_gradv2_chunk(const double* __restrict__
 // gradV evaluations of k_gradv2_chunk for the same partial layout.
 __global__ __launch_bounds__(256) void k_gradv2_sym(const double* __restrict__ pos, int64_t plane, int nalloc,
                                                     const int* __restrict__ nbs, BoxDev box, AzizDev az, int C,
-                                                    double* __restrict__ fpart) {
+                                                    int need, double* __restrict__ fpart) {
     __shared__ double lp[3][256];
     __shared__ double fj[4][3][256];
     const int m = blockIdx.y, c = blockIdx.x;
+    if (!((need >> (m & 1)) & 1)) return;
     const int n = nbs[m];
     const int i = threadIdx.x, wave = threadIdx.x >> 6;
     const double* px = pos + (int64_t)m * nalloc;
@@ -1019,13 +1036,13 @@ __global__ __launch_bounds__(256) void k_gradv2_sym(const double* __restrict__ p
     }
 }
 
-__global__ __launch_bounds__(256) void k_gradv2_sum(const int* __restrict__ nbs, int nalloc, int C,
+__global__ __launch_bounds__(256) void k_gradv2_sum(const int* __restrict__ nbs, int nalloc, int C, int need,
                                                     const double* __restrict__ fpart, double* __restrict__ part) {
     __shared__ double red[4];
     const int m = blockIdx.y, b = blockIdx.x;
     const int i = b * 256 + threadIdx.x;
     double f2 = 0.0;
-    if (i < nbs[m]) {
+    if (i < nbs[m] && ((need >> (m & 1)) & 1)) {
         double fx = 0.0, fy = 0.0, fz = 0.0;
         for (int c = 0; c < C; ++c) {
             const double* o = fpart + (((int64_t)m * C + c) * nalloc + i) * 3;
@@ -1059,16 +1076,21 @@ __device__ __forceinline__ double group16_sum(double v) {
 // old (y even) or new (y odd) position of request bead y/2.  Every workgroup
 // builds the bead's interaction list (the Vnn partner set, in index order) in
 // LDS; workgroup c takes list entries bead2 = 16c .. 16c+15, 16 lanes each over
-// bead3, and writes {sum of |F2|^2 + 2 F2.F3, F1} with F1 = -sum F2.
+// bead3, and writes {sum of |F2|^2 + 2 F2.F3, F1} with F1 = -sum F2.  F3 depends on
+// the list alone, so where every bead is in it whatever the position (gnn_shared:
+// rc beyond the largest separation, no cells) one workgroup serves both positions
+// and y is the bead.
 template <int MODE>
 __device__ __forceinline__ void gradvnn_body(const VnnArgs& A, const VnnInline& req, const AzizDev& az, int lds_beads,
                                              double* __restrict__ part, int c, int y) {
     extern __shared__ double lds[];   // x | y | z (lds_beads each), then the list (int[nalloc])
     __shared__ int wcount[4];
     __shared__ int list_n;
-    __shared__ double red[4][4];
-    const int bead = y >> 1, which = y & 1;
+    __shared__ double red[4][8];
+    const int bead = A.gnn_shared ? y : y >> 1, which = A.gnn_shared ? 0 : y & 1;
     const VnnBead q = A.beads ? A.beads[bead] : req.beads[bead];
+    // a slice without a finite gradVFactor has no correction: its partials are not read
+    if (!(((q.slice & 1) ? A.gvf1 : A.gvf0) > kCorrEps)) return;
     const VnnSubject v = vnn_subject(A, q);
     double* out = part + (((int64_t)bead * 2 + which) * A.gnn_chunks + c) * 4;
     if (which == 1 && !v.has_new) {
@@ -1148,18 +1170,22 @@ __device__ __forceinline__ void gradvnn_body(const VnnArgs& A, const VnnInline& 
     f3x = group16_sum(f3x);
     f3y = group16_sum(f3y);
     f3z = group16_sum(f3z);
+    // the position's terms: lane 0 of a group at (x1, y1, z1); where the list serves
+    // both positions, lane 1 takes the new one
     double term = 0.0, f1x = 0.0, f1y = 0.0, f1z = 0.0;
-    if (n2 < nl && gl == 0) {
+    const bool second = A.gnn_shared && gl == 1;
+    if (n2 < nl && (gl == 0 || (second && v.has_new))) {
+        const double ax = second ? v.nx : x1, ay = second ? v.ny : y1, az1 = second ? v.nz : z1;
         // beadSep = Path::getSeparation(bead2, bead1) = r2 - r1
         double dx, dy, dz;
         if (MODE == 0) {
-            dx = min_image_fast(x2 - x1, A.box.L, A.box.invL);
-            dy = min_image_fast(y2 - y1, A.box.L, A.box.invL);
-            dz = min_image_fast(z2 - z1, A.box.L, A.box.invL);
+            dx = min_image_fast(x2 - ax, A.box.L, A.box.invL);
+            dy = min_image_fast(y2 - ay, A.box.L, A.box.invL);
+            dz = min_image_fast(z2 - az1, A.box.L, A.box.invL);
         } else {
-            dx = min_image_exact(x2 - x1, A.box.L, A.box.invL);
-            dy = min_image_exact(y2 - y1, A.box.L, A.box.invL);
-            dz = min_image_exact(z2 - z1, A.box.L, A.box.invL);
+            dx = min_image_exact(x2 - ax, A.box.L, A.box.invL);
+            dy = min_image_exact(y2 - ay, A.box.L, A.box.invL);
+            dz = min_image_exact(z2 - az1, A.box.L, A.box.invL);
         }
         const double g = grad_factor_from_r2<MODE>(norm2_exact(dx, dy, dz), az, inv_dr);
         const double f2x = g * dx, f2y = g * dy, f2z = g * dz;
@@ -1168,19 +1194,28 @@ __device__ __forceinline__ void gradvnn_body(const VnnArgs& A, const VnnInline& 
         f1y = -f2y;
         f1z = -f2z;
     }
-    term = wave_sum(term);
-    f1x = wave_sum(f1x);
-    f1y = wave_sum(f1y);
-    f1z = wave_sum(f1z);
-    if (lane == 0) {
-        red[wave][0] = term;
-        red[wave][1] = f1x;
-        red[wave][2] = f1y;
-        red[wave][3] = f1z;
+    // lanes 0, 16, 32 and 48 of a wave hold the first position's terms, lanes 1, 17,
+    // 33 and 49 the second's
+    term += __shfl_xor(term, 16, 64);
+    term += __shfl_xor(term, 32, 64);
+    f1x += __shfl_xor(f1x, 16, 64);
+    f1x += __shfl_xor(f1x, 32, 64);
+    f1y += __shfl_xor(f1y, 16, 64);
+    f1y += __shfl_xor(f1y, 32, 64);
+    f1z += __shfl_xor(f1z, 16, 64);
+    f1z += __shfl_xor(f1z, 32, 64);
+    if (lane < 2) {
+        red[wave][4 * lane + 0] = term;
+        red[wave][4 * lane + 1] = f1x;
+        red[wave][4 * lane + 2] = f1y;
+        red[wave][4 * lane + 3] = f1z;
     }
     __syncthreads();
-    if (threadIdx.x < 4) out[threadIdx.x] = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) +
-                                            red[3][threadIdx.x];
+    const int t = threadIdx.x;
+    if (t < (A.gnn_shared ? 8 : 4)) {
+        double* o = t < 4 ? out + t : out + (int64_t)A.gnn_chunks * 4 + (t - 4);
+        *o = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+    }
 }
 template <int MODE>
 __global__ __launch_bounds__(256) void k_gradvnn(VnnArgs A, VnnInline req, AzizDev az, int lds_beads,
@@ -1533,11 +1568,17 @@ __global__ __launch_bounds__(256) void k_kinetic(const double* __restrict__ pos,
 }
 
 // out[0] = sum of n partials in order
-__global__ void k_sum_partials(const double* __restrict__ partials, int n, double* __restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// One workgroup; out is mapped host memory, read after a later kernel's publication.
+__global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__ partials, int n,
+                                                      double* __restrict__ out) {
+    __shared__ double red[4];
     double tot = 0.0;
-    for (int k = 0; k < n; ++k) tot += partials[k];
-    out[0] = tot;
+    for (int k = threadIdx.x; k < n; k += 256) tot += partials[k];
+    const double s = block_sum<256>(tot, red);
+    if (threadIdx.x == 0) {
+        out[0] = s;
+        __threadfence_system();
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1577,7 +1618,7 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
                               const double* pos, const AzizDev& az, int lds_beads, double* partials, double* v_slice,
                               double* action, const KernelTimer* timer, bool finalize, unsigned long long* done,
                               unsigned long long seq, const double* g2_part, int g2_blocks, double* g2_slice,
-                              const int* perm) {
+                              const int* perm, double* v_host) {
     (void)hipGetLastError();  // drop any stale error of an earlier call
     if (n_tiles <= 0 || G <= 0) return hipSuccess;
     const bool spatial = perm != nullptr;
@@ -1615,7 +1656,7 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
     if (timer && timer->stop) (void)hipEventRecord(timer->stop, st);
     if (finalize)
         hipLaunchKernelGGL(k_pair_finalize, dim3(1), dim3(kFinThreads), 0, st, n_tiles, slices, n_slices, walkers,
-                           n_walkers, partials, v_slice, action, done, seq, g2_part, g2_blocks, g2_slice);
+                           n_walkers, partials, v_slice, action, done, seq, g2_part, g2_blocks, g2_slice, v_host);
     return hipGetLastError();
 }
 
@@ -1736,7 +1777,7 @@ hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInlin
         // one launch for both workgroup sets (a timed call keeps two, so each
         // kernel has its own duration)
         const size_t lds = sizeof(double) * 3 * (size_t)lds_beads + sizeof(int) * (size_t)A.nalloc;
-        dim3 gg(A.chunks * A.n_beads + A.gnn_chunks * 2 * A.n_beads);
+        dim3 gg(A.chunks * A.n_beads + A.gnn_chunks * (A.gnn_shared ? 1 : 2) * A.n_beads);
         if (mode == 0)
             hipLaunchKernelGGL(k_vnn_gnn<0>, gg, dim3(256), lds, st, A, req, az, lds_beads, gnn_part);
         else if (mode == 1)
@@ -1756,7 +1797,7 @@ hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInlin
     if (gnn_part) {
         VnnArgs B = A;
         const size_t lds = sizeof(double) * 3 * (size_t)lds_beads + sizeof(int) * (size_t)A.nalloc;
-        dim3 gg(A.gnn_chunks, 2 * A.n_beads);
+        dim3 gg(A.gnn_chunks, (A.gnn_shared ? 1 : 2) * A.n_beads);
         if (gnn_timer && gnn_timer->start) (void)hipEventRecord(gnn_timer->start, st);
         if (mode == 0)
             hipLaunchKernelGGL(k_gradvnn<0>, gg, dim3(256), lds, st, B, req, az, lds_beads, gnn_part);
@@ -1772,38 +1813,38 @@ hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInlin
 
 hipError_t launch_gradv2(int mode, hipStream_t st, const double* pos, int64_t plane, int nalloc, int num_slices,
                          const int* nbs, const BoxDev& box, const AzizDev& az, int lds_beads, double* part,
-                         int* blocks_per_slice, int chunks, double* fpart) {
+                         int* blocks_per_slice, int chunks, double* fpart, int need) {
     (void)hipGetLastError();
     const int B = (nalloc + 255) / 256;
     *blocks_per_slice = B;
     const size_t lds = sizeof(double) * 3 * (size_t)lds_beads;
     if (chunks > 1 && fpart && mode == 0 && nalloc <= 256) {
         hipLaunchKernelGGL(k_gradv2_sym, dim3(chunks, num_slices), dim3(256), 0, st, pos, plane, nalloc, nbs, box, az,
-                           chunks, fpart);
-        hipLaunchKernelGGL(k_gradv2_sum, dim3(B, num_slices), dim3(256), 0, st, nbs, nalloc, chunks, fpart, part);
+                           chunks, need, fpart);
+        hipLaunchKernelGGL(k_gradv2_sum, dim3(B, num_slices), dim3(256), 0, st, nbs, nalloc, chunks, need, fpart, part);
         return hipGetLastError();
     }
     if (chunks > 1 && fpart) {
         dim3 gc(B * chunks, num_slices), b(256);
         if (mode == 0)
             hipLaunchKernelGGL(k_gradv2_chunk<0>, gc, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, chunks,
-                               fpart);
+                               need, fpart);
         else if (mode == 1)
             hipLaunchKernelGGL(k_gradv2_chunk<1>, gc, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, chunks,
-                               fpart);
+                               need, fpart);
         else
             hipLaunchKernelGGL(k_gradv2_chunk<2>, gc, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, chunks,
-                               fpart);
-        hipLaunchKernelGGL(k_gradv2_sum, dim3(B, num_slices), b, 0, st, nbs, nalloc, chunks, fpart, part);
+                               need, fpart);
+        hipLaunchKernelGGL(k_gradv2_sum, dim3(B, num_slices), b, 0, st, nbs, nalloc, chunks, need, fpart, part);
         return hipGetLastError();
     }
     dim3 g(B, num_slices), b(256);
     if (mode == 0)
-        hipLaunchKernelGGL(k_gradv2<0>, g, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, part);
+        hipLaunchKernelGGL(k_gradv2<0>, g, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, need, part);
     else if (mode == 1)
-        hipLaunchKernelGGL(k_gradv2<1>, g, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, part);
+        hipLaunchKernelGGL(k_gradv2<1>, g, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, need, part);
     else
-        hipLaunchKernelGGL(k_gradv2<2>, g, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, part);
+        hipLaunchKernelGGL(k_gradv2<2>, g, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, need, part);
     return hipGetLastError();
 }
 
@@ -1863,7 +1904,7 @@ hipError_t launch_kinetic(hipStream_t st, const double* pos, int64_t plane, int 
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(k_kinetic, dim3(blocks), dim3(256), 0, st, pos, plane, nalloc, num_slices, nbs, next, box,
                        partials);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(64), 0, st, partials, blocks, out);
+    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, partials, blocks, out);
     return hipGetLastError();
 }
 

@@ -222,6 +222,7 @@ __global__ __launch_bounds__(256) void k_virial(VirialArgs A, AzizDev az) {
     if (threadIdx.x < kVirialTerms) {
         const int q = threadIdx.x;
         A.part[((int64_t)m * gridDim.x + b) * kVirialTerms + q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
+        if (A.part_on_host) __threadfence_system();
     }
 }
 
@@ -291,6 +292,7 @@ __global__ __launch_bounds__(256) void k_virial_sum(VirialArgs A) {
     if (threadIdx.x < kVirialTerms) {
         const int q = threadIdx.x;
         A.part[((int64_t)m * gridDim.x + b) * kVirialTerms + q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
+        if (A.part_on_host) __threadfence_system();
     }
 }
 
