@@ -42,21 +42,27 @@ struct pimc_chain {
     // scratch
     std::vector<int32_t> sp;
     std::vector<double> np, op;
-    // device-resident runs: MTRand state, winding table, per-move outputs
-    uint32_t* d_mt = nullptr;
-    int* d_wind = nullptr;
-    int* d_kinds = nullptr;
-    int* d_acc = nullptr;
-    double* d_info = nullptr;
-    int* d_near = nullptr;
-    int cap_moves = 0;
+    // device-resident runs led by this chain: one block with every chain's
+    // arguments and stream state on its way in, one with the results on their way
+    // out (pinned on the host; grown to the largest run)
+    char* h_in = nullptr;
+    char* d_in = nullptr;
+    size_t cap_in = 0;
+    char* h_out = nullptr;
+    char* d_out = nullptr;
+    size_t cap_out = 0;
+    double* h_beads = nullptr;   // mapped: the moved worldlines
+    double* d_beads = nullptr;   // its device address
+    size_t cap_beads = 0;
     ~pimc_chain() {
-        for (void* p : {(void*)d_mt, (void*)d_wind, (void*)d_kinds, (void*)d_acc, (void*)d_info, (void*)d_near})
+        for (void* p : {(void*)d_in, (void*)d_out})
             if (p) (void)hipFree(p);
+        for (void* p : {(void*)h_in, (void*)h_out, (void*)h_beads})
+            if (p) (void)hipHostFree(p);
     }
     int check_device(int n_moves, const int* kinds);
-    int device_args(int n_moves, const int* kinds, pimc::ChainRunArgs* A, pimc::AzizDev* az);
-    int device_results(int n_moves, int* accepted, double* info, int* near);
+    int device_args(int n_moves, pimc::ChainRunArgs* A, pimc::AzizDev* az);
+    hipError_t room(size_t in, size_t out, size_t beads);
 
     double* P(int m, int i) { return pos.data() + 3 * ((size_t)m * N + i); }
     int fail(int code, const std::string& m) {
@@ -337,34 +343,8 @@ int pimc_chain::check_device(int n_moves, const int* kinds) {
     return PIMC_OK;
 }
 
-int pimc_chain::device_args(int n_moves, const int* kinds, pimc::ChainRunArgs* A, pimc::AzizDev* az) {
-    auto chk = [&](hipError_t e, const char* what) {
-        return e == hipSuccess ? PIMC_OK : fail(PIMC_E_HIP, std::string(what) + ": " + hipGetErrorString(e));
-    };
+int pimc_chain::device_args(int n_moves, pimc::ChainRunArgs* A, pimc::AzizDev* az) {
     int r;
-    if (!d_mt) {
-        if ((r = chk(hipMalloc(&d_mt, sizeof(uint32_t) * (MtRand::N + 2)), "hipMalloc"))) return r;
-        if ((r = chk(hipMalloc(&d_wind, sizeof(int) * wind.size()), "hipMalloc"))) return r;
-        if ((r = chk(hipMalloc(&d_near, sizeof(int)), "hipMalloc"))) return r;
-        if ((r = chk(hipMemcpy(d_wind, wind.data(), sizeof(int) * wind.size(), hipMemcpyHostToDevice), "upload")))
-            return r;
-    }
-    if (cap_moves < n_moves) {
-        for (void* p : {(void*)d_kinds, (void*)d_acc, (void*)d_info})
-            if (p) (void)hipFree(p);
-        d_kinds = d_acc = nullptr;
-        d_info = nullptr;
-        if ((r = chk(hipMalloc(&d_kinds, sizeof(int) * n_moves), "hipMalloc"))) return r;
-        if ((r = chk(hipMalloc(&d_acc, sizeof(int) * n_moves), "hipMalloc"))) return r;
-        if ((r = chk(hipMalloc(&d_info, sizeof(double) * 3 * n_moves), "hipMalloc"))) return r;
-        cap_moves = n_moves;
-    }
-    uint32_t mt[MtRand::N + 2];
-    std::memcpy(mt, rng.s, sizeof(uint32_t) * MtRand::N);
-    mt[MtRand::N] = (uint32_t)rng.left;
-    mt[MtRand::N + 1] = (uint32_t)rng.next;
-    if ((r = chk(hipMemcpy(d_mt, mt, sizeof(mt), hipMemcpyHostToDevice), "upload"))) return r;
-    if ((r = chk(hipMemcpy(d_kinds, kinds, sizeof(int) * n_moves, hipMemcpyHostToDevice), "upload"))) return r;
     *az = pimc::context_aziz(ctx, &r);
     if (r) return fail(r, pimc_last_error(ctx));
     *A = pimc::ChainRunArgs{};
@@ -391,38 +371,42 @@ int pimc_chain::device_args(int n_moves, const int* kinds, pimc::ChainRunArgs* A
     A->levels = d.levels;
     A->var_updates = d.var_updates;
     A->num_wind = (int)cumrho0.size();
-    A->wind = d_wind;
-    A->mt = d_mt;
-    A->kinds = d_kinds;
     A->n_moves = n_moves;
-    A->accepted = d_acc;
-    A->info = d_info;
-    A->near = d_near;
     return PIMC_OK;
 }
 
-int pimc_chain::device_results(int n_moves, int* accepted, double* info, int* near) {
-    auto chk = [&](hipError_t e, const char* what) {
-        return e == hipSuccess ? PIMC_OK : fail(PIMC_E_HIP, std::string(what) + ": " + hipGetErrorString(e));
+// Room for a run's blocks (each grown, never shrunk, while the chain lives).
+hipError_t pimc_chain::room(size_t in, size_t out, size_t beads) {
+    auto grow = [](char** h, char** dv, size_t* cap, size_t need) -> hipError_t {
+        if (need <= *cap) return hipSuccess;
+        if (*h) (void)hipHostFree(*h);
+        if (*dv) (void)hipFree(*dv);
+        *h = *dv = nullptr;
+        *cap = 0;
+        hipError_t e = hipHostMalloc((void**)h, need, hipHostMallocDefault);
+        if (e == hipSuccess) e = hipMalloc((void**)dv, need);
+        if (e == hipSuccess) *cap = need;
+        return e;
     };
-    int r;
-    uint32_t mt[MtRand::N + 2];
-    if ((r = chk(hipMemcpy(mt, d_mt, sizeof(mt), hipMemcpyDeviceToHost), "download"))) return r;
-    if (accepted && (r = chk(hipMemcpy(accepted, d_acc, sizeof(int) * n_moves, hipMemcpyDeviceToHost), "download")))
-        return r;
-    if (info && (r = chk(hipMemcpy(info, d_info, sizeof(double) * 3 * n_moves, hipMemcpyDeviceToHost), "download")))
-        return r;
-    int nr = 0;
-    if ((r = chk(hipMemcpy(&nr, d_near, sizeof(int), hipMemcpyDeviceToHost), "download"))) return r;
-    std::memcpy(rng.s, mt, sizeof(uint32_t) * MtRand::N);
-    rng.left = (int)mt[MtRand::N];
-    rng.next = (int)mt[MtRand::N + 1];
-    if (near) *near = nr;
-    // the host copy follows the device path
-    r = pimc_download_path(ctx, pos.data());
-    if (r) return fail(r, pimc_last_error(ctx));
-    return PIMC_OK;
+    hipError_t e = grow(&h_in, &d_in, &cap_in, in);
+    if (e == hipSuccess) e = grow(&h_out, &d_out, &cap_out, out);
+    if (e == hipSuccess && beads > cap_beads) {
+        if (h_beads) (void)hipHostFree(h_beads);
+        h_beads = nullptr;
+        cap_beads = 0;
+        e = hipHostMalloc((void**)&h_beads, beads, hipHostMallocMapped | hipHostMallocCoherent);
+        if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&d_beads, h_beads, 0);
+        if (e == hipSuccess) cap_beads = beads;
+    }
+    return e;
 }
+
+namespace {
+size_t align16(size_t b) { return (b + 15) & ~size_t(15); }
+// Moved worldlines up to this size leave the device compactly; a larger run
+// downloads every chain's path.
+constexpr size_t kMovedBytesMax = size_t(64) << 20;
+}  // namespace
 
 static int run_chains_on_device(pimc_chain* const* chains, int n, int n_moves, const int* kinds, int* accepted,
                                 double* info, int* near) {
@@ -447,35 +431,111 @@ static int run_chains_on_device(pimc_chain* const* chains, int n, int n_moves, c
     for (int c = 0; c < n; ++c)
         if (hipStreamSynchronize(chains[c]->ctx->stream) != hipSuccess)
             return chains[c]->fail(PIMC_E_HIP, "stream synchronisation failed");
-    std::vector<pimc::ChainRunArgs> args(n);
-    std::vector<pimc::AzizDev> azs(n);
-    for (int c = 0; c < n; ++c) {
-        int r = chains[c]->device_args(n_moves, kinds, &args[c], &azs[c]);
-        if (r) return r;
-    }
     pimc_chain* lead = chains[0];
-    pimc::ChainRunArgs* d_args = nullptr;
-    pimc::AzizDev* d_azs = nullptr;
+    // In: arguments | Aziz constants | MTRand states | move kinds | winding tables
+    // (one per max_wind).  Out: MTRand states | info | accepted | near | moved-bead
+    // flags.  One copy each way whatever the number of chains (128 chains of N = 64 x
+    // 96, 12 moves: 15.4 -> 2.7 ms against eight copies per chain; the kernel takes
+    // 0.27 ms, the callers' copies of the positions most of the rest).
+    const size_t mt_words = MtRand::N + 2;
+    const size_t o_az = align16(sizeof(pimc::ChainRunArgs) * n);
+    const size_t o_mt = align16(o_az + sizeof(pimc::AzizDev) * n);
+    const size_t o_kinds = align16(o_mt + sizeof(uint32_t) * mt_words * n);
+    const size_t o_wind = align16(o_kinds + sizeof(int) * n_moves);
+    std::vector<int> wind_of(n);
+    size_t n_wind = 0;
+    for (int c = 0; c < n; ++c) {
+        wind_of[c] = (int)n_wind;
+        int e = 0;
+        while (e < c && chains[e]->d.max_wind != chains[c]->d.max_wind) ++e;
+        if (e < c)
+            wind_of[c] = wind_of[e];
+        else
+            n_wind += chains[c]->wind.size();
+    }
+    const size_t in_bytes = align16(o_wind + sizeof(int) * n_wind);
+    size_t flags = 0, moved = 0;
+    std::vector<size_t> flag_of(n), moved_of(n);
+    for (int c = 0; c < n; ++c) {
+        flag_of[c] = flags;
+        moved_of[c] = moved;
+        flags += chains[c]->N;
+        moved += 3 * (size_t)std::min(n_moves, chains[c]->N) * chains[c]->M;   // a move touches one worldline
+    }
+    const bool compact = sizeof(double) * moved <= kMovedBytesMax;
+    const size_t q_info = align16(sizeof(uint32_t) * mt_words * n);
+    const size_t q_acc = align16(q_info + sizeof(double) * 3 * (size_t)n * n_moves);
+    const size_t q_near = align16(q_acc + sizeof(int) * (size_t)n * n_moves);
+    const size_t q_flags = align16(q_near + sizeof(int) * n);
+    const size_t out_bytes = align16(q_flags + flags);
+    hipError_t e = lead->room(in_bytes, out_bytes, compact ? sizeof(double) * moved : 0);
+    if (e != hipSuccess) return lead->fail(PIMC_E_NOMEM, std::string("chain run: ") + hipGetErrorString(e));
+    auto* args = reinterpret_cast<pimc::ChainRunArgs*>(lead->h_in);
+    auto* azs = reinterpret_cast<pimc::AzizDev*>(lead->h_in + o_az);
+    for (int c = 0; c < n; ++c) {
+        pimc::ChainRunArgs A;
+        int r = chains[c]->device_args(n_moves, &A, &azs[c]);
+        if (r) return r;
+        uint32_t* mt = reinterpret_cast<uint32_t*>(lead->h_in + o_mt) + mt_words * c;
+        std::memcpy(mt, chains[c]->rng.s, sizeof(uint32_t) * MtRand::N);
+        mt[MtRand::N] = (uint32_t)chains[c]->rng.left;
+        mt[MtRand::N + 1] = (uint32_t)chains[c]->rng.next;
+        std::memcpy(lead->h_in + o_wind + sizeof(int) * (size_t)wind_of[c], chains[c]->wind.data(),
+                    sizeof(int) * chains[c]->wind.size());
+        A.mt = reinterpret_cast<const uint32_t*>(lead->d_in + o_mt) + mt_words * c;
+        A.kinds = reinterpret_cast<const int*>(lead->d_in + o_kinds);
+        A.wind = reinterpret_cast<const int*>(lead->d_in + o_wind) + wind_of[c];
+        A.mt_out = reinterpret_cast<uint32_t*>(lead->d_out) + mt_words * c;
+        A.info = reinterpret_cast<double*>(lead->d_out + q_info) + 3 * (size_t)n_moves * c;
+        A.accepted = reinterpret_cast<int*>(lead->d_out + q_acc) + (size_t)n_moves * c;
+        A.near = reinterpret_cast<int*>(lead->d_out + q_near) + c;
+        A.moved = reinterpret_cast<unsigned char*>(lead->d_out + q_flags) + flag_of[c];
+        A.moved_beads = compact ? lead->d_beads + moved_of[c] : nullptr;
+        args[c] = A;
+    }
+    std::memcpy(lead->h_in + o_kinds, kinds, sizeof(int) * n_moves);
+    const auto* d_args = reinterpret_cast<const pimc::ChainRunArgs*>(lead->d_in);
+    const auto* d_azs = reinterpret_cast<const pimc::AzizDev*>(lead->d_in + o_az);
     hipStream_t st = lead->ctx->stream;
-    hipError_t e = hipMalloc(&d_args, sizeof(pimc::ChainRunArgs) * n);
-    if (e == hipSuccess) e = hipMalloc(&d_azs, sizeof(pimc::AzizDev) * n);
-    if (e == hipSuccess) e = hipMemcpy(d_args, args.data(), sizeof(pimc::ChainRunArgs) * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_azs, azs.data(), sizeof(pimc::AzizDev) * n, hipMemcpyHostToDevice);
+    e = hipMemcpyAsync(lead->d_in, lead->h_in, in_bytes, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) {
         lead->ctx->timed_begin(8);
         e = pimc::launch_chain_run(lead->ctx->desc.v_mode, lead->ctx->correction(), st, n, d_args, d_azs);
         lead->ctx->timed_end();
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (d_args) (void)hipFree(d_args);
-    if (d_azs) (void)hipFree(d_azs);
+    if (e == hipSuccess && compact) e = pimc::launch_chain_moved(st, n, d_args);
+    if (e == hipSuccess) e = hipMemcpyAsync(lead->h_out, lead->d_out, out_bytes, hipMemcpyDeviceToHost, st);
+    const hipError_t e1 = hipStreamSynchronize(st);   // quiet after an error too: the blocks are reused
+    if (e == hipSuccess) e = e1;
     if (e != hipSuccess) return lead->fail(PIMC_E_HIP, std::string("chain kernel: ") + hipGetErrorString(e));
     for (int c = 0; c < n; ++c) ++chains[c]->ctx->path_version;   // the launch moved their beads
     for (int c = 0; c < n; ++c) {
-        int r = chains[c]->device_results(n_moves, accepted ? accepted + (size_t)c * n_moves : nullptr,
-                                          info ? info + (size_t)c * 3 * n_moves : nullptr, near ? near + c : nullptr);
-        if (r) return r;
+        pimc_chain& ch = *chains[c];
+        const uint32_t* mt = reinterpret_cast<const uint32_t*>(lead->h_out) + mt_words * c;
+        std::memcpy(ch.rng.s, mt, sizeof(uint32_t) * MtRand::N);
+        ch.rng.left = (int)mt[MtRand::N];
+        ch.rng.next = (int)mt[MtRand::N + 1];
+        if (near) near[c] = reinterpret_cast<const int*>(lead->h_out + q_near)[c];
+        // the host copy follows the device path: the moved worldlines, in bead order
+        if (compact) {
+            const char* flag = lead->h_out + q_flags + flag_of[c];
+            const double* src = lead->h_beads + moved_of[c];
+            for (int i = 0; i < ch.N; ++i) {
+                if (!flag[i]) continue;
+                double* dst = ch.P(0, i);
+                for (int m = 0; m < ch.M; ++m, src += 3, dst += 3 * (size_t)ch.N) {
+                    dst[0] = src[0];
+                    dst[1] = src[1];
+                    dst[2] = src[2];
+                }
+            }
+        } else {
+            const int r = pimc_download_path(ch.ctx, ch.pos.data());
+            if (r) return ch.fail(r, pimc_last_error(ch.ctx));
+        }
     }
+    if (accepted) std::memcpy(accepted, lead->h_out + q_acc, sizeof(int) * (size_t)n * n_moves);
+    if (info) std::memcpy(info, lead->h_out + q_info, sizeof(double) * 3 * (size_t)n * n_moves);
     return PIMC_OK;
 }
 

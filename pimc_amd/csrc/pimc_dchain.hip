@@ -353,6 +353,7 @@ __device__ void correction_pass(const ChainRunArgs& A, const AzizDev& az, ChainL
 // Write list entries [k0, nb) to the path, with the cell-list update of
 // Path::updateBead; the beads sit on distinct slices, one lane each.
 __device__ void commit_list(const ChainRunArgs& A, ChainLds& L, int k0) {
+    if (threadIdx.x == 0) A.moved[L.ptcl] = 1;
     for (int k = k0 + (int)threadIdx.x; k < L.nb; k += (int)blockDim.x) {
         const int m = L.slice[k], i = L.ptcl;
         const double* r = L.newp[L.at[k]];
@@ -674,6 +675,7 @@ __global__ __launch_bounds__(COR ? kChainThreadsCor : kChainThreads) void k_chai
     const ChainRunArgs A = args[blockIdx.x];
     const AzizDev az = azs[blockIdx.x];
     for (int t = threadIdx.x; t < kMt; t += (int)blockDim.x) L.mt.s[0][t] = A.mt[t];
+    for (int t = threadIdx.x; t < A.nalloc; t += (int)blockDim.x) A.moved[t] = 0;
     if (threadIdx.x == 0) {
         L.mt.cur = 0;
         L.mt.next = (int)A.mt[kMt + 1];
@@ -698,15 +700,54 @@ __global__ __launch_bounds__(COR ? kChainThreadsCor : kChainThreads) void k_chai
             com<MODE, COR>(A, az, L, acc, info);
         __syncthreads();
     }
-    for (int t = threadIdx.x; t < kMt; t += (int)blockDim.x) A.mt[t] = L.mt.s[L.mt.cur][t];
+    for (int t = threadIdx.x; t < kMt; t += (int)blockDim.x) A.mt_out[t] = L.mt.s[L.mt.cur][t];
     if (threadIdx.x == 0) {
-        A.mt[kMt] = (uint32_t)(kMt - L.mt.next);
-        A.mt[kMt + 1] = (uint32_t)L.mt.next;
+        A.mt_out[kMt] = (uint32_t)(kMt - L.mt.next);
+        A.mt_out[kMt + 1] = (uint32_t)L.mt.next;
         A.near[0] = L.near;
     }
 }
 
+// One workgroup per chain: the run's moved worldlines, in bead order, straight into
+// mapped host memory (a run of 12 moves touches at most 12 of a chain's worldlines,
+// so this is a fraction of the path; the writes run at the link's rate).
+__global__ __launch_bounds__(256) void k_chain_moved(const ChainRunArgs* __restrict__ args) {
+    __shared__ int list[256];
+    __shared__ int cnt;
+    const ChainRunArgs A = args[blockIdx.x];
+    int done = 0;   // worldlines written so far
+    for (int i0 = 0; i0 < A.nalloc; i0 += 256) {
+        const int i = i0 + threadIdx.x;
+        const bool on = i < A.nalloc && A.moved[i];
+        // places in bead order: waves in order, ballots within a wave
+        __shared__ int wave_n[4];
+        const unsigned long long b = __ballot(on);
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        if (lane == 0) wave_n[wave] = __popcll(b);
+        __syncthreads();
+        int at = __popcll(b & ((1ull << lane) - 1ull));
+        for (int w = 0; w < wave; ++w) at += wave_n[w];
+        if (on) list[at] = i;
+        if (threadIdx.x == 0) cnt = wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
+        __syncthreads();
+        const int per = 3 * A.num_slices;
+        double* out = A.moved_beads + (int64_t)done * per;
+        for (int t = threadIdx.x; t < cnt * per; t += 256) {
+            const int k = t / per, r = t - k * per, m = r / 3, d = r - 3 * m;
+            out[t] = A.pos[(int64_t)m * A.nalloc + list[k] + d * A.plane];
+        }
+        done += cnt;
+        __syncthreads();
+    }
+}
+
 }  // namespace
+
+hipError_t launch_chain_moved(hipStream_t st, int n_chains, const ChainRunArgs* args) {
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_chain_moved, dim3(n_chains), dim3(256), 0, st, args);
+    return hipGetLastError();
+}
 
 hipError_t launch_chain_run(int mode, bool cor, hipStream_t st, int n_chains, const ChainRunArgs* args,
                             const AzizDev* azs) {

@@ -277,16 +277,21 @@ struct ChainRunArgs {
     double sqrtLambdaTau, sqrt2LambdaTau, com_delta;
     int Mbar, levels, var_updates, num_wind;
     const int* wind;     // [num_wind][3]
-    uint32_t* mt;        // MTRand state [624], left, next (read and written back)
+    const uint32_t* mt;  // MTRand state [624], left, next
+    uint32_t* mt_out;    // the state after the run
     const int* kinds;    // [n_moves]: 0 staging, 1 bisection, 2 centre of mass
     int n_moves;
     int* accepted;       // [n_moves]
     double* info;        // [n_moves][3]: attempted, last Delta, length
     int* near;           // decisions inside the guard band
+    unsigned char* moved;   // [nalloc]: 1 where the run wrote to the worldline's beads
+    double* moved_beads;    // mapped host memory: those worldlines [k][num_slices][3], or null
 };
 // args / azs: device arrays, one entry per chain (workgroup).
 hipError_t launch_chain_run(int mode, bool cor, hipStream_t st, int n_chains, const ChainRunArgs* args,
                             const AzizDev* azs);
+// The moved worldlines of each chain into moved_beads, in bead order.
+hipError_t launch_chain_moved(hipStream_t st, int n_chains, const ChainRunArgs* args);
 hipError_t launch_virial(int mode, hipStream_t st, const VirialArgs& A, const AzizDev& az, int* blocks_per_slice);
 hipError_t launch_update_beads(hipStream_t st, const int* sp, const double* p3, int n, double* pos, int64_t plane,
                                int nalloc, int num_slices, int* cell, int* label, int* numlab, int* hash,
