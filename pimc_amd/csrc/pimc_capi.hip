@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -367,16 +368,27 @@ bool pimc_ctx::direct_ready(int mode) {
     if (direct_state < 0) {
         direct_state = 0;
         if (pimc::direct_ring_create(device, &dring)) {
+            // the kernels' entries in the loaded code object: looked up once per device
+            static std::mutex mu;
+            static std::map<int, std::array<pimc::DirectKernel, 6>> found;
+            std::lock_guard<std::mutex> lk(mu);
             bool all = true;
-            for (int m = 0; m < 3 && all; ++m)
-                all = pimc::direct_kernel(device, pimc::vnn_direct_stub(m), stream, pimc::kVdirBytes, &dk_vdir[m]);
+            if (found.count(device)) {
+                for (int k = 0; k < 6; ++k) dk_vdir[k] = found[device][k];
+            } else {
+                for (int k = 0; k < 6 && all; ++k)
+                    all = pimc::direct_kernel(device, pimc::vnn_direct_stub(k / 2, k % 2 != 0), stream,
+                                              pimc::kVdirBytes, &dk_vdir[k]);
+                if (all)
+                    for (int k = 0; k < 6; ++k) found[device][k] = dk_vdir[k];
+            }
             if (all)
                 direct_state = 1;
             else
                 pimc::direct_ring_release(&dring);
         }
     }
-    return direct_state == 1 && mode >= 0 && mode < 3 && dk_vdir[mode].ok();
+    return direct_state == 1 && mode >= 0 && mode < 3 && dk_vdir[2 * mode].ok();
 }
 
 bool pimc_ctx::stream_quiet() {
@@ -676,11 +688,11 @@ int pimc_ctx_create(const pimc_desc* d, pimc_ctx** out) {
         std::memset(c->h_map, 0, sizeof(double) * 64);
         e = hipHostGetDevicePointer((void**)&c->d_map, c->h_map, 0);
         if (e != hipSuccess) return fail(nullptr, PIMC_E_HIP, std::string("hipHostGetDevicePointer: ") + hipGetErrorString(e));
-        e = hipHostMalloc((void**)&c->h_vdir, sizeof(VnnDirectOut) * kVnnInline,
+        e = hipHostMalloc((void**)&c->h_vdir, sizeof(VnnDirectOut) * kVnnDirectMax,
                           hipHostMallocMapped | hipHostMallocCoherent);
         if (e != hipSuccess) return fail(nullptr, PIMC_E_NOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
         c->host_allocs.push_back((void*)c->h_vdir);
-        std::memset(c->h_vdir, 0, sizeof(VnnDirectOut) * kVnnInline);
+        std::memset(c->h_vdir, 0, sizeof(VnnDirectOut) * kVnnDirectMax);
         e = hipHostGetDevicePointer((void**)&c->d_vdir, c->h_vdir, 0);
         if (e != hipSuccess) return fail(nullptr, PIMC_E_HIP, std::string("hipHostGetDevicePointer: ") + hipGetErrorString(e));
     }
@@ -1412,23 +1424,29 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
     A.done = c->d_done();
     A.seq = ++c->seq;
     VnnInline req;
-    // short requests without the correction or per-bead outputs: one workgroup
-    // per bead publishes its two sums; the weighted bead terms are added here in
-    // bead order
-    if (inline_req && A.chunks == 1 && !cor && !per_bead && !cor_out && out3) {
-        std::memcpy(req.beads, c->h_req_beads, sizeof(VnnBead) * n);
+    // requests without the correction or per-bead outputs: one workgroup per bead
+    // publishes its two sums; the weighted bead terms are added here in bead order
+    if (n <= kVnnDirectMax && A.chunks == 1 && !cor && !per_bead && !cor_out && out3) {
+        if (inline_req)
+            std::memcpy(req.beads, c->h_req_beads, sizeof(VnnBead) * n);
+        else
+            A.beads = c->h_req_beads;   // pinned: read in place
         const KernelTimer kt = c->kernel_timer(1);
         // a packet on the device's AQL queue when the call is not timed (the
         // timing events live on the stream) and the context's stream is quiet:
         // the two never run work of one context at once
-        const bool packet = !kt.start && c->direct_ready(c->desc.v_mode) && c->stream_quiet();
+        // Setting up the queue's argument ring takes about 12 us, two requests'
+        // gain: a context's first long request goes through HIP.
+        const bool first_long = !inline_req && c->direct_state < 0 && !c->asked_long;
+        c->asked_long |= !inline_req;
+        const bool packet = !kt.start && !first_long && c->direct_ready(c->desc.v_mode) && c->stream_quiet();
         if (packet) {
             VnnDirectOut* outp = c->d_vdir;
             const pimc::ArgPiece pieces[4] = {{&A, 0, (uint32_t)sizeof(VnnArgs)},
-                                              {req.beads, pimc::kVdirOffReq, (uint32_t)(sizeof(VnnBead) * n)},
+                                              {req.beads, pimc::kVdirOffReq, inline_req ? (uint32_t)(sizeof(VnnBead) * n) : 0u},
                                               {&az, pimc::kVdirOffAz, (uint32_t)sizeof(AzizDev)},
                                               {&outp, pimc::kVdirOffOut, (uint32_t)sizeof(outp)}};
-            pimc::direct_dispatch(&c->dring, c->dk_vdir[c->desc.v_mode], pieces, 4, (uint32_t)n,
+            pimc::direct_dispatch(&c->dring, c->dk_vdir[2 * c->desc.v_mode + (inline_req ? 0 : 1)], pieces, 4, (uint32_t)n,
                                   (uint32_t)kVnnDirectThreads);
             ++c->direct_count;
         } else {
@@ -1438,7 +1456,7 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         const double tau_s = shift * c->desc.tau;
         double ao = 0.0, an = 0.0, du = 0.0;
         for (int k = 0; k < n; ++k) {
-            const double co = ((req.beads[k].slice & 1) ? A.vfactor1 : A.vfactor0) * tau_s;
+            const double co = ((c->h_req_beads[k].slice & 1) ? A.vfactor1 : A.vfactor0) * tau_s;
             const double vo = c->h_vdir[k].v_old, vn = c->h_vdir[k].v_new;
             ao += co * vo;
             an += co * vn;

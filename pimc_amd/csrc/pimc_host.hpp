@@ -117,8 +117,9 @@ struct pimc_ctx {
     // kernel-argument ring and k_vnn_direct per mode; direct_state -1: not set
     // up yet, 0: launched through HIP, 1: packets)
     pimc::DirectRing dring;
-    pimc::DirectKernel dk_vdir[3];
+    pimc::DirectKernel dk_vdir[6];   // [2 mode + listed]
     int direct_state = -1;
+    bool asked_long = false;   // a request of more than kVnnInline beads has been made
     long direct_count = 0;   // requests dispatched as packets
     bool direct_ready(int mode);
     // Every entry point returns only after its work on the stream has finished

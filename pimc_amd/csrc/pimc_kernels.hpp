@@ -144,6 +144,11 @@ constexpr int kGnnGroup = 16;   // bead2 per three-body workgroup (16 lanes each
 
 // Requests of up to kVnnInline beads travel in the kernel arguments.
 constexpr int kVnnInline = 32;
+// The direct form takes requests of up to this many beads (a whole worldline of the
+// workloads).  Its host side adds the bead terms, one cache line per two beads; a
+// centre-of-mass move of N = 181 x 143 takes 15 us from Python (21 us as one kernel
+// with a hand-off, launched through HIP after a copy of the list).
+constexpr int kVnnDirectMax = 512;
 struct VnnInline {
     VnnBead beads[kVnnInline];
 };
@@ -241,13 +246,14 @@ int pair_grid_for(int lds_beads, int num_cus);
 hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInline& req, const AzizDev& az,
                       const KernelTimer* timer = nullptr, double* gnn_part = nullptr, int lds_beads = 0,
                       const KernelTimer* gnn_timer = nullptr);
-// The direct form (k_vnn_direct): at most kVnnInline beads travelling inline, at
-// most kVnnChunk beads per slice; out [n_beads] is host-mapped.
+// The direct form (k_vnn_direct): at most kVnnDirectMax beads, up to kVnnInline of
+// them travelling inline, more at A.beads (mapped host memory: each workgroup reads
+// its own 64 bytes), at most kVnnChunk beads per slice; out [n_beads] is host-mapped.
 hipError_t launch_vnn_direct(int mode, hipStream_t st, const VnnArgs& A, const VnnInline& req, const AzizDev& az,
                              VnnDirectOut* out, const KernelTimer* timer = nullptr);
 // k_vnn_direct<mode>'s host stub, and its argument block as the AMDGPU ABI lays
 // it out (each by-value argument at its alignment), for a dispatch packet
-const void* vnn_direct_stub(int mode);
+const void* vnn_direct_stub(int mode, bool listed);
 constexpr uint32_t karg_align(uint32_t o, uint32_t a) { return (o + a - 1) / a * a; }
 constexpr uint32_t kVdirOffReq = karg_align(sizeof(VnnArgs), alignof(VnnInline));
 constexpr uint32_t kVdirOffAz = karg_align(kVdirOffReq + sizeof(VnnInline), alignof(AzizDev));

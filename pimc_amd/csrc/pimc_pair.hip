@@ -1330,7 +1330,7 @@ __device__ __forceinline__ void vnn_finalize_body(const VnnArgs& A, const VnnInl
 
 __global__ __launch_bounds__(256) void k_vnn_finalize(VnnArgs A, VnnInline req) { vnn_finalize_body(A, req); }
 
-// Delta V of a short request with no hand-off between workgroups: workgroup b
+// Delta V of a request with no hand-off between workgroups: workgroup b
 // sums bead b's Vnn over all its partners (the slice holds at most kVnnChunk
 // beads) at the old position on its first 256 lanes and at the new position on
 // the other 256, so each lane's chain is one pair term per partner; it commits
@@ -1339,13 +1339,15 @@ __global__ __launch_bounds__(256) void k_vnn_finalize(VnnArgs A, VnnInline req) 
 // number straight into the caller's mapped block, slot b.  The caller adds the
 // beads' weighted terms in bead order once every slot carries the sequence
 // number.  A lane's partners, and so its sum, are those of the two-position
-// kernels' lanes, and the waves are added in the same order.
-template <int MODE>
+// kernels' lanes, and the waves are added in the same order.  LISTED: the beads
+// come from A.beads; a variant of its own, since a pointer test before the load
+// costs a short request about 0.3 us (one more dependent argument load).
+template <int MODE, bool LISTED>
 __global__ __launch_bounds__(kVnnDirectThreads) void k_vnn_direct(VnnArgs A, VnnInline req, AzizDev az,
                                                                   VnnDirectOut* out) {
     __shared__ double red[kVnnDirectThreads / 64];
     const int b = blockIdx.x;
-    const VnnBead q = req.beads[b];
+    const VnnBead q = LISTED ? A.beads[b] : req.beads[b];
     const VnnSubject v = vnn_subject(A, q);
     const double inv_dr = 1.0 / az.dr;
     const bool at_new = threadIdx.x >= kVnnThreads;
@@ -1735,23 +1737,28 @@ hipError_t launch_vnn_direct(int mode, hipStream_t st, const VnnArgs& A, const V
                              VnnDirectOut* out, const KernelTimer* timer) {
     (void)hipGetLastError();  // drop any stale error of an earlier call
     if (A.n_beads <= 0) return hipSuccess;
-    if (A.n_beads > kVnnInline || A.nalloc > kVnnChunk || A.beads) return hipErrorInvalidValue;
+    if (A.n_beads > kVnnDirectMax || A.nalloc > kVnnChunk || (A.n_beads > kVnnInline && !A.beads))
+        return hipErrorInvalidValue;
     dim3 g(A.n_beads), b(kVnnDirectThreads);
     if (timer && timer->start) (void)hipEventRecord(timer->start, st);
-    if (mode == 0)
-        hipLaunchKernelGGL(k_vnn_direct<0>, g, b, 0, st, A, req, az, out);
-    else if (mode == 1)
-        hipLaunchKernelGGL(k_vnn_direct<1>, g, b, 0, st, A, req, az, out);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, b, 0, st, A, req, az, out); };
+    if (A.beads)
+        mode == 0 ? go(k_vnn_direct<0, true>) : mode == 1 ? go(k_vnn_direct<1, true>) : go(k_vnn_direct<2, true>);
     else
-        hipLaunchKernelGGL(k_vnn_direct<2>, g, b, 0, st, A, req, az, out);
+        mode == 0 ? go(k_vnn_direct<0, false>) : mode == 1 ? go(k_vnn_direct<1, false>) : go(k_vnn_direct<2, false>);
     if (timer && timer->stop) (void)hipEventRecord(timer->stop, st);
     return hipGetLastError();
 }
 
-const void* vnn_direct_stub(int mode) {
-    if (mode == 0) return reinterpret_cast<const void*>(&k_vnn_direct<0>);
-    if (mode == 1) return reinterpret_cast<const void*>(&k_vnn_direct<1>);
-    return reinterpret_cast<const void*>(&k_vnn_direct<2>);
+template <bool LISTED>
+static const void* vnn_direct_stub_of(int mode) {
+    if (mode == 0) return reinterpret_cast<const void*>(&k_vnn_direct<0, LISTED>);
+    if (mode == 1) return reinterpret_cast<const void*>(&k_vnn_direct<1, LISTED>);
+    return reinterpret_cast<const void*>(&k_vnn_direct<2, LISTED>);
+}
+
+const void* vnn_direct_stub(int mode, bool listed) {
+    return listed ? vnn_direct_stub_of<true>(mode) : vnn_direct_stub_of<false>(mode);
 }
 
 hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInline& req, const AzizDev& az,
