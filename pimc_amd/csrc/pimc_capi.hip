@@ -1053,9 +1053,9 @@ static int launch_virial_terms(pimc_ctx* c, const int32_t* next_links, int windo
     V->mapped = mapped ? c->h_map + pimc_ctx::kSqSlot + 2 * M : nullptr;
     A.part = mapped ? c->d_map + pimc_ctx::kSqSlot + 2 * M : c->d_virial;
     A.part_on_host = mapped;
-    A.chunks = gradv2_chunks(N, M, c->num_cus);
+    virial_chunks(&A, c->num_cus);
     A.fpart = nullptr;
-    if (A.chunks > 1) {
+    if (A.tiles || A.chunks > 1) {
         const size_t fneed = (size_t)M * A.chunks * N * 9;
         if (c->cap_vf < fneed) {
             free_dev(c, c->d_vf);

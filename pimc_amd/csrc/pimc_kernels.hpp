@@ -89,9 +89,13 @@ struct VirialArgs {
     BoxDev box;
     double* part;        // [M][blocks][kVirialTerms]
     int part_on_host;    // part is mapped host memory, read after a later kernel's publication
-    int chunks;          // partner chunks (1: one pass per row block)
-    double* fpart;       // chunk partials [M][chunks][nalloc][9] = F, T (chunks > 1)
+    int tiles;           // k_virial_sym: tiles of 64 beads (0: not that form),
+    int waves, wgs;      // waves per workgroup and workgroups
+    int chunks;          // partials per slice (sym), or partner chunks (1: one pass per row block)
+    double* fpart;       // partials [M][chunks][nalloc][9] = F, T (sym, or chunks > 1)
 };
+
+constexpr int kVirialSymBeads = 1024;   // 16 tiles of 64
 
 // A Vnn evaluation request for one bead: partners are the active beads of its slice.
 struct VnnBead {
@@ -298,6 +302,7 @@ hipError_t launch_chain_run(int mode, bool cor, hipStream_t st, int n_chains, co
                             const AzizDev* azs);
 // The moved worldlines of each chain into moved_beads, in bead order.
 hipError_t launch_chain_moved(hipStream_t st, int n_chains, const ChainRunArgs* args);
+void virial_chunks(VirialArgs* A, int num_cus);   // sets tiles, wgs, chunks
 hipError_t launch_virial(int mode, hipStream_t st, const VirialArgs& A, const AzizDev& az, int* blocks_per_slice);
 hipError_t launch_update_beads(hipStream_t st, const int* sp, const double* p3, int n, double* pos, int64_t plane,
                                int nalloc, int num_slices, int* cell, int* label, int* numlab, int* hash,
