@@ -323,14 +323,17 @@ void pimc_ctx::resolve_timing() {
 // spin on a host cache line instead of a stream synchronisation (whose wake-up
 // costs several microseconds).  After 0.2 s it falls back to the stream
 // synchronisation, which also returns an error the stream may hold.
-int pimc_ctx::wait_done(unsigned long long s) {
+// packet: as in wait_direct below.
+int pimc_ctx::wait_done(unsigned long long s, bool packet) {
     const unsigned long long* f = reinterpret_cast<const unsigned long long*>(h_map + kDoneSlot);
     const auto t0 = std::chrono::steady_clock::now();
+    const auto limit = std::chrono::milliseconds(packet ? 10000 : 200);
     for (unsigned it = 1;; ++it) {
         if (__atomic_load_n(f, __ATOMIC_ACQUIRE) == s) return 0;
-        if ((it & 4095u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(200)) break;
+        if ((it & 4095u) == 0 && std::chrono::steady_clock::now() - t0 > limit) break;
         __builtin_ia32_pause();
     }
+    if (packet) return -1;
     const hipError_t e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return (int)e;
     return __atomic_load_n(f, __ATOMIC_ACQUIRE) == s ? 0 : -1;
@@ -389,6 +392,19 @@ bool pimc_ctx::direct_ready(int mode) {
         }
     }
     return direct_state == 1 && mode >= 0 && mode < 3 && dk_vdir[2 * mode].ok();
+}
+
+// May the kernels of an action go as packets?  For calls whose
+// kernels take a few tens of microseconds (a packet holds up the device queue's later
+// ones, other contexts' too); untimed.  A context's first such call goes through HIP:
+// setting the ring up costs more than one call gains.
+bool pimc_ctx::packets_ready() {
+    constexpr double kMostPairs = 1.6e7;
+    const double N = desc.num_alloc;
+    if (timing || 0.5 * N * N * desc.num_slices > kMostPairs) return false;
+    const bool first = direct_state < 0 && !asked_packets;
+    asked_packets = true;
+    return !first && direct_ready(desc.v_mode) && stream_quiet();
 }
 
 bool pimc_ctx::stream_quiet() {
@@ -585,7 +601,10 @@ static void fill_walker(pimc_ctx* c, WalkerDesc* w, int shift, const double vf[2
 
 // gradVSquared(slice) into c->d_g2part (partials per slice) of the even (need bit
 // 0) and odd (bit 1) slices; 0 for the others.
-static int run_gradv2(pimc_ctx* c, const AzizDev& az, int need) {
+// packets: the kernels go there where the sum runs in chunks; else *chunked is cleared
+// and nothing is launched.
+static int run_gradv2(pimc_ctx* c, const AzizDev& az, int need, PacketList* packets = nullptr,
+                      bool* chunked = nullptr) {
     const int M = c->desc.num_slices, N = c->desc.num_alloc;
     if (c->desc.v_mode == PIMC_V_TABLE && !az.dtable)
         return fail(c, PIMC_E_STATE, "gradVSquared in the table mode needs the dV/dr table");
@@ -604,10 +623,14 @@ static int run_gradv2(pimc_ctx* c, const AzizDev& az, int need) {
         if ((r = ctx_dalloc(c, &c->d_g2f, (size_t)M * C * N * 3))) return r;
         c->cap_g2f = (size_t)M * C * N * 3;
     }
+    if (packets && C <= 1) {
+        *chunked = false;
+        return PIMC_OK;
+    }
     int blocks = 0;
     c->timed_begin(5);
     HIP_OR_FAIL(c, launch_gradv2(c->desc.v_mode, c->stream, c->d_pos, c->plane, N, M, c->d_nbs, c->box, az,
-                                 c->lds_beads, c->d_g2part, &blocks, C, c->d_g2f, need));
+                                 c->lds_beads, c->d_g2part, &blocks, C, c->d_g2f, need, packets));
     c->timed_end();
     c->g2_blocks = blocks;
     return PIMC_OK;
@@ -896,7 +919,7 @@ int pimc_potential_slices(pimc_ctx* c, double* v_slices, int32_t* sep_hist) {
 // gradVFactor is finite (the context's action carries the correction).  Without
 // with_correction the action leaves the correction out and only V(slice) is asked for.
 static int total_action(pimc_ctx* c, int shift, const double vfactor[2], double* action, double* v_slices, double* g2,
-                        bool with_correction = true) {
+                        bool with_correction = true, bool own_kernels = true) {
     if (!c || !action) return fail(c, PIMC_E_ARG, "null argument");
     if (!c->have_path) return fail(c, PIMC_E_STATE, "no path uploaded");
     if (shift < 1) return fail(c, PIMC_E_ARG, "shift must be >= 1");
@@ -907,14 +930,16 @@ static int total_action(pimc_ctx* c, int shift, const double vfactor[2], double*
     WalkerDesc w;
     std::memset(&w, 0, sizeof(w));
     fill_walker(c, &w, shift, vfactor);
+    bool on_stream = !own_kernels;   // the call has put other work on the stream
     if (!c->walker_valid || std::memcmp(&w, &c->walker_cache, sizeof(w)) != 0) {
         HIP_OR_FAIL(c, hipMemcpyAsync(c->d_walker, &w, sizeof(w), hipMemcpyHostToDevice, c->stream));
         c->walker_cache = w;
         c->walker_valid = true;
+        on_stream = true;
     }
     if (c->n_tiles > 0) {
         const bool cor = with_correction && c->correction();
-        if (cor && (r = run_gradv2(c, az, (c->gvf[0] > kCorrEps ? 1 : 0) | (c->gvf[1] > kCorrEps ? 2 : 0)))) return r;
+        const int need = (c->gvf[0] > kCorrEps ? 1 : 0) | (c->gvf[1] > kCorrEps ? 2 : 0);
         const bool spatial = c->pair_spatial && c->desc.v_mode == PIMC_V_MIXED;
         if (spatial && c->perm_version != c->path_version) {
             HIP_OR_FAIL(c, launch_slice_order(c->stream, c->d_slices, M, c->d_pos, c->box.invL, c->d_perm));
@@ -926,17 +951,34 @@ static int total_action(pimc_ctx* c, int shift, const double vfactor[2], double*
         // spin on the completion word covers both (a copy and a stream
         // synchronisation took ~10 us more)
         const bool mapped = v_slices && 2 * M <= pimc_ctx::kMappedSq;
-        HIP_OR_FAIL(c, launch_pair_action(c->desc.v_mode, c->stream, c->d_tiles, c->n_tiles, c->d_ranges, c->n_groups,
-                                          c->d_slices, M, c->d_walker, 1, c->d_pos, az, c->pair_lds, c->d_partials,
-                                          c->d_vslice, c->d_map, &kt, true, c->d_done(), seq,
-                                          cor ? c->d_g2part : nullptr, c->g2_blocks, c->d_g2slice,
-                                          spatial ? c->d_perm : nullptr,
-                                          mapped ? c->d_map + pimc_ctx::kSqSlot : nullptr));
+        double* v_host = mapped ? c->d_map + pimc_ctx::kSqSlot : nullptr;
+        // As packets: the queue that the moves' Delta V requests use takes the action
+        // too, and nothing waits for the stream's queue to wake (three requests and an
+        // action at N = 256, M = 167: 55.5 -> 54.1 us; an action alone gains 0.2 us).
+        bool packet = !on_stream && !spatial && (mapped || !v_slices) && c->packets_ready();
+        auto launch = [&](PacketList* list) -> int {
+            bool chunked = true;
+            if (cor && (r = run_gradv2(c, az, need, list, &chunked))) return r;
+            packet = packet && chunked;
+            if (list && !packet) return PIMC_OK;
+            HIP_OR_FAIL(c, launch_pair_action(c->desc.v_mode, c->stream, c->d_tiles, c->n_tiles, c->d_ranges,
+                                              c->n_groups, c->d_slices, M, c->d_walker, 1, c->d_pos, az, c->pair_lds,
+                                              c->d_partials, c->d_vslice, c->d_map, list ? nullptr : &kt, true,
+                                              c->d_done(), seq, cor ? c->d_g2part : nullptr, c->g2_blocks,
+                                              c->d_g2slice, spatial ? c->d_perm : nullptr, v_host, list));
+            return PIMC_OK;
+        };
+        if (packet) {
+            PacketList list(&c->dring, c->stream);
+            if ((r = launch(&list))) return r;
+            packet = packet && list.send();
+        }
+        if (!packet && (r = launch(nullptr))) return r;
         if (v_slices && !mapped) {
             HIP_OR_FAIL(c, hipMemcpyAsync(c->h_stage, c->d_vslice, sizeof(double) * M, hipMemcpyDeviceToHost,
                                           c->stream));
             HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-        } else if (c->wait_done(seq) != 0) {
+        } else if (c->wait_done(seq, packet) != 0) {
             return fail(c, PIMC_E_HIP, "pair action: completion not published");
         }
         *action = c->h_map[0];
@@ -1135,7 +1177,7 @@ int pimc_virial_energy(pimc_ctx* c, const int32_t* next_links, int window, doubl
     double act = 0.0;
     int r = launch_virial_terms(c, next_links, window, &V);
     if (r) return r;
-    if ((r = total_action(c, 1, vf1, &act, vs.data(), nullptr, false))) return r;
+    if ((r = total_action(c, 1, vf1, &act, vs.data(), nullptr, false, false))) return r;
     if ((r = collect_virial(c, V, c->n_tiles > 0, S))) return r;
     virial_slice_terms(c, S, terms.data());
     // VirialEnergyEstimator::accumulate (src/estimator.cpp:1086-1251), one call
@@ -1321,7 +1363,7 @@ int pimc_energy(pimc_ctx* c, const int32_t* next_links, double mu, double* out9)
     std::vector<double> g2(M, 0.0);
     const double vf1[2] = {1.0, 1.0};
     double act = 0.0;
-    if ((r = total_action(c, 1, vf1, &act, vs.data(), c->correction() ? g2.data() : nullptr))) return r;
+    if ((r = total_action(c, 1, vf1, &act, vs.data(), c->correction() ? g2.data() : nullptr, true, false))) return r;
     if (c->n_tiles == 0) HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     const double link_sum = c->h_map[kKineticSlot];
     // EnergyEstimator::accumulate (src/estimator.cpp:940-1029) with the context's action factors
@@ -1467,15 +1509,30 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         out3[2] = du;
         return PIMC_OK;
     }
+    const int gnn_lds = c->desc.num_alloc <= kLdsBeads ? c->desc.num_alloc : 0;
     if (inline_req) {
         std::memcpy(req.beads, c->h_req_beads, sizeof(VnnBead) * n);
+        // a short request with the correction: both kernels as packets (N = 256:
+        // 21.6 us, 23.0 through HIP; N = 16: 16.1 and 18.4)
+        if (cor && A.chunks == 1 && !per_bead && !cor_out && out3 && !c->timing && c->direct_ready(c->desc.v_mode) &&
+            c->stream_quiet()) {
+            PacketList list(&c->dring, c->stream);
+            list.long_arg_bytes = (uint32_t)(sizeof(VnnBead) * n);
+            HIP_OR_FAIL(c, launch_vnn(c->desc.v_mode, c->stream, A, req, az, nullptr, c->d_gnn_part, gnn_lds, nullptr,
+                                      &list));
+            if (list.send()) {
+                ++c->direct_count;
+                if (c->wait_done(A.seq, true) != 0) return fail(c, PIMC_E_HIP, "delta action: completion not published");
+                for (int k = 0; k < 3; ++k) out3[k] = c->h_map[8 + k];
+                return PIMC_OK;
+            }
+        }
     } else {
         HIP_OR_FAIL(c, hipMemcpyAsync(c->d_req_beads, c->h_req_beads, sizeof(VnnBead) * n, hipMemcpyHostToDevice,
                                       c->stream));
     }
     const KernelTimer kt = c->kernel_timer(1);
     const KernelTimer kg = cor ? c->kernel_timer(6) : KernelTimer{};
-    const int gnn_lds = c->desc.num_alloc <= kLdsBeads ? c->desc.num_alloc : 0;
     HIP_OR_FAIL(c, launch_vnn(c->desc.v_mode, c->stream, A, req, az, &kt, cor ? c->d_gnn_part : nullptr, gnn_lds,
                               &kg));
     if (per_bead || cor_out) {

@@ -21,6 +21,7 @@
 #include <stdlib.h>
 
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 
@@ -357,7 +358,7 @@ bool direct_kernel(int device, const void* host_stub, hipStream_t stream, uint32
         return false;
     // the argument block must be exactly what the caller writes (no hidden
     // arguments the packet would have to supply) and fit one ring slot
-    if (obj == 0 || karg != bytes || bytes > kDirectSlotBytes || priv != 0) return false;
+    if (obj == 0 || karg < bytes || karg > (bytes + 7) / 8 * 8 || bytes > kDirectSlotBytes || priv != 0) return false;
     k->object = obj;
     k->kernarg_bytes = karg;
     k->group_bytes = group;
@@ -378,17 +379,17 @@ void direct_flush(int device) {
 }
 
 namespace {
-void write_packet(hsa_queue_t* q, const DirectKernel& k, const char* kernargs, uint32_t grid_x, uint32_t block_x) {
+void write_packet(hsa_queue_t* q, const DirectKernel& k, const char* kernargs, dim3 g, dim3 b) {
     const uint64_t idx = hsa_queue_add_write_index_relaxed(q, 1);
     while (idx - hsa_queue_load_read_index_scacquire(q) >= q->size) _mm_pause();
     hsa_kernel_dispatch_packet_t* p = static_cast<hsa_kernel_dispatch_packet_t*>(q->base_address) +
                                       (idx & (q->size - 1));
-    p->workgroup_size_x = (uint16_t)block_x;
+    p->workgroup_size_x = (uint16_t)b.x;
     p->workgroup_size_y = 1;
     p->workgroup_size_z = 1;
     p->reserved0 = 0;
-    p->grid_size_x = grid_x * block_x;
-    p->grid_size_y = 1;
+    p->grid_size_x = g.x * b.x;
+    p->grid_size_y = g.y;
     p->grid_size_z = 1;
     p->private_segment_size = 0;
     p->group_segment_size = k.group_bytes;
@@ -404,7 +405,7 @@ void write_packet(hsa_queue_t* q, const DirectKernel& k, const char* kernargs, u
                             (1 << HSA_PACKET_HEADER_BARRIER) |
                             (HSA_FENCE_SCOPE_AGENT << HSA_PACKET_HEADER_SCACQUIRE_FENCE_SCOPE) |
                             (HSA_FENCE_SCOPE_AGENT << HSA_PACKET_HEADER_SCRELEASE_FENCE_SCOPE);
-    const uint16_t setup = 1 << HSA_KERNEL_DISPATCH_PACKET_SETUP_DIMENSIONS;
+    const uint16_t setup = (g.y > 1 ? 2 : 1) << HSA_KERNEL_DISPATCH_PACKET_SETUP_DIMENSIONS;
     __atomic_store_n(reinterpret_cast<uint32_t*>(p), (uint32_t)header | ((uint32_t)setup << 16), __ATOMIC_RELEASE);
     hsa_signal_store_screlease(q->doorbell_signal, (hsa_signal_value_t)idx);
 }
@@ -412,12 +413,12 @@ void write_packet(hsa_queue_t* q, const DirectKernel& k, const char* kernargs, u
 
 void direct_submit(DirectRing* r, const DirectKernel& k, const char* kernargs, uint32_t grid_x, uint32_t block_x) {
     if (r->own_queue) {
-        write_packet(static_cast<hsa_queue_t*>(r->own_queue), k, kernargs, grid_x, block_x);
+        write_packet(static_cast<hsa_queue_t*>(r->own_queue), k, kernargs, dim3(grid_x), dim3(block_x));
         return;
     }
     DeviceQueue& D = g_dev[r->device];
     std::lock_guard<std::mutex> lk(D.m);
-    write_packet(D.q, k, kernargs, grid_x, block_x);
+    write_packet(D.q, k, kernargs, dim3(grid_x), dim3(block_x));
 }
 
 void direct_dispatch(DirectRing* r, const DirectKernel& k, const ArgPiece* pieces, int n_pieces, uint32_t grid_x,
@@ -425,6 +426,43 @@ void direct_dispatch(DirectRing* r, const DirectKernel& k, const ArgPiece* piece
     const char* slot = direct_stage(r, pieces, n_pieces);
     direct_flush(r->device);
     direct_submit(r, k, slot, grid_x, block_x);
+}
+
+const DirectKernel* direct_kernel_of(int device, const void* host_stub, hipStream_t stream, uint32_t bytes) {
+    static std::mutex mu;
+    static std::map<std::pair<int, const void*>, DirectKernel> known;
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = known.find({device, host_stub});
+    if (it == known.end()) {
+        DirectKernel k;
+        if (!direct_kernel(device, host_stub, stream, bytes, &k)) k = DirectKernel{};
+        it = known.emplace(std::make_pair(device, host_stub), k).first;
+    }
+    return it->second.ok() ? &it->second : nullptr;
+}
+
+void PacketList::add_blob(const void* stub, dim3 g, dim3 b, size_t lds, const char* blob, uint32_t bytes) {
+    constexpr size_t kLdsPerWorkgroup = 160 * 1024;
+    if (!ok) return;
+    const DirectKernel* k =
+        n < kMost && bytes <= kDirectSlotBytes ? direct_kernel_of(ring->device, stub, stream, bytes) : nullptr;
+    if (!k || k->group_bytes + lds > kLdsPerWorkgroup) {
+        ok = false;
+        return;
+    }
+    const ArgPiece piece{blob, 0, bytes};
+    list[n] = {*k, direct_stage(ring, &piece, 1), g, b};
+    list[n++].k.group_bytes += (uint32_t)lds;
+}
+
+bool PacketList::send() {
+    if (!ok || n == 0) return false;
+    direct_flush(ring->device);
+    DeviceQueue& D = g_dev[ring->device];
+    std::lock_guard<std::mutex> lk(D.m);
+    for (int i = 0; i < n; ++i) write_packet(D.q, list[i].k, list[i].args, list[i].g, list[i].b);
+    n = 0;
+    return true;
 }
 
 namespace {

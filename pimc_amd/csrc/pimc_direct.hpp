@@ -17,6 +17,8 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <cstring>
+#include <type_traits>
 
 namespace pimc {
 
@@ -74,6 +76,70 @@ void direct_dispatch(DirectRing* r, const DirectKernel& k, const ArgPiece* piece
 char* direct_stage(DirectRing* r, const ArgPiece* pieces, int n_pieces);
 void direct_flush(int device);
 void direct_submit(DirectRing* r, const DirectKernel& k, const char* kernargs, uint32_t grid_x, uint32_t block_x);
+// direct_kernel, remembered per device and function for the life of the process (a
+// loaded code object stays); null when the function cannot be dispatched.
+const DirectKernel* direct_kernel_of(int device, const void* host_stub, hipStream_t stream, uint32_t bytes);
+
+// The kernels of one call, in order, as packets behind one flush on the device's
+// queue.  (A packet without the barrier bit, to run beside the one before it, gained
+// nothing: the first kernel's workgroups are all dispatched before it.)  send() queues nothing and returns false when a kernel cannot
+// be dispatched: the caller then launches all of them through HIP.
+class PacketList {
+public:
+    PacketList(DirectRing* r, hipStream_t st) : ring(r), stream(st) {}
+    // Bytes copied of an argument of more than 1 KB (a request's inline bead list).
+    uint32_t long_arg_bytes = UINT32_MAX;
+    template <class... Ps, class... As>
+    void add(void (*kern)(Ps...), dim3 g, dim3 b, size_t lds, const As&... as) {
+        static_assert(sizeof...(Ps) == sizeof...(As), "one value per parameter");
+        alignas(16) char blob[kDirectSlotBytes];
+        uint32_t end = 0;
+        (put<Ps>(blob, &end, as), ...);
+        add_blob(reinterpret_cast<const void*>(kern), g, b, lds, blob, end);
+    }
+    bool send();
+
+private:
+    static constexpr int kMost = 8;
+    struct Packet {
+        DirectKernel k;
+        const char* args;
+        dim3 g, b;
+    };
+    template <class P, class A>
+    void put(char* blob, uint32_t* end, const A& a) {
+        using T = std::remove_cv_t<P>;
+        static_assert(std::is_trivially_copyable_v<T>, "an argument is copied bytewise");
+        const uint32_t o = (*end + alignof(T) - 1) / alignof(T) * alignof(T);
+        *end = o + sizeof(T);
+        if (*end > kDirectSlotBytes) return;   // add_blob refuses it
+        if constexpr (std::is_same_v<T, A>) {
+            std::memcpy(blob + o, &a, sizeof(T) > 1024 && long_arg_bytes < sizeof(T) ? long_arg_bytes : sizeof(T));
+        } else {
+            const T t = a;
+            std::memcpy(blob + o, &t, sizeof(T));
+        }
+    }
+    void add_blob(const void* stub, dim3 g, dim3 b, size_t lds, const char* blob, uint32_t bytes);
+    DirectRing* ring;
+    hipStream_t stream;
+    Packet list[kMost];
+    int n = 0;
+    bool ok = true;
+};
+
+// One kernel of a call: a packet, or a launch on the stream.
+struct Launcher {
+    hipStream_t st;
+    PacketList* packets = nullptr;
+    template <class... Ps, class... As>
+    void operator()(void (*kern)(Ps...), dim3 g, dim3 b, size_t lds, const As&... as) const {
+        if (packets)
+            packets->add(kern, g, b, lds, as...);
+        else
+            hipLaunchKernelGGL(kern, g, b, lds, st, as...);
+    }
+};
 
 // Copies from device to page-locked host memory on the DMA engines, outside any
 // HIP stream: the caller starts one when the data is complete (after an event or a

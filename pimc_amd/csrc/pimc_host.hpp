@@ -108,7 +108,7 @@ struct pimc_ctx {
     unsigned long long* d_done() { return reinterpret_cast<unsigned long long*>(d_map + kDoneSlot); }
     // the arrival counter of the S(q) kernel (zero between calls): past d_out's 16
     unsigned* d_ticket() { return reinterpret_cast<unsigned*>(d_out + 16); }
-    int wait_done(unsigned long long s);   // spin, then fall back to a stream sync
+    int wait_done(unsigned long long s, bool packet = false);   // spin, then fall back to a stream sync
     // the direct Delta V form's per-bead results (mapped, coherent pinned block)
     pimc::VnnDirectOut* h_vdir = nullptr;
     pimc::VnnDirectOut* d_vdir = nullptr;
@@ -122,6 +122,8 @@ struct pimc_ctx {
     bool asked_long = false;   // a request of more than kVnnInline beads has been made
     long direct_count = 0;   // requests dispatched as packets
     bool direct_ready(int mode);
+    bool asked_packets = false;   // an action could have gone as packets
+    bool packets_ready();
     // Every entry point returns only after its work on the stream has finished
     // or its last kernel has published its result (nothing of that kernel is
     // left but its exit), so the stream is quiet between calls -- unless a call

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "pimc_device.hpp"
+#include "pimc_direct.hpp"
 
 namespace pimc {
 
@@ -229,6 +230,7 @@ __device__ __forceinline__ int xcd_contiguous_item(int b, int G) {
 // v_host (host-mapped, or null) receives the slice sums before it.
 // g2_part (or null): gradVSquared partials [n_slices][g2_blocks] whose slice sums
 // (written to g2_slice) enter the walkers' actions with the gradient correction.
+// packets (or null): the kernels go there instead of onto the stream.
 // perm (or null): mixed mode, the window form (k_pair_window, tiles from
 // append_row_tiles(..., window = true)) over slices in the spatial order
 // launch_slice_order wrote (slice s at perm + slices[s].pos).
@@ -238,7 +240,7 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
                               double* action, const KernelTimer* timer = nullptr, bool finalize = true,
                               unsigned long long* done = nullptr, unsigned long long seq = 0,
                               const double* g2_part = nullptr, int g2_blocks = 0, double* g2_slice = nullptr,
-                              const int* perm = nullptr, double* v_host = nullptr);
+                              const int* perm = nullptr, double* v_host = nullptr, PacketList* packets = nullptr);
 // Spatial order of every slice (slices of at most kLdsBeads beads, one box):
 // perm[slices[s].pos + t], t < slices[s].n, lists slice s's beads by the index of
 // their cell along a Hilbert curve through a 32^3 grid over the box, ties by
@@ -249,7 +251,7 @@ hipError_t launch_slice_order(hipStream_t st, const SliceDesc* slices, int n_sli
 int pair_grid_for(int lds_beads, int num_cus);
 hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInline& req, const AzizDev& az,
                       const KernelTimer* timer = nullptr, double* gnn_part = nullptr, int lds_beads = 0,
-                      const KernelTimer* gnn_timer = nullptr);
+                      const KernelTimer* gnn_timer = nullptr, PacketList* packets = nullptr);
 // The direct form (k_vnn_direct): at most kVnnDirectMax beads, up to kVnnInline of
 // them travelling inline, more at A.beads (mapped host memory: each workgroup reads
 // its own 64 bytes), at most kVnnChunk beads per slice; out [n_beads] is host-mapped.
@@ -264,10 +266,12 @@ constexpr uint32_t kVdirOffAz = karg_align(kVdirOffReq + sizeof(VnnInline), alig
 constexpr uint32_t kVdirOffOut = karg_align(kVdirOffAz + sizeof(AzizDev), alignof(VnnDirectOut*));
 constexpr uint32_t kVdirBytes = kVdirOffOut + sizeof(VnnDirectOut*);
 // gradVSquared(slice) partials [M][blocks_per_slice] for the even (need bit 0) and
-// odd (bit 1) slices, 0 for the others.
+// odd (bit 1) slices, 0 for the others.  packets takes the chunked form only (chunks >
+// 1).
 hipError_t launch_gradv2(int mode, hipStream_t st, const double* pos, int64_t plane, int nalloc, int num_slices,
                          const int* nbs, const BoxDev& box, const AzizDev& az, int lds_beads, double* part,
-                         int* blocks_per_slice, int chunks = 1, double* fpart = nullptr, int need = 3);
+                         int* blocks_per_slice, int chunks = 1, double* fpart = nullptr, int need = 3,
+                         PacketList* packets = nullptr);
 // Partner chunks of the gradVSquared sum that fill the CUs (1: one pass).
 int gradv2_chunks(int nalloc, int num_slices, int num_cus);
 // Device-resident chain (pimc_dchain.hip): one workgroup runs n_moves moves.

@@ -364,13 +364,13 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_action(const RowTile* __r
                                                               const int* __restrict__ ranges,
                                                               const WalkerDesc* __restrict__ walkers,
                                                               const double* __restrict__ pos, AzizDev az,
-                                                              double* __restrict__ partials) {
+                                                              double* __restrict__ partials, int groups) {
     // x | y | z of one slice, PSL each, then the block sum's wave partials: a
     // static array, so its address is a constant folded into the reads' offsets
     constexpr int PSL = pair_lds_plane<PS>();
     __shared__ double lds[3 * PSL + kPairThreads / 64];
     double* red = lds + 3 * PSL;
-    const int r = xcd_contiguous_item(blockIdx.x, gridDim.x);
+    const int r = xcd_contiguous_item(blockIdx.x, groups);
     const int k_begin = ranges[r], k_end = ranges[r + 1];
     if (k_begin >= k_end) return;
     int staged = -1;
@@ -1053,7 +1053,7 @@ __global__ __launch_bounds__(256) void k_gradv2_sum(const int* __restrict__ nbs,
         f2 = norm2_exact(fx, fy, fz);
     }
     const double s = block_sum<256>(f2, red);
-    if (threadIdx.x == 0) part[(int64_t)m * gridDim.x + b] = s;
+    if (threadIdx.x == 0) part[(int64_t)m * ((nalloc + 255) >> 8) + b] = s;
 }
 
 int gradv2_chunks(int nalloc, int num_slices, int num_cus) {
@@ -1620,7 +1620,7 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
                               const double* pos, const AzizDev& az, int lds_beads, double* partials, double* v_slice,
                               double* action, const KernelTimer* timer, bool finalize, unsigned long long* done,
                               unsigned long long seq, const double* g2_part, int g2_blocks, double* g2_slice,
-                              const int* perm, double* v_host) {
+                              const int* perm, double* v_host, PacketList* packets) {
     (void)hipGetLastError();  // drop any stale error of an earlier call
     if (n_tiles <= 0 || G <= 0) return hipSuccess;
     const bool spatial = perm != nullptr;
@@ -1630,7 +1630,8 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
     // reads share one address)
     const int PS = lds_beads <= 0 ? 0 : lds_beads <= 256 ? 256 : lds_beads <= 512 ? 512 : lds_beads <= 1024 ? 1024 : 2048;
     if (lds_beads > kLdsBeads) return hipErrorInvalidValue;
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, b, 0, st, tiles, ranges, walkers, pos, az, partials); };
+    const Launcher launch{st, packets};
+    auto go = [&](auto kern) { launch(kern, g, b, 0, tiles, ranges, walkers, pos, az, partials, G); };
     auto by_ps = [&](auto mode_tag) {
         constexpr int MODE = decltype(mode_tag)::value;
         if (MODE == 0 && spatial) {
@@ -1657,8 +1658,8 @@ hipError_t launch_pair_action(int mode, hipStream_t st, const RowTile* tiles, in
         by_ps(std::integral_constant<int, 2>{});
     if (timer && timer->stop) (void)hipEventRecord(timer->stop, st);
     if (finalize)
-        hipLaunchKernelGGL(k_pair_finalize, dim3(1), dim3(kFinThreads), 0, st, n_tiles, slices, n_slices, walkers,
-                           n_walkers, partials, v_slice, action, done, seq, g2_part, g2_blocks, g2_slice, v_host);
+        launch(k_pair_finalize, dim3(1), dim3(kFinThreads), 0, n_tiles, slices, n_slices, walkers, n_walkers, partials,
+               v_slice, action, done, seq, g2_part, g2_blocks, g2_slice, v_host);
     return hipGetLastError();
 }
 
@@ -1762,7 +1763,8 @@ const void* vnn_direct_stub(int mode, bool listed) {
 }
 
 hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInline& req, const AzizDev& az,
-                      const KernelTimer* timer, double* gnn_part, int lds_beads, const KernelTimer* gnn_timer) {
+                      const KernelTimer* timer, double* gnn_part, int lds_beads, const KernelTimer* gnn_timer,
+                      PacketList* packets) {
     (void)hipGetLastError();  // drop any stale error of an earlier call
     if (A.n_beads <= 0) return hipSuccess;
     dim3 g(A.chunks, A.n_beads), b(kVnnThreads);
@@ -1785,13 +1787,10 @@ hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInlin
         // kernel has its own duration)
         const size_t lds = sizeof(double) * 3 * (size_t)lds_beads + sizeof(int) * (size_t)A.nalloc;
         dim3 gg(A.chunks * A.n_beads + A.gnn_chunks * (A.gnn_shared ? 1 : 2) * A.n_beads);
-        if (mode == 0)
-            hipLaunchKernelGGL(k_vnn_gnn<0>, gg, dim3(256), lds, st, A, req, az, lds_beads, gnn_part);
-        else if (mode == 1)
-            hipLaunchKernelGGL(k_vnn_gnn<1>, gg, dim3(256), lds, st, A, req, az, lds_beads, gnn_part);
-        else
-            hipLaunchKernelGGL(k_vnn_gnn<2>, gg, dim3(256), lds, st, A, req, az, lds_beads, gnn_part);
-        hipLaunchKernelGGL(k_vnn_finalize, dim3(1), dim3(256), 0, st, A, req);
+        const Launcher launch{st, packets};
+        auto gnn = [&](auto kern) { launch(kern, gg, dim3(256), lds, A, req, az, lds_beads, gnn_part); };
+        mode == 0 ? gnn(k_vnn_gnn<0>) : mode == 1 ? gnn(k_vnn_gnn<1>) : gnn(k_vnn_gnn<2>);
+        launch(k_vnn_finalize, dim3(1), dim3(256), 0, A, req);
         return hipGetLastError();
     }
     if (mode == 0)
@@ -1820,29 +1819,24 @@ hipError_t launch_vnn(int mode, hipStream_t st, const VnnArgs& A, const VnnInlin
 
 hipError_t launch_gradv2(int mode, hipStream_t st, const double* pos, int64_t plane, int nalloc, int num_slices,
                          const int* nbs, const BoxDev& box, const AzizDev& az, int lds_beads, double* part,
-                         int* blocks_per_slice, int chunks, double* fpart, int need) {
+                         int* blocks_per_slice, int chunks, double* fpart, int need, PacketList* packets) {
     (void)hipGetLastError();
     const int B = (nalloc + 255) / 256;
     *blocks_per_slice = B;
     const size_t lds = sizeof(double) * 3 * (size_t)lds_beads;
-    if (chunks > 1 && fpart && mode == 0 && nalloc <= 256) {
-        hipLaunchKernelGGL(k_gradv2_sym, dim3(chunks, num_slices), dim3(256), 0, st, pos, plane, nalloc, nbs, box, az,
-                           chunks, need, fpart);
-        hipLaunchKernelGGL(k_gradv2_sum, dim3(B, num_slices), dim3(256), 0, st, nbs, nalloc, chunks, need, fpart, part);
-        return hipGetLastError();
-    }
     if (chunks > 1 && fpart) {
-        dim3 gc(B * chunks, num_slices), b(256);
-        if (mode == 0)
-            hipLaunchKernelGGL(k_gradv2_chunk<0>, gc, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, chunks,
-                               need, fpart);
-        else if (mode == 1)
-            hipLaunchKernelGGL(k_gradv2_chunk<1>, gc, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, chunks,
-                               need, fpart);
-        else
-            hipLaunchKernelGGL(k_gradv2_chunk<2>, gc, b, lds, st, pos, plane, nalloc, nbs, box, az, lds_beads, chunks,
-                               need, fpart);
-        hipLaunchKernelGGL(k_gradv2_sum, dim3(B, num_slices), b, 0, st, nbs, nalloc, chunks, need, fpart, part);
+        const Launcher launch{st, packets};
+        if (mode == 0 && nalloc <= 256) {
+            launch(k_gradv2_sym, dim3(chunks, num_slices), dim3(256), 0, pos, plane, nalloc, nbs, box, az, chunks,
+                   need, fpart);
+        } else {
+            auto go = [&](auto kern) {
+                launch(kern, dim3(B * chunks, num_slices), dim3(256), lds, pos, plane, nalloc, nbs, box, az,
+                       lds_beads, chunks, need, fpart);
+            };
+            mode == 0 ? go(k_gradv2_chunk<0>) : mode == 1 ? go(k_gradv2_chunk<1>) : go(k_gradv2_chunk<2>);
+        }
+        launch(k_gradv2_sum, dim3(B, num_slices), dim3(256), 0, nbs, nalloc, chunks, need, fpart, part);
         return hipGetLastError();
     }
     dim3 g(B, num_slices), b(256);

@@ -319,8 +319,9 @@ struct SymShare {
 // of tiles both waves of a tile pair take half of the offsets.  The groups share out
 // the offsets.  16 waves per CU (126 VGPRs), each workgroup with an equal
 // share of all slices' offsets: with half a slice with T or a whole one without it
-// as the unit, N = 256 and M = 166 took 72 us (two uneven rounds of the CUs).  A sum entry is nine doubles (18 banks: the 32 lanes
-// of a half-wave hit 32 different pairs of banks).
+// as the unit, N = 256 and M = 166 took 72 us (two uneven rounds of the CUs).
+// A sum entry is nine doubles (18 banks: the 32 lanes of a half-wave hit 32 different
+// pairs of banks).
 // N = 256, M = 166, T on odd slices: 41 us (61 % of it issuing VALU instructions),
 // against 55 us as ordered pairs with chunks of partners.
 template <int MODE>
@@ -466,7 +467,7 @@ __global__ __launch_bounds__(256) void k_virial_sum(VirialArgs A) {
     __syncthreads();
     if (threadIdx.x < kVirialTerms) {
         const int q = threadIdx.x;
-        A.part[((int64_t)m * gridDim.x + b) * kVirialTerms + q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
+        A.part[((int64_t)m * ((A.nalloc + 255) >> 8) + b) * kVirialTerms + q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
         if (A.part_on_host) __threadfence_system();
     }
 }

@@ -1,0 +1,67 @@
+"""Actions, energies and Delta V with the gradient correction as packets on the device
+queue against the same kernels launched through HIP: bit for bit, in every mode, for
+repeated calls between moves, with links given and changed, and from two threads whose
+contexts share the queue."""
+import threading
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_direct import _context
+
+pytestmark = pytest.mark.gpu
+
+GSF = ((2.0 / 3.0, 4.0 / 3.0), (0.0, 2.0 / 9.0), 2)
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import pimc_amd
+    return pimc_amd
+
+
+def _walk(gpu, packets, mode, M, N, correction, seed):
+    L = (N / 0.02198) ** (1.0 / 3.0)
+    rng = np.random.default_rng(seed)
+    b = rng.uniform(-0.5 * L, 0.5 * L, size=(M, N, 3))
+    ctx = _context(gpu, L, M, N, 0.004, L, mode, b, packets=packets)
+    if correction:
+        ctx.set_action_factors(*GSF)
+    nxt = np.stack([(np.arange(M)[:, None] + 1) % M + np.zeros((1, N), int),
+                    np.zeros((M, 1), int) + np.arange(N)], axis=-1).astype(np.int32)
+    swap = nxt.copy()
+    if N > 1:
+        swap[M - 1, 0, 1], swap[M - 1, 1, 1] = 1, 0
+    out = []
+    for k in range(6):
+        n = min(M, 7 + 5 * k)
+        sp = np.stack([rng.permutation(M)[:n], rng.integers(0, N, n)], axis=-1).astype(np.int32)
+        new = rng.uniform(-0.5 * L, 0.5 * L, size=(n, 3))
+        out.append(np.asarray(ctx.delta_action(sp, new, commit=True)))
+        a, v = ctx.potentialAction(with_slices=True)
+        out += [np.asarray(a), np.asarray(v), np.asarray(ctx.potentialAction())]
+        links = (None, nxt, swap)[k % 3]
+        out.append(np.asarray(list(ctx.energy(next_links=links).values())))
+        out.append(np.asarray(list(ctx.virial_energy(3, next_links=links).values())))
+    return out, ctx.download_path()
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("M,N,correction", [(40, 64, True), (41, 65, False), (20, 300, True), (6, 1, True)])
+def test_packets_equal_launches(gpu, mode, M, N, correction):
+    a, pa = _walk(gpu, True, mode, M, N, correction, M)
+    b, pb = _walk(gpu, False, mode, M, N, correction, M)
+    assert np.array_equal(pa, pb)
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y, equal_nan=True), k
+
+
+def test_two_threads(gpu):
+    want = {s: _walk(gpu, False, 0, 40, 64, True, s) for s in (1, 2)}
+    got = {}
+    ts = [threading.Thread(target=lambda s=s: got.update({s: _walk(gpu, True, 0, 40, 64, True, s)})) for s in (1, 2)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for s in (1, 2):
+        assert np.array_equal(got[s][1], want[s][1])
+        assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(got[s][0], want[s][0]))
