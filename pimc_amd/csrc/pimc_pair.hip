@@ -664,12 +664,32 @@ __global__ __launch_bounds__(kFinThreads) void k_pair_finalize(int n_items, cons
         if (threadIdx.x == 0) fi[n_slices] = n_items;
     }
     __syncthreads();
-    const double* src = staged ? sp : partials;
-    for (int sl = threadIdx.x; sl < n_slices; sl += kFinThreads) {
+    // Sixteen lanes per slice where the partials stay in HBM (a large slice has a few
+    // hundred: one lane's chain of loads took 16 us at N = 777 x 61, 9 us so), one
+    // where they are in LDS.
+    const int per = !staged && small ? 16 : 1;
+    const int sub = threadIdx.x & (per - 1);
+    for (int sl = threadIdx.x / per; sl < n_slices; sl += kFinThreads / per) {
         const int b = small ? fi[sl] : slices[sl].first_item;
         const int e = small ? fi[sl + 1] : ((sl + 1 < n_slices) ? slices[sl + 1].first_item : n_items);
         double v = 0.0;
-        for (int k = b; k < e; ++k) v += src[k];
+        if (staged)
+            for (int k = b; k < e; ++k) v += sp[k];
+        else
+            for (int k = b + sub; k < e; k += 16 * per) {
+                double t[16];   // sixteen loads in flight
+#pragma unroll
+                for (int u = 0; u < 16; ++u) t[u] = k + u * per < e ? partials[k + u * per] : 0.0;
+#pragma unroll
+                for (int u = 0; u < 16; ++u) v += t[u];
+            }
+        if (per == 16) {
+            v += __shfl_xor(v, 8, 16);
+            v += __shfl_xor(v, 4, 16);
+            v += __shfl_xor(v, 2, 16);
+            v += __shfl_xor(v, 1, 16);
+            if (sub) continue;
+        }
         v_slice[sl] = v;
         if (small) vs[sl] = v;
         if (v_host) v_host[sl] = v;
