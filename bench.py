@@ -464,7 +464,9 @@ def large_leg(pimc_amd, cpu, reps=10, sq_reps=3):
     ctx.close()
     rho_s = (rho_ms + rho2_ms) / max(rho_n + rho2_n, 1) * 1e-3
     lag_s = lag_ms / max(lag_n, 1) * 1e-3
-    rho_flop = nq * M * N * F_QB + nq * M * F_QMT
+    # one density mode per pair of q and -q (the list is symmetric and holds q = 0)
+    n_modes = (nq + 1) // 2
+    rho_flop = n_modes * M * N * F_QB + n_modes * M * F_QMT
     out = {"workload": "He-4 N=2048, rho=0.02198 A^-3, T=1.0 K, tau=0.004, M=250, rc=L/2, Aziz 1979, "
                        "Gaussian-bridge worldlines; full action + S(q) + F(q,tau) on 100401 lattice q (|q|<=4 A^-1)",
            "action": a, "pairs_per_launch": pairs, "total_action_wall_ms": wall * 1e3,
@@ -475,7 +477,7 @@ def large_leg(pimc_amd, cpu, reps=10, sq_reps=3):
                              "avg_launch_us": pa_s * 1e6, "flop_per_pair": F_PAIR},
            "n_q": int(nq), "ssf_wall_ms": ssf_wall * 1e3, "isf_wall_ms": isf_wall * 1e3,
            "isf_wall_ms_pageable_result": isf_wall_pageable * 1e3,
-           "roofline_rho": {"bound": "valu", "kernel": "k_rho_lattice", "achieved": rho_flop / rho_s / 1e12,
+           "roofline_rho": {"bound": "mfma", "kernel": "k_rho_matrix", "n_modes": int(n_modes), "achieved": rho_flop / rho_s / 1e12,
                             "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                             "frac": rho_flop / rho_s / 1e12 / PEAK_FP32_TFLOPS, "avg_launch_ms": rho_s * 1e3,
                             "flop_per_q_bead": F_QB, "q_bead_phasors_per_s": nq * M * N / rho_s},

@@ -456,17 +456,16 @@ int pimc_set_timing(pimc_ctx* ctx, int enable);
 int pimc_set_timing_kinds(pimc_ctx* ctx, unsigned kinds);
 /* Besides the names above, "delta_packets" counts the Delta V requests sent as
  * dispatch packets straight into the device's AQL queue (total_ms 0): requests
- * of up to 32 beads on slices of up to 1024, without the gradient correction
- * or per-bead outputs, while timing of "delta_action" is off.  The environment
+ * of up to 512 beads on slices of up to 1024 (32 with the gradient correction),
+ * without per-bead outputs, while timing of "delta_action" (with the correction: of
+ * any kernel) is off.  The environment
  * variable PIMC_DIRECT_DISPATCH=0, read when a context is created, sends them
- * through hipLaunchKernel instead.  "isf_chunks" counts the q chunks of
- * pimc_isf calls that took the chunked form (total_ms 0): lattice q only, at
- * least 2048 of them, results of 4 MB and more into page-locked memory
- * (pimc_host_alloc), while timing of "rho" and "isf" is off; lists of up to
- * 68 000 q run as two halves, longer ones in chunks of 34 000 q (more when the
- * list exceeds 64 chunks); each chunk computes its density modes and lags
- * while the previous chunk's rows are copied out on a second stream, with the
- * same values as one launch per kernel. */
+ * through hipLaunchKernel instead.  "isf_chunks" counts the q of pimc_isf calls
+ * that took the piecewise form, in parts of 34 000 and at least two per call
+ * (total_ms 0): lattice q only, at least 2048 of them, results of 4 MB and more
+ * into page-locked memory (pimc_host_alloc), while timing of "rho" and "isf" is
+ * off; each piece computes its density modes and lags while the DMA engines copy
+ * the previous piece's rows out, with the same values as one launch per kernel. */
 int pimc_kernel_time(pimc_ctx* ctx, const char* name, double* total_ms, long* count);
 int pimc_device_synchronize(void);
 /* Page-locked host memory for large results (no counterpart in the reference,
