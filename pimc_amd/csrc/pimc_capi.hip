@@ -394,10 +394,10 @@ bool pimc_ctx::direct_ready(int mode) {
     return direct_state == 1 && mode >= 0 && mode < 3 && dk_vdir[2 * mode].ok();
 }
 
-// May the kernels of an action go as packets?  For calls whose
-// kernels take a few tens of microseconds (a packet holds up the device queue's later
-// ones, other contexts' too); untimed.  A context's first such call goes through HIP:
-// setting the ring up costs more than one call gains.
+// May the kernels of an action go as packets?  Untimed calls whose kernels take a few
+// tens of microseconds (a packet holds up the device queue's later ones, other
+// contexts' too).  A context's first such call goes through HIP: setting the ring up
+// costs more than one call gains.
 bool pimc_ctx::packets_ready() {
     constexpr double kMostPairs = 1.6e7;
     const double N = desc.num_alloc;
@@ -1476,7 +1476,7 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         const KernelTimer kt = c->kernel_timer(1);
         // a packet on the device's AQL queue when the call is not timed (the
         // timing events live on the stream) and the context's stream is quiet:
-        // the two never run work of one context at once
+        // the two never run work of one context at once.
         // Setting up the queue's argument ring takes about 12 us, two requests'
         // gain: a context's first long request goes through HIP.
         const bool first_long = !inline_req && c->direct_state < 0 && !c->asked_long;
