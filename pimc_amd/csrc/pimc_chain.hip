@@ -36,6 +36,10 @@ struct pimc_chain {
     double side = 0, tau = 0, lambda = 0;
     double sqrtLambdaTau = 0, sqrt2LambdaTau = 0;
     std::vector<double> pos;              // [M][N][3], equal to the device copy
+    // the context's path_version `pos` is the copy of; any other value: beads have
+    // been changed past the chain, and the next device run takes the whole path back
+    uint64_t copied = 0;
+    static constexpr uint64_t kNoCopy = ~0ull;
     std::vector<int> wind;                // winding sectors, 3 per sector
     std::vector<double> cumrho0;
     std::string err;
@@ -507,6 +511,12 @@ static int run_chains_on_device(pimc_chain* const* chains, int n, int n_moves, c
     if (e == hipSuccess) e = hipMemcpyAsync(lead->h_out, lead->d_out, out_bytes, hipMemcpyDeviceToHost, st);
     const hipError_t e1 = hipStreamSynchronize(st);   // quiet after an error too: the blocks are reused
     if (e == hipSuccess) e = e1;
+    // the host copies that were the device path's before this run
+    std::vector<char> current(n);
+    for (int c = 0; c < n; ++c) {
+        current[c] = chains[c]->copied == chains[c]->ctx->path_version;
+        chains[c]->copied = pimc_chain::kNoCopy;   // until the run's beads have come back
+    }
     if (e != hipSuccess) return lead->fail(PIMC_E_HIP, std::string("chain kernel: ") + hipGetErrorString(e));
     for (int c = 0; c < n; ++c) ++chains[c]->ctx->path_version;   // the launch moved their beads
     for (int c = 0; c < n; ++c) {
@@ -516,8 +526,9 @@ static int run_chains_on_device(pimc_chain* const* chains, int n, int n_moves, c
         ch.rng.left = (int)mt[MtRand::N];
         ch.rng.next = (int)mt[MtRand::N + 1];
         if (near) near[c] = reinterpret_cast<const int*>(lead->h_out + q_near)[c];
-        // the host copy follows the device path: the moved worldlines, in bead order
-        if (compact) {
+        // the host copy follows the device path: the moved worldlines, in bead order,
+        // or all of it where beads have been changed past the chain
+        if (compact && current[c]) {
             const char* flag = lead->h_out + q_flags + flag_of[c];
             const double* src = lead->h_beads + moved_of[c];
             for (int i = 0; i < ch.N; ++i) {
@@ -533,6 +544,7 @@ static int run_chains_on_device(pimc_chain* const* chains, int n, int n_moves, c
             const int r = pimc_download_path(ch.ctx, ch.pos.data());
             if (r) return ch.fail(r, pimc_last_error(ch.ctx));
         }
+        ch.copied = ch.ctx->path_version;
     }
     if (accepted) std::memcpy(accepted, lead->h_out + q_acc, sizeof(int) * (size_t)n * n_moves);
     if (info) std::memcpy(info, lead->h_out + q_info, sizeof(double) * 3 * (size_t)n * n_moves);
@@ -586,6 +598,7 @@ int pimc_chain_create(pimc_ctx* ctx, const pimc_chain_desc* d, pimc_chain** out)
     ch->pos.resize(3 * (size_t)M * N);
     const int r = pimc_download_path(ctx, ch->pos.data());
     if (r) return r;
+    ch->copied = ctx->path_version;
     *out = ch.release();
     return PIMC_OK;
 }
@@ -607,16 +620,16 @@ int pimc_chain_run_device_many(pimc_chain* const* chains, int n_chains, int n_mo
 
 int pimc_chain_move(pimc_chain* ch, int kind, int* accepted, double* info3) {
     if (!ch || !accepted) return PIMC_E_ARG;
-    double info[3] = {0.0, 0.0, 0.0};
-    int r;
-    if (kind == 0)
-        r = ch->staging(accepted, info);
-    else if (kind == 1)
-        r = ch->bisection(accepted, info);
-    else if (kind == 2)
-        r = ch->com(accepted, info);
-    else
+    if (kind < 0 || kind > 2)
         return ch->fail(PIMC_E_ARG, "move kind must be 0 (staging), 1 (bisection) or 2 (center of mass)");
+    double info[3] = {0.0, 0.0, 0.0};
+    // a move writes the same beads to both copies; one that fails may not have
+    const bool current = ch->copied == ch->ctx->path_version;
+    ch->copied = pimc_chain::kNoCopy;
+    const int r = kind == 0   ? ch->staging(accepted, info)
+                  : kind == 1 ? ch->bisection(accepted, info)
+                              : ch->com(accepted, info);
+    if (current && r == PIMC_OK) ch->copied = ch->ctx->path_version;
     if (info3) std::memcpy(info3, info, sizeof(info));
     return r;
 }

@@ -42,3 +42,32 @@ def test_uneven_chains(gpu, moves):
         # a host-driven move goes on from there
         c.move("com")
         assert np.array_equal(c.positions(), ctx.download_path())
+
+
+@pytest.mark.parametrize("how", ["update_beads", "delta_action", "upload_path", "another chain"])
+def test_beads_changed_past_the_chain(gpu, how):
+    """Beads changed through the context, or by another chain on it, between two device
+    runs: after the second the chain's host copy is the device path, whichever worldlines
+    that run moved."""
+    rng = np.random.default_rng(3)
+    N, M = 40, 12
+    ctx, chain = _chain(gpu, N, M, 1, 6)
+    other = gpu.Chain(ctx, 5, 6, 2, True, 1, 0.3)
+    chain.run_device(KINDS)
+    sp = np.stack([np.arange(M), rng.integers(0, N, M)], axis=-1).astype(np.int32)
+    new = rng.uniform(-3.0, 3.0, size=(M, 3))
+    if how == "update_beads":
+        ctx.update_beads(sp, new)
+    elif how == "delta_action":
+        ctx.delta_action(sp, new, commit=True)
+    elif how == "upload_path":
+        ctx.upload_path(np.ascontiguousarray(ctx.download_path()[:, ::-1]))
+    else:
+        other.run_device(KINDS)
+        other.move("staging")
+    chain.run_device(["staging"])
+    assert np.array_equal(chain.positions(), ctx.download_path())
+    # and in step again: a host-driven move, then a run that moves few worldlines
+    chain.move("com")
+    chain.run_device(["bisection"])
+    assert np.array_equal(chain.positions(), ctx.download_path())
