@@ -183,6 +183,10 @@ AzizDev make_aziz_dev(const AzizParams& p, double max_sep) {
     a.A = p.A;
     a.alpha = p.alpha;
     a.beta = p.beta;
+    const long double l2e = 1.442695040888963407359924681001892137L;
+    a.e2_alpha = (double)(-(long double)p.alpha * l2e);
+    a.e2_beta = (double)((long double)p.beta * l2e);
+    a.e2_lo = (double)(-(long double)p.alpha * l2e - (long double)a.e2_alpha);
     a.D = p.D;
     a.C6 = p.C6;
     a.C8 = p.C8;

@@ -39,6 +39,9 @@ struct AzizDev {
     double eC6k, eC8k, eC10k, Ds;
     // FP64 closed form
     double eps, A, alpha, beta, D, C6, C8, C10;
+    // its repulsion A exp(-alpha x + beta x^2) = A 2^(x (e2_alpha + e2_beta x + e2_lo)):
+    // -alpha log2 e and beta log2 e rounded, and what -alpha log2 e lost
+    double e2_alpha, e2_beta, e2_lo;
     double eps_rm;         // epsilon / rm (dV/dr = (epsilon/rm) dV/dx)
     double inv_rm;         // 1 / rm
     const double* table;   // device lookupV (PIMC_V_TABLE)
@@ -178,51 +181,70 @@ __device__ __forceinline__ double recip64(double x) {
     return fma(r, fma(-x, r, 1.0), r);
 }
 
-// A constant kept in scalar registers across a loop: as the third operand of an FMA it
-// costs nothing, as a literal two moves each time.
+// A constant kept in scalar registers across a loop (LOOP): as the third operand of an
+// FMA it costs nothing, as a literal two moves each time.  The kernels that evaluate a
+// pair or two per lane take literals: the scalar registers hold their arguments, and
+// spilling those would give them a scratch segment.
+template <bool LOOP>
 __device__ __forceinline__ double in_sgpr(double x) {
-    asm("" : "+s"(x));
+    if (LOOP) asm("" : "+s"(x));
     return x;
 }
 
-// 2^(u v) in FP64, u v finite and far from the overflow (an underflow gives 0): the
-// nearest whole power times a polynomial of degree 11 in the rest f, |f| <= 1/2, the
-// minimax one of the relative error (Remez exchange in 60 digits; 3e-18).  f takes the
-// product unrounded.  17 instructions,
-// where the library's exp takes 40 with its range checks and literals (full action in
-// FP64, N = 777 x 61: 150 -> 141 us).
-__device__ __forceinline__ double exp2_64(double u, double v) {
-    const double n = __builtin_rint(u * v), f = fma(u, v, -n);
-    double p = in_sgpr(0x1.e7aa1ce7ef177p-32);
-    p = fma(p, f, in_sgpr(0x1.e620fb1d29654p-28));
-    p = fma(p, f, in_sgpr(0x1.b5267881823dep-24));
-    p = fma(p, f, in_sgpr(0x1.62bfc3c215fd6p-20));
-    p = fma(p, f, in_sgpr(0x1.ffcbfba7bdac9p-17));
-    p = fma(p, f, in_sgpr(0x1.43091310bf3d3p-13));
-    p = fma(p, f, in_sgpr(0x1.5d87fe78cf25ap-10));
-    p = fma(p, f, in_sgpr(0x1.3b2ab6fb9f414p-7));
-    p = fma(p, f, in_sgpr(0x1.c6b08d7049fd1p-5));
-    p = fma(p, f, in_sgpr(0x1.ebfbdff82c5adp-3));
-    p = fma(p, f, in_sgpr(0x1.62e42fefa39efp-1));
+// 2^(u v + lo v) in FP64, u v finite and far from the overflow (an underflow gives 0), lo
+// below the rounding of u: the nearest whole power times a polynomial of degree 11 in
+// the rest f, |f| <= 1/2, the minimax one of the relative error (Remez exchange in 60
+// digits; 3e-18).  f takes the product unrounded.  18 instructions, where the library's
+// exp takes 40 with its range checks and literals (full action in FP64, N = 777 x 61:
+// 150 -> 141 us).  lo carries the part of a coefficient that its rounding cut off:
+// without it the repulsion of the 1995 parameters is off by 9.2e-16 (rms over x = 0.6 ..
+// 0.9) where the plain FP64 exponential of the exponent is off by 7.7e-16; with it 7.0e-16
+// (1979: 4.3e-16 against 6.7e-16, 1987: 7.0e-16 against 7.6e-16).
+template <bool LOOP>
+__device__ __forceinline__ double exp2_64(double u, double lo, double v) {
+    const double n = __builtin_rint(u * v);
+    double f = fma(u, v, -n);
+    if (!(__builtin_constant_p(lo) && lo == 0.0)) f = fma(lo, v, f);
+    double p = in_sgpr<LOOP>(0x1.e7aa1ce7ef177p-32);
+    p = fma(p, f, in_sgpr<LOOP>(0x1.e620fb1d29654p-28));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.b5267881823dep-24));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.62bfc3c215fd6p-20));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.ffcbfba7bdac9p-17));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.43091310bf3d3p-13));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.5d87fe78cf25ap-10));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.3b2ab6fb9f414p-7));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.c6b08d7049fd1p-5));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.ebfbdff82c5adp-3));
+    p = fma(p, f, in_sgpr<LOOP>(0x1.62e42fefa39efp-1));
     p = fma(p, f, 1.0);
     return __builtin_amdgcn_ldexp(p, (int)n);
 }
-constexpr double kLog2e = 1.4426950408889634074;
+// exp(-u) of the damping factor, u >= 0 (what log2 e loses by its rounding is below 2e-17 u)
+template <bool LOOP>
+__device__ __forceinline__ double exp_neg64(double u) { return exp2_64<LOOP>(-1.4426950408889634074, 0.0, u); }
+// exp(-alpha x + beta x^2) of the repulsion
+template <bool LOOP>
+__device__ __forceinline__ double aziz_exp64(double x, const AzizDev& a) {
+    return exp2_64<LOOP>(fma(a.e2_beta, x, a.e2_alpha), a.e2_lo, x);
+}
 
 // valueV at the bin radius, FP64 arithmetic.  Requires k_eps <= k < table_length.
+template <bool LOOP = false>
 __device__ __forceinline__ double aziz_v64(int k, const AzizDev& a) {
     const double x = (double)k * a.s;
-    const double ix = recip64(x);
-    const double ix2 = ix * ix;
+    // 1/x^2 by one reciprocal of the square, two roundings as in the quotient 1 / (x x);
+    // the square of a reciprocal takes three (relative rms error of V over x = 1.5 .. 2:
+    // 4.6e-16 against 3.2e-16)
+    const double ix2 = recip64(x * x);
     const double disp = (ix2 * ix2 * ix2) * fma(fma(a.C10, ix2, a.C8), ix2, a.C6);
     // the repulsion is below the rounding of the difference in a wave of far bins
     double rep = 0.0;
-    if (__builtin_amdgcn_ballot_w64(k < a.k_far)) rep = a.A * exp2_64(fma(kLog2e * a.beta, x, -kLog2e * a.alpha), x);
+    if (__builtin_amdgcn_ballot_w64(k < a.k_far)) rep = a.A * aziz_exp64<LOOP>(x, a);
     if (k < a.k_hc) return a.eps * rep;
     double F = 1.0;
     if (k < a.k_d) {
-        const double u = fma(a.D, ix, -1.0);
-        F = exp2_64(-kLog2e, u * u);
+        const double u = fma(a.D * x, ix2, -1.0);
+        F = exp_neg64<LOOP>(u * u);
     }
     return a.eps * fma(-disp, F, rep);
 }
@@ -231,7 +253,7 @@ __device__ __forceinline__ double aziz_v64(int k, const AzizDev& a) {
 // Requires k_eps <= k < table_length.
 __device__ __forceinline__ double aziz_dvdr64(int k, const AzizDev& a) {
     const double x = (double)k * a.s;
-    const double T1 = a.A * (-a.alpha + 2.0 * a.beta * x) * exp2_64(fma(kLog2e * a.beta, x, -kLog2e * a.alpha), x);
+    const double T1 = a.A * (-a.alpha + 2.0 * a.beta * x) * aziz_exp64<true>(x, a);
     if (k < a.k_hc) return a.eps_rm * T1;
     const double ix = 1.0 / x;
     const double ix2 = ix * ix;
@@ -240,7 +262,7 @@ __device__ __forceinline__ double aziz_dvdr64(int k, const AzizDev& a) {
     double F = 1.0, dF = 0.0;
     if (k < a.k_d) {
         const double t = a.D * ix - 1.0;
-        const double e = exp2_64(-kLog2e, t * t);
+        const double e = exp_neg64<true>(t * t);
         F = e;
         dF = 2.0 * a.D * ix2 * t * e;
     }
@@ -255,7 +277,7 @@ __device__ __forceinline__ double aziz_dvdr64(int k, const AzizDev& a) {
 __device__ __forceinline__ double aziz_d2vdr2_64(int k, const AzizDev& a) {
     const double x = (double)k * a.s;
     const double ab = (a.alpha - 2.0 * a.beta * x) * (a.alpha - 2.0 * a.beta * x);
-    const double T1 = a.A * (2.0 * a.beta + ab) * exp2_64(fma(kLog2e * a.beta, x, -kLog2e * a.alpha), x);
+    const double T1 = a.A * (2.0 * a.beta + ab) * aziz_exp64<true>(x, a);
     if (k < a.k_hc) return a.eps_rm * T1;
     const double ix = 1.0 / x;
     const double ix2 = ix * ix;
@@ -265,7 +287,7 @@ __device__ __forceinline__ double aziz_d2vdr2_64(int k, const AzizDev& a) {
     double F = 1.0, dF = 0.0, d2F = 0.0;
     if (k < a.k_d) {
         const double t = a.D * ix - 1.0;
-        const double e = exp2_64(-kLog2e, t * t);
+        const double e = exp_neg64<true>(t * t);
         F = e;
         dF = 2.0 * a.D * ix2 * t * e;
         const double D = a.D;

@@ -149,7 +149,7 @@ __device__ __forceinline__ double pair_term_exact(const RowMixed& q, double xi, 
     }
     const bool in = (unsigned)(k - a.k_eps) < (unsigned)(a.table_length - a.k_eps);
     if (MODE == 2) return in ? a.table[k] : 0.0;
-    const double v = aziz_v64(in ? k : a.k_hc, a);
+    const double v = aziz_v64<true>(in ? k : a.k_hc, a);
     return in ? v : 0.0;
 }
 

@@ -706,8 +706,8 @@ void pimc_server::build_batch(BatchLaunch* L) {
 // is unavailable, and every batch then launches through HIP.
 bool pimc_server::setup_direct() {
     if (hipGetDevice(&device) != hipSuccess) return false;
-    static_assert(sizeof(ServeVnnArgs) == 272 && offsetof(ServeVnnArgs, az) == 32 &&
-                      offsetof(ServeVnnArgs, chunk) == 256 && offsetof(ServeVnnArgs, partials) == 264 &&
+    static_assert(sizeof(ServeVnnArgs) == 296 && offsetof(ServeVnnArgs, az) == 32 &&
+                      offsetof(ServeVnnArgs, chunk) == 280 && offsetof(ServeVnnArgs, partials) == 288 &&
                       sizeof(ServeFinArgs) == 48,
                   "serve argument blocks");
     const void* vnn[3] = {reinterpret_cast<const void*>(&k_serve_vnn<0>),
