@@ -153,16 +153,18 @@ __device__ __forceinline__ double aziz_vmid(double kd, double y, const AzizDev& 
 
 // valueV of any bin kd >= 1 (an integer in FP64) from y, the reciprocal-root
 // estimate of |w| (kd <= |w| < kd + 1): aziz_vmix without the FP64 reciprocal,
-// which takes four issue slots.  1/kd^2 is y^2 and one Newton step, off by 4/kd^2:
-// under 4e-10 down to x = 0.1, below which the damping factor exp(-(D/x - 1)^2) <
-// e^-120 leaves nothing of the dispersion.  (512 walkers of N = 16 .. 256: 1.85 ->
-// 1.73 ms per batch, with the bin kept as an FP64 whole number.)
+// which takes four issue slots.  y^2 is off from 1/kd^2 by e = 2/kd + 2^-22 at most, and
+// a third-order step leaves e^3, below the 2^-46 of aziz_vmix down to x = 0.1 (1e-14);
+// nearer, the damping factor exp(-(D/x - 1)^2) < e^-80 leaves nothing of the dispersion.
+// (512 walkers of N = 16 .. 256: 1.85 -> 1.73 ms per batch with a Newton step, whose e^2
+// is 2e-12 at x = 2, and the bin kept as an FP64 whole number.)
 template <bool BETA0 = false>
 __device__ __forceinline__ double aziz_vmix_y(double kd, double y, const AzizDev& a, double k_d) {
     const double rep = split_exp2(BETA0 ? fma(a.rep_c1, kd, a.rep_c0) : fma(fma(a.rep_c2, kd, a.rep_c1), kd, a.rep_c0));
     const double q = kd * kd;
     const double r0 = y * y;
-    const double iq = fma(r0, fma(-q, r0, 1.0), r0);
+    const double e = fma(-q, r0, 1.0);
+    const double iq = fma(r0, fma(e, e, e), r0);
     const double disp = (iq * iq * iq) * fma(fma(a.eC10k, iq, a.eC8k), iq, a.eC6k);
     double v = rep - disp;
     if (kd < k_d) {

@@ -4,7 +4,12 @@ FP64 mode: V and dV/dr at the bin radius x = k s, whose reciprocals and exponent
 the kernels' own, are no further off than the reference's formulas in plain FP64 (IEEE
 quotients and square root, the library's exponential): rms over 20 000 to 50 000 bins of
 each range of x, within the 5 % that two such samples may differ by, over the sizes of the
-terms that make them up."""
+terms that make them up.
+
+Mixed mode: V of far pairs that share a wave with a pair of another kind takes the form
+with the damping test.  Beyond x = 3 the repulsion, whose exponential is FP32, is below
+1e-8 of the dispersion and its error below 1e-15; 1/k^2 is within 2^-46, so V is within
+3 2^-46 and some fifty roundings of the coefficients and the sum."""
 import numpy as np
 import pytest
 
@@ -106,3 +111,28 @@ def test_dv_fp64(gpu, year):
         got = _rms((np.sqrt(got.astype(LD) / 2) - want) / size)
         assert got <= 1.05 * plain, (lo, hi, got, plain)
 
+
+def test_v_mixed_far_beside_others(gpu):
+    p, M, L = YEARS[1979], 4000, 41.234
+    dr, half = _dr(p), 0.5 * L
+    assert 0.1 < (np.sqrt(0.75) * L / dr) % 1.0 < 0.9   # bead 2 is past the table from bead 0
+    s = dr / p["rm"]
+    k = np.random.default_rng(1).integers(int(3.0 / s), int(6.5 / s), 3 * M)
+    r01 = (k + 0.5) * dr
+    r12 = np.sqrt((half - r01) ** 2 + 2.0 * half ** 2)
+    w = r12 / dr
+    ok = (w % 1.0 > 0.1) & (w % 1.0 < 0.9)
+    r01, k01, k12 = r01[ok][:M], k[ok][:M], np.floor(w[ok][:M])
+    assert len(r01) == M
+    beads = np.zeros((M, 3, 3))
+    beads[:, 1, 0] = r01
+    beads[:, 2] = -half
+    ctx = gpu.Context(L, M, 3, 0.004, 6.0596, L)
+    ctx.upload_path(beads)
+    _, v = ctx.potentialAction(with_slices=True)
+    got = np.asarray(v).reshape(M, -1)[:, -1]
+    want = 0
+    for kk in (k01, k12):
+        rep, disp, F = _v_terms(kk.astype(LD) * LD(s), p, LD)
+        want = want + LD(p["eps"]) * (rep - disp * F)
+    assert np.abs((got - want) / want).max() <= 3 * 2.0 ** -46 + 50 * 2.0 ** -53
