@@ -441,8 +441,8 @@ static int ctx_dalloc(pimc_ctx* c, T** p, size_t n) {
     return PIMC_OK;
 }
 template <typename T>
-static int ctx_halloc(pimc_ctx* c, T** p, size_t n) {
-    hipError_t e = hipHostMalloc((void**)p, sizeof(T) * std::max<size_t>(n, 1), hipHostMallocDefault);
+static int ctx_halloc(pimc_ctx* c, T** p, size_t n, unsigned flags = hipHostMallocDefault) {
+    hipError_t e = hipHostMalloc((void**)p, sizeof(T) * std::max<size_t>(n, 1), flags);
     if (e != hipSuccess) return fail(c, PIMC_E_NOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
     c->host_allocs.push_back((void*)*p);
     return PIMC_OK;
@@ -817,7 +817,10 @@ static int ensure_req(pimc_ctx* c, int n) {
     int cap = std::max(64, n);
     int r;
     if ((r = ctx_dalloc(c, &c->d_req_beads, cap))) return r;
-    if ((r = ctx_halloc(c, &c->h_req_beads, cap))) return r;
+    // coherent: the direct form's kernels read a long list in place, as packets whose
+    // agent-scope acquire does not make host writes to cached memory visible
+    if ((r = ctx_halloc(c, &c->h_req_beads, cap, hipHostMallocMapped | hipHostMallocCoherent))) return r;
+    HIP_OR_FAIL(c, hipHostGetDevicePointer((void**)&c->m_req_beads, c->h_req_beads, 0));
     if ((r = ctx_dalloc(c, &c->d_req_sp, 2 * (size_t)cap))) return r;
     if ((r = ctx_dalloc(c, &c->d_req_pos, 3 * (size_t)cap))) return r;
     if ((r = ctx_halloc(c, &c->h_req_sp, 2 * (size_t)cap))) return r;
@@ -1476,7 +1479,7 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         if (inline_req)
             std::memcpy(req.beads, c->h_req_beads, sizeof(VnnBead) * n);
         else
-            A.beads = c->h_req_beads;   // pinned: read in place
+            A.beads = c->m_req_beads;   // mapped: read in place
         const KernelTimer kt = c->kernel_timer(1);
         // a packet on the device's AQL queue when the call is not timed (the
         // timing events live on the stream) and the context's stream is quiet:

@@ -156,7 +156,8 @@ struct pimc_ctx {
     // requests
     int cap_req = 0;
     pimc::VnnBead* d_req_beads = nullptr;
-    pimc::VnnBead* h_req_beads = nullptr;
+    pimc::VnnBead* h_req_beads = nullptr;   // mapped, coherent
+    pimc::VnnBead* m_req_beads = nullptr;   // its device address
     int* d_req_sp = nullptr;
     double* d_req_pos = nullptr;
     int* h_req_sp = nullptr;

@@ -45,3 +45,23 @@ def test_long_requests(gpu, mode, n, M, N, cells):
         assert np.array_equal(c.download_path(), ref.download_path())
         a, r = c.cell_lists(), ref.cell_lists()
         assert all(np.array_equal(a[k], r[k]) for k in ("grid", "bead_label", "num_labels"))
+
+
+def test_lists_rewritten_in_place(gpu):
+    """The list's block is written again for every request and read in place by the packet's
+    kernel: requests of changing lengths, beads and positions, one after another, are those
+    of a context that launches through HIP, bit for bit."""
+    rng = np.random.default_rng(8)
+    M, N = 512, 24
+    L = (N / 0.02198) ** (1.0 / 3.0)
+    b = rng.uniform(-0.5 * L, 0.5 * L, size=(M, N, 3))
+    a, h = (_context(gpu, L, M, N, 0.004, L, 0, b, packets=p) for p in (True, False))
+    for k in range(60):
+        n = int(rng.integers(33, M + 1))
+        sp = np.stack([rng.permutation(M)[:n], rng.integers(0, N, n)], axis=-1).astype(np.int32)
+        new = rng.uniform(-0.5 * L, 0.5 * L, size=(n, 3))
+        commit = k % 5 == 4
+        assert np.array_equal(a.delta_action(sp, new, commit=commit), h.delta_action(sp, new, commit=commit)), (k, n)
+    assert a.kernel_time("delta_packets")[1] == 60 - 1   # the first long request goes through HIP
+    assert h.kernel_time("delta_packets")[1] == 0
+    assert np.array_equal(a.download_path(), h.download_path())
