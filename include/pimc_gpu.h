@@ -458,9 +458,9 @@ int pimc_set_timing_kinds(pimc_ctx* ctx, unsigned kinds);
  * dispatch packets straight into the device's AQL queue (total_ms 0): requests
  * of up to 512 beads on slices of up to 1024 (32 with the gradient correction),
  * without per-bead outputs, while timing of "delta_action" (with the correction: of
- * any kernel) is off.  The environment
- * variable PIMC_DIRECT_DISPATCH=0, read when a context is created, sends them
- * through hipLaunchKernel instead.  "isf_chunks" counts the q of pimc_isf calls
+ * any kernel) is off.  "action_packets" counts the total actions sent so: untimed
+ * calls of up to 1.6e7 pairs.  The environment variable PIMC_DIRECT_DISPATCH=0,
+ * read when a context is created, sends both through hipLaunchKernel instead.  "isf_chunks" counts the q of pimc_isf calls
  * that took the piecewise form, in parts of 34 000 and at least two per call
  * (total_ms 0): lattice q only, at least 2048 of them, results of 4 MB and more
  * into page-locked memory (pimc_host_alloc), while timing of "rho" and "isf" is

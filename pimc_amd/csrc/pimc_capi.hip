@@ -8,7 +8,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -371,31 +370,19 @@ static hipError_t dalloc(T** p, size_t n) {
     return hipMalloc((void**)p, sizeof(T) * std::max<size_t>(n, 1));
 }
 
-bool pimc_ctx::direct_ready(int mode) {
-    if (direct_state < 0) {
-        direct_state = 0;
-        if (pimc::direct_ring_create(device, &dring)) {
-            // the kernels' entries in the loaded code object: looked up once per device
-            static std::mutex mu;
-            static std::map<int, std::array<pimc::DirectKernel, 6>> found;
-            std::lock_guard<std::mutex> lk(mu);
-            bool all = true;
-            if (found.count(device)) {
-                for (int k = 0; k < 6; ++k) dk_vdir[k] = found[device][k];
-            } else {
-                for (int k = 0; k < 6 && all; ++k)
-                    all = pimc::direct_kernel(device, pimc::vnn_direct_stub(k / 2, k % 2 != 0), stream,
-                                              pimc::kVdirBytes, &dk_vdir[k]);
-                if (all)
-                    for (int k = 0; k < 6; ++k) found[device][k] = dk_vdir[k];
-            }
-            if (all)
-                direct_state = 1;
-            else
-                pimc::direct_ring_release(&dring);
-        }
+bool pimc_ctx::ring_ready() {
+    if (direct_state < 0) direct_state = pimc::direct_ring_create(device, &dring) ? 1 : 0;
+    return direct_state == 1;
+}
+
+const pimc::DirectKernel* pimc_ctx::vdir_kernel(int mode, bool listed) {
+    if (mode < 0 || mode > 2 || !ring_ready()) return nullptr;
+    const int k = 2 * mode + (listed ? 1 : 0);
+    if (!asked_vdir[k]) {
+        asked_vdir[k] = true;
+        dk_vdir[k] = pimc::direct_kernel_of(device, pimc::vnn_direct_stub(mode, listed), stream, pimc::kVdirBytes);
     }
-    return direct_state == 1 && mode >= 0 && mode < 3 && dk_vdir[2 * mode].ok();
+    return dk_vdir[k];
 }
 
 // May the kernels of an action go as packets?  Untimed calls whose kernels take a few
@@ -408,7 +395,7 @@ bool pimc_ctx::packets_ready() {
     if (timing || 0.5 * N * N * desc.num_slices > kMostPairs) return false;
     const bool first = direct_state < 0 && !asked_packets;
     asked_packets = true;
-    return !first && direct_ready(desc.v_mode) && stream_quiet();
+    return !first && ring_ready() && stream_quiet();
 }
 
 bool pimc_ctx::stream_quiet() {
@@ -979,6 +966,7 @@ static int total_action(pimc_ctx* c, int shift, const double vfactor[2], double*
             PacketList list(&c->dring, c->stream);
             if ((r = launch(&list))) return r;
             packet = packet && list.send();
+            c->action_packets += packet;
         }
         if (!packet && (r = launch(nullptr))) return r;
         if (v_slices && !mapped) {
@@ -1488,15 +1476,16 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         // gain: a context's first long request goes through HIP.
         const bool first_long = !inline_req && c->direct_state < 0 && !c->asked_long;
         c->asked_long |= !inline_req;
-        const bool packet = !kt.start && !first_long && c->direct_ready(c->desc.v_mode) && c->stream_quiet();
+        const pimc::DirectKernel* kernel =
+            kt.start || first_long ? nullptr : c->vdir_kernel(c->desc.v_mode, !inline_req);
+        const bool packet = kernel && c->stream_quiet();
         if (packet) {
             VnnDirectOut* outp = c->d_vdir;
             const pimc::ArgPiece pieces[4] = {{&A, 0, (uint32_t)sizeof(VnnArgs)},
                                               {req.beads, pimc::kVdirOffReq, inline_req ? (uint32_t)(sizeof(VnnBead) * n) : 0u},
                                               {&az, pimc::kVdirOffAz, (uint32_t)sizeof(AzizDev)},
                                               {&outp, pimc::kVdirOffOut, (uint32_t)sizeof(outp)}};
-            pimc::direct_dispatch(&c->dring, c->dk_vdir[2 * c->desc.v_mode + (inline_req ? 0 : 1)], pieces, 4, (uint32_t)n,
-                                  (uint32_t)kVnnDirectThreads);
+            pimc::direct_dispatch(&c->dring, *kernel, pieces, 4, (uint32_t)n, (uint32_t)kVnnDirectThreads);
             ++c->direct_count;
         } else {
             HIP_OR_FAIL(c, launch_vnn_direct(c->desc.v_mode, c->stream, A, req, az, c->d_vdir, &kt));
@@ -1521,7 +1510,7 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         std::memcpy(req.beads, c->h_req_beads, sizeof(VnnBead) * n);
         // a short request with the correction: both kernels as packets (N = 256:
         // 21.6 us, 23.0 through HIP; N = 16: 16.1 and 18.4)
-        if (cor && A.chunks == 1 && !per_bead && !cor_out && out3 && !c->timing && c->direct_ready(c->desc.v_mode) &&
+        if (cor && A.chunks == 1 && !per_bead && !cor_out && out3 && !c->timing && c->ring_ready() &&
             c->stream_quiet()) {
             PacketList list(&c->dring, c->stream);
             list.long_arg_bytes = (uint32_t)(sizeof(VnnBead) * n);
@@ -1796,6 +1785,11 @@ int pimc_kernel_time(pimc_ctx* c, const char* name, double* total_ms, long* coun
     if (std::strcmp(name, "delta_packets") == 0) {
         if (total_ms) *total_ms = 0.0;
         if (count) *count = c->direct_count;
+        return PIMC_OK;
+    }
+    if (std::strcmp(name, "action_packets") == 0) {
+        if (total_ms) *total_ms = 0.0;
+        if (count) *count = c->action_packets;
         return PIMC_OK;
     }
     if (std::strcmp(name, "isf_chunks") == 0) {

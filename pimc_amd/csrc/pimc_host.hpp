@@ -117,12 +117,15 @@ struct pimc_ctx {
     // kernel-argument ring and k_vnn_direct per mode; direct_state -1: not set
     // up yet, 0: launched through HIP, 1: packets)
     pimc::DirectRing dring;
-    pimc::DirectKernel dk_vdir[6];   // [2 mode + listed]
+    const pimc::DirectKernel* dk_vdir[6] = {};   // [2 mode + listed], looked up when first asked for
+    bool asked_vdir[6] = {};
     int direct_state = -1;
     bool asked_long = false;   // a request of more than kVnnInline beads has been made
     long direct_count = 0;   // requests dispatched as packets
-    bool direct_ready(int mode);
+    bool ring_ready();
+    const pimc::DirectKernel* vdir_kernel(int mode, bool listed);   // null: not as a packet
     bool asked_packets = false;   // an action could have gone as packets
+    long action_packets = 0;      // actions that did
     bool packets_ready();
     // Every entry point returns only after its work on the stream has finished
     // or its last kernel has published its result (nothing of that kernel is

@@ -1,7 +1,8 @@
 """Actions, energies and Delta V with the gradient correction as packets on the device
 queue against the same kernels launched through HIP: bit for bit, in every mode, for
 repeated calls between moves, with links given and changed, and from two threads whose
-contexts share the queue."""
+contexts share the queue.  The counts of requests and actions sent show that the packets
+are what ran: a kernel the queue refuses would go through HIP with the same values."""
 import threading
 
 import numpy as np
@@ -43,15 +44,21 @@ def _walk(gpu, packets, mode, M, N, correction, seed):
         links = (None, nxt, swap)[k % 3]
         out.append(np.asarray(list(ctx.energy(next_links=links).values())))
         out.append(np.asarray(list(ctx.virial_energy(3, next_links=links).values())))
-    return out, ctx.download_path()
+    sent = [ctx.kernel_time(k)[1] for k in ("delta_packets", "action_packets")]
+    return out, ctx.download_path(), sent
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("M,N,correction", [(40, 64, True), (41, 65, False), (20, 300, True), (6, 1, True)])
 def test_packets_equal_launches(gpu, mode, M, N, correction):
-    a, pa = _walk(gpu, True, mode, M, N, correction, M)
-    b, pb = _walk(gpu, False, mode, M, N, correction, M)
+    a, pa, sent = _walk(gpu, True, mode, M, N, correction, M)
+    b, pb, none = _walk(gpu, False, mode, M, N, correction, M)
     assert np.array_equal(pa, pb)
+    # every request is one; an action is one where the walker's factors are on the device
+    # already (energy and virial_energy ask for unit factors in between), and with one bead
+    # a slice there is nothing to launch
+    assert sent == [6, 0 if N == 1 else 6 if correction else 11]
+    assert none == [0, 0]
     for k, (x, y) in enumerate(zip(a, b)):
         assert np.array_equal(x, y, equal_nan=True), k
 
