@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <optional>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -385,10 +386,10 @@ const pimc::DirectKernel* pimc_ctx::vdir_kernel(int mode, bool listed) {
     return dk_vdir[k];
 }
 
-// May the kernels of an action go as packets?  Untimed calls whose kernels take a few
-// tens of microseconds (a packet holds up the device queue's later ones, other
-// contexts' too).  A context's first such call goes through HIP: setting the ring up
-// costs more than one call gains.
+// May the kernels of an action go as packets (given a turn on the queue)?  Untimed calls
+// of up to a few hundred microseconds: one that a brief call of another context has just
+// missed holds that one up.  A context's first such call goes through HIP: setting the
+// ring up costs more than one call gains.
 bool pimc_ctx::packets_ready() {
     constexpr double kMostPairs = 1.6e7;
     const double N = desc.num_alloc;
@@ -950,6 +951,8 @@ static int total_action(pimc_ctx* c, int shift, const double vfactor[2], double*
         // too, and nothing waits for the stream's queue to wake (three requests and an
         // action at N = 256, M = 167: 55.5 -> 54.1 us; an action alone gains 0.2 us).
         bool packet = !on_stream && !spatial && (mapped || !v_slices) && c->packets_ready();
+        std::optional<QueueTurn> turn;   // until the result is there
+        if (packet) packet = (bool)turn.emplace(c->device, true);
         auto launch = [&](PacketList* list) -> int {
             bool chunked = true;
             if (cor && (r = run_gradv2(c, az, need, list, &chunked))) return r;
@@ -1478,7 +1481,8 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         c->asked_long |= !inline_req;
         const pimc::DirectKernel* kernel =
             kt.start || first_long ? nullptr : c->vdir_kernel(c->desc.v_mode, !inline_req);
-        const bool packet = kernel && c->stream_quiet();
+        std::optional<QueueTurn> turn;   // until the results are there
+        const bool packet = kernel && c->stream_quiet() && turn.emplace(c->device, !inline_req);
         if (packet) {
             VnnDirectOut* outp = c->d_vdir;
             const pimc::ArgPiece pieces[4] = {{&A, 0, (uint32_t)sizeof(VnnArgs)},
@@ -1510,8 +1514,9 @@ static int run_vnn(pimc_ctx* c, int n, int shift, const double vf[2], bool commi
         std::memcpy(req.beads, c->h_req_beads, sizeof(VnnBead) * n);
         // a short request with the correction: both kernels as packets (N = 256:
         // 21.6 us, 23.0 through HIP; N = 16: 16.1 and 18.4)
+        std::optional<QueueTurn> turn;
         if (cor && A.chunks == 1 && !per_bead && !cor_out && out3 && !c->timing && c->ring_ready() &&
-            c->stream_quiet()) {
+            c->stream_quiet() && turn.emplace(c->device, true)) {
             PacketList list(&c->dring, c->stream);
             list.long_arg_bytes = (uint32_t)(sizeof(VnnBead) * n);
             HIP_OR_FAIL(c, launch_vnn(c->desc.v_mode, c->stream, A, req, az, nullptr, c->d_gnn_part, gnn_lds, nullptr,

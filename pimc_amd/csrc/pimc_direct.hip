@@ -20,6 +20,7 @@
 #include <limits.h>
 #include <stdlib.h>
 
+#include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -39,6 +40,7 @@ struct DeviceQueue {
     volatile uint32_t* hdp = nullptr;
     hsa_signal_t drain{};
     std::mutex m;   // packet slots, doorbell and the drain signal
+    std::atomic<int> brief{0}, lengthy{0};   // calls on the queue (QueueTurn)
 };
 
 std::mutex g_init;
@@ -439,6 +441,29 @@ const DirectKernel* direct_kernel_of(int device, const void* host_stub, hipStrea
         it = known.emplace(std::make_pair(device, host_stub), k).first;
     }
     return it->second.ok() ? &it->second : nullptr;
+}
+
+QueueTurn::QueueTurn(int dev, bool long_call) : device(dev), lengthy(long_call), taken(false) {
+    DeviceQueue& D = g_dev[device];
+    // each side announces itself before it looks for the other
+    if (lengthy) {
+        if (D.lengthy.exchange(1)) return;
+        taken = D.brief.load() == 0;
+        if (!taken) D.lengthy.store(0);
+    } else {
+        D.brief.fetch_add(1);
+        taken = D.lengthy.load() == 0;
+        if (!taken) D.brief.fetch_sub(1);
+    }
+}
+
+QueueTurn::~QueueTurn() {
+    if (!taken) return;
+    DeviceQueue& D = g_dev[device];
+    if (lengthy)
+        D.lengthy.store(0);
+    else
+        D.brief.fetch_sub(1);
 }
 
 void PacketList::add_blob(const void* stub, dim3 g, dim3 b, size_t lds, const char* blob, uint32_t bytes) {

@@ -80,6 +80,26 @@ void direct_submit(DirectRing* r, const DirectKernel& k, const char* kernargs, u
 // loaded code object stays); null when the function cannot be dispatched.
 const DirectKernel* direct_kernel_of(int device, const void* host_stub, hipStream_t stream, uint32_t bytes);
 
+// A call's turn on the device's queue, which all contexts share and whose packets run one
+// after another: a lengthy call (an action, a corrected or a long Delta V request) takes
+// it only while no other call is on it, a brief one while no lengthy call is.  A call
+// that gets no turn launches on its context's stream, beside the others, so no context
+// waits behind another's kernels.  Actions of N = 256 x 167 from one, two and four threads
+// with a context each, us per action: 23.7, 13.7 and 11.5; every action on the queue 23.7,
+// 18.8 and 18.8; every action on its stream 25.1, 14.2 and 15.5.
+class QueueTurn {
+public:
+    QueueTurn(int device, bool lengthy);
+    ~QueueTurn();
+    QueueTurn(const QueueTurn&) = delete;
+    QueueTurn& operator=(const QueueTurn&) = delete;
+    explicit operator bool() const { return taken; }
+
+private:
+    int device;
+    bool lengthy, taken;
+};
+
 // The kernels of one call, in order, as packets behind one flush on the device's
 // queue.  (A packet without the barrier bit, to run beside the one before it, gained
 // nothing: the first kernel's workgroups are all dispatched before it.)  send() queues nothing and returns false when a kernel cannot

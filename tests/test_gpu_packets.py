@@ -72,3 +72,38 @@ def test_two_threads(gpu):
     for s in (1, 2):
         assert np.array_equal(got[s][1], want[s][1])
         assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(got[s][0], want[s][0]))
+
+
+def _mixed_calls(gpu, packets, M, N, correction, seed):
+    """Actions between short and long requests, one in three of them committed."""
+    L = (N / 0.02198) ** (1.0 / 3.0)
+    rng = np.random.default_rng(seed)
+    b = rng.uniform(-0.5 * L, 0.5 * L, size=(M, N, 3))
+    ctx = _context(gpu, L, M, N, 0.004, L, 0, b, packets=packets)
+    if correction:
+        ctx.set_action_factors(*GSF)
+    out = []
+    for k in range(40):
+        n = (5, 31, min(M, 90))[k % 3]
+        sp = np.stack([rng.permutation(M)[:n], rng.integers(0, N, n)], axis=-1).astype(np.int32)
+        new = rng.uniform(-0.5 * L, 0.5 * L, size=(n, 3))
+        out += [np.asarray(ctx.potentialAction()), np.array(ctx.delta_action(sp, new, commit=k % 3 == 1))]
+    return out, ctx.download_path(), [ctx.kernel_time(k)[1] for k in ("delta_packets", "action_packets")]
+
+
+def test_turns_of_four_threads(gpu):
+    """Contexts of four threads take turns on the queue and launch on their streams when
+    they get none: the values are those of one context alone."""
+    cases = {0: (40, 64, True), 1: (125, 16, False), 2: (100, 200, False), 3: (60, 33, True)}
+    want = {s: _mixed_calls(gpu, False, *c, s) for s, c in cases.items()}
+    alone = _mixed_calls(gpu, True, *cases[1], 1)
+    assert alone[2] == [40, 39]   # the first action comes before there is a ring
+    got = {}
+    ts = [threading.Thread(target=lambda s=s, c=c: got.update({s: _mixed_calls(gpu, True, *c, s)}))
+          for s, c in cases.items()]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for s in cases:
+        assert np.array_equal(got[s][1], want[s][1])
+        assert all(np.array_equal(x, y) for x, y in zip(got[s][0], want[s][0])), s
+    assert sum(g[2][0] for g in got.values()) > 0
