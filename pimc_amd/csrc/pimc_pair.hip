@@ -54,8 +54,8 @@ __device__ __forceinline__ double sep_bins_mixed(const RowMixed& q, double xj, d
     const double wy = fma(__builtin_amdgcn_fract(fma(yj, q.invL, q.cy)), q.S, q.Sh);
     const double wz = fma(__builtin_amdgcn_fract(fma(zj, q.invL, q.cz)), q.S, q.Sh);
     const double r2 = fma(wz, wz, fma(wy, wy, wx * wx));
-    // |w|: the hardware FP64 reciprocal-root estimate (relative error ~2^-23)
-    // and one Newton step, |w| = r0 + (r2 - r0^2) y / 2 (~2^-46)
+    // |w|: the hardware FP64 reciprocal-root estimate (relative error e <= 2^-23)
+    // and one Newton step, |w| = r0 + (r2 - r0^2) y / 2 (1.5 e^2)
     const double y = __builtin_amdgcn_rsq(r2);
     *y_out = y;
     const double r0 = r2 * y;
@@ -124,14 +124,19 @@ __device__ __forceinline__ double pair_term_mixed(const RowMixed& q, double x, d
 }
 
 // One pair term of the exact modes (FP64 closed form, table), the bin the host's bit
-// for bit.  The mixed mode's |w| is within ~1e-6 bin of |r|/dr (2e-9 from the
-// separation, the rest from the root after one Newton step, below 2^-40 relative at
-// up to 1.5e7 bins), so away from a whole number by kBinGuard its floor is the
-// host's int(sqrt(r2)/dr); a lane nearer than that (2 in 10 000) has its bin
-// evaluated as the host does, with the reference's minimum image, IEEE root and
+// for bit.  With beads in the box the mixed mode's |w| is off from |r|/dr by
+//   1.5 e^2 |w|, e <= 2^-23 the error of the root estimate (5.3e-8 at most over 2e9
+//   arguments) and 1.5 e^2 what one Newton step leaves of it, and by
+//   4 sqrt(3) 2^-53 S, four roundings of a few box units per axis,
+// under kBinGuard whatever the box, since a bin is an int.  So away from a whole number by
+// kBinGuard its floor is the host's int(sqrt(r2)/dr); a lane nearer than that (2 in 10 000)
+// has its bin evaluated as the host does, with the reference's minimum image, IEEE root and
 // division, which would cost ~35 instructions on every pair (full action in FP64,
 // N = 777 x 61: 179 -> 155 us with the quotients of aziz_v64 as well).
 constexpr double kBinGuard = 1.0e-4;
+constexpr double kMostBins = 0x1p31;   // |w| <= sqrt(3)/2 S
+static_assert(1.5 * 0x1p-46 * kMostBins + 4.0 * 1.7321 * 0x1p-53 * (kMostBins / 0.866) < kBinGuard,
+              "the guard covers the longest table");
 template <int MODE>
 __device__ __forceinline__ double pair_term_exact(const RowMixed& q, double xi, double yi, double zi, double x,
                                                   double y, double z, const BoxDev& box, const AzizDev& a) {

@@ -57,3 +57,30 @@ def test_coincident_and_half_box(orc, gpu, mode, N):
     b[2, 1] = b[2, 0] - np.sign(b[2, 0]) * np.array([0.5 * L, 0.5 * L, 0])
     b[3, 0], b[3, 1] = -0.5 * L, 0.0      # |r| = maxSep, past the table
     _compare(orc, gpu, b, L, mode)
+
+
+@pytest.mark.parametrize("L", [100.0, 700.0, 7000.0])
+def test_bins_of_large_boxes(gpu, L):
+    """Up to 2e9 bins, the most an int holds: |r| = (k + e) dr at half the longest separations,
+    e around 0.  V ~ k^-6, so one bin off moves it by 6/k of itself, 3e-9 and more."""
+    dr, s = 1.0e-6 * RM, 1.0e-6 * RM / RM
+    rng = np.random.default_rng(int(L))
+    M = 3000
+    k = rng.integers(int(0.3 * L / dr), int(0.49 * np.sqrt(3.0) * L / dr), M)
+    e = rng.choice([-1.5e-4, -9e-5, -5e-5, -1e-5, -1e-6, 0.0, 1e-6, 1e-5, 5e-5, 9e-5, 1.5e-4], M)
+    u = rng.uniform(0.9, 1.0, size=(M, 3))
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    b = np.zeros((M, 2, 3))
+    b[:, 0] = -0.25 * L
+    b[:, 1] = b[:, 0] + (k + e)[:, None] * dr * u
+    # the reference's bin: separation, minimum image, norm, root and quotient in its order
+    d = b[:, 1] - b[:, 0]
+    d = d - L * np.floor(d * (1.0 / L) + 0.5)
+    bins = (np.sqrt((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2]) / dr).astype(np.int64)
+    assert bins.max() < 2 ** 31 and len(set(bins - k)) > 1
+    ctx = gpu.Context(L, M, 2, 0.004, 6.0596, L, v_mode=1)
+    ctx.upload_path(b)
+    v = ctx.potential_slices()[:, 1]
+    x2 = (bins * s) ** -2.0
+    want = -10.8 * (1.3732412 * x2 ** 3 + 0.4253785 * x2 ** 4 + 0.1781 * x2 ** 5)
+    assert (np.abs(v / want - 1.0) < 2.0 / bins).all()
