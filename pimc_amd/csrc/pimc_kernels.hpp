@@ -273,6 +273,7 @@ hipError_t launch_gradv2(int mode, hipStream_t st, const double* pos, int64_t pl
                          int* blocks_per_slice, int chunks = 1, double* fpart = nullptr, int need = 3,
                          PacketList* packets = nullptr);
 // Partner chunks of the gradVSquared sum that fill the CUs (1: one pass).
+constexpr int kGradChunks = 16;
 int gradv2_chunks(int nalloc, int num_slices, int num_cus);
 // Device-resident chain (pimc_dchain.hip): one workgroup runs n_moves moves.
 constexpr int kChainThreads = 768;      // 12 waves: three per SIMD

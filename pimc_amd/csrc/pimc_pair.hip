@@ -1061,6 +1061,10 @@ __global__ __launch_bounds__(256) void k_gradv2_sym(const double* __restrict__ p
     }
 }
 
+// The chunks' partials of each row in chunk order, four chunks' loads in flight: a slice
+// in two being corrected, small systems get up to sixteen chunks, and one chunk at a time
+// their loads were most of the kernel (GSF action of N = 16 x 125 24.1 -> 21.7 us, 64 x 96
+// 26.3 -> 23.6, 256 x 167 44.9 -> 43.7; all sixteen at once, behind a test each, 27.6).
 __global__ __launch_bounds__(256) void k_gradv2_sum(const int* __restrict__ nbs, int nalloc, int C, int need,
                                                     const double* __restrict__ fpart, double* __restrict__ part) {
     __shared__ double red[4];
@@ -1068,9 +1072,24 @@ __global__ __launch_bounds__(256) void k_gradv2_sum(const int* __restrict__ nbs,
     const int i = b * 256 + threadIdx.x;
     double f2 = 0.0;
     if (i < nbs[m] && ((need >> (m & 1)) & 1)) {
+        const double* o = fpart + ((int64_t)m * C * nalloc + i) * 3;
+        const int64_t step = (int64_t)nalloc * 3;
         double fx = 0.0, fy = 0.0, fz = 0.0;
-        for (int c = 0; c < C; ++c) {
-            const double* o = fpart + (((int64_t)m * C + c) * nalloc + i) * 3;
+        int c = 0;
+        for (; c + 4 <= C; c += 4, o += 4 * step) {
+            double f[4][3];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) f[u][q] = o[u * step + q];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                fx += f[u][0];
+                fy += f[u][1];
+                fz += f[u][2];
+            }
+        }
+        for (; c < C; ++c, o += step) {
             fx += o[0];
             fy += o[1];
             fz += o[2];
@@ -1086,7 +1105,7 @@ int gradv2_chunks(int nalloc, int num_slices, int num_cus) {
     const int64_t blocks = (int64_t)B * num_slices;
     const int64_t want = 4LL * std::max(1, num_cus);
     if (blocks >= want) return 1;
-    return (int)std::min<int64_t>(16, (want + blocks - 1) / blocks);
+    return (int)std::min<int64_t>(kGradChunks, (want + blocks - 1) / blocks);
 }
 
 __device__ __forceinline__ double group16_sum(double v) {
