@@ -460,12 +460,15 @@ int pimc_set_timing_kinds(pimc_ctx* ctx, unsigned kinds);
  * without per-bead outputs, while timing of "delta_action" (with the correction: of
  * any kernel) is off.  "action_packets" counts the total actions sent so: untimed
  * calls of up to 1.6e7 pairs.  The environment variable PIMC_DIRECT_DISPATCH=0,
- * read when a context is created, sends both through hipLaunchKernel instead.  "isf_chunks" counts the q of pimc_isf calls
- * that took the piecewise form, in parts of 34 000 and at least two per call
- * (total_ms 0): lattice q only, at least 2048 of them, results of 4 MB and more
- * into page-locked memory (pimc_host_alloc), while timing of "rho" and "isf" is
- * off; each piece computes its density modes and lags while the DMA engines copy
- * the previous piece's rows out, with the same values as one launch per kernel. */
+ * read when a context is created, sends both through hipLaunchKernel instead.  "isf_chunks" counts the pieces of pimc_isf
+ * calls that took the piecewise form (total_ms 0): lattice q only, at least 2048
+ * of them, results of 4 MB and more into page-locked memory (pimc_host_alloc),
+ * while timing of "rho" and "isf" is off.  A piece computes its density modes and
+ * lags while the DMA engines copy the previous piece's rows out, with the same
+ * values as one launch per kernel; a list of up to some 5000 q is one piece.
+ * "isf_dma" counts the pieces whose rows left so: those of a list whose order keeps
+ * the pieces' rows together (the reference's does); the rows of any other list are
+ * copied at the end. */
 int pimc_kernel_time(pimc_ctx* ctx, const char* name, double* total_ms, long* count);
 int pimc_device_synchronize(void);
 /* Page-locked host memory for large results (no counterpart in the reference,

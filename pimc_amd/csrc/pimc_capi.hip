@@ -1802,6 +1802,11 @@ int pimc_kernel_time(pimc_ctx* c, const char* name, double* total_ms, long* coun
         if (count) *count = c->isf_chunks;
         return PIMC_OK;
     }
+    if (std::strcmp(name, "isf_dma") == 0) {
+        if (total_ms) *total_ms = 0.0;
+        if (count) *count = c->isf_dma;
+        return PIMC_OK;
+    }
     for (int k = 0; k < pimc_ctx::kKinds; ++k)
         if (std::strcmp(name, kKernelNames[k]) == 0) {
             if (total_ms) *total_ms = c->kernel_ms[k];

@@ -174,9 +174,9 @@ int general_rho(pimc_ctx* c, const std::vector<double>& qv, int nq) {
 }
 
 // F(q, tau) of a long lattice q list written straight into page-locked memory:
-// the modes run in pieces of row tiles, each piece's modes and lags on the
-// context's stream, and the list rows it completes are copied out while the next
-// piece computes.  A mode's sums do not depend on what
+// the modes run in pieces of row tiles (a list of up to 16 jobs in one), each
+// piece's modes and lags on the context's stream, and the list rows it completes
+// are copied out while the next piece computes.  A mode's sums do not depend on what
 // shares its launch, so the values are those of the one-launch path bit for bit.
 // 100 401 q x 250 lags are 200 MB, 3.5 ms at the 57 GB/s the link gives, beside
 // 2.8 ms of kernels; S(q) and F of that list took 39.6 ms together and now take
@@ -195,10 +195,6 @@ bool isf_pieces_pay(pimc_ctx* c, int n, int M, const double* fqt) {
     (void)hipGetLastError();   // a pageable pointer may report an error here
     return e == hipSuccess && at.type == hipMemoryTypeHost;
 }
-
-// What pimc_kernel_time counts as "isf_chunks": the q of such a call in parts of
-// 34 000, at least two.
-int isf_parts(int n) { return std::max(2, (n + 33999) / 34000); }
 
 // The list rows of modes [u0, u_end) as at most two runs {first row, rows}: their
 // first q and their second q (those of -q), each a run when the rows named are
@@ -276,7 +272,8 @@ int isf_lattice_pieces(pimc_ctx* c, const RhoPlan& P, const std::vector<int>& n3
     const hipError_t e1 = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = e1;
     if (e != hipSuccess) return sfail(c, PIMC_E_HIP, std::string("F(q,tau) in pieces: ") + hipGetErrorString(e));
-    c->isf_chunks += isf_parts(n);
+    c->isf_chunks += pieces;
+    if (moved) c->isf_dma += pieces;
     return PIMC_OK;
 }
 
@@ -366,8 +363,10 @@ int lattice_qs(const double* q, int nq, double L, std::vector<int>& n3, std::vec
 // stages, shorter in the matrix form (one block, 14 modes: 17.7 against 19.4 us).
 constexpr int kModesPerBlock = 72, kFewBlocks = 4;
 
-// Jobs of a launch that fill the workgroups of one round: 16 waves each, one
-// workgroup per slice (k_rho_matrix), and most chips' worth of slices.
+// Jobs of a piece: those of one workgroup of k_rho_matrix per slice, which at M = 250 is
+// one round of the 256 CUs.  With fewer slices a piece leaves CUs idle, which its copy
+// hides where the list is long: 42 499 q at N = 2048 take 1.42 ms at M = 40, 1.56 at 96
+// and 1.96 at 167, of which the link takes 0.24, 0.57 and 1.00.
 constexpr int kPieceJobs = 16;
 
 void make_rho_plan(const int* n3, int nq, int max_pieces, RhoPlan* P) {

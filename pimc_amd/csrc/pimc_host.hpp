@@ -53,7 +53,7 @@ struct RhoPlan {
     std::vector<int> mode_at, row_at, row_mode, row_cols, mode_row, mode_nz, order, at;
     std::vector<int2> list_rows;
 };
-// max_pieces: 1 for one launch; more: as many as fill the chip, at most that many
+// max_pieces: 1 for one launch; more: pieces of 16 jobs and more, at most that many
 void make_rho_plan(const int* n3, int nq, int max_pieces, RhoPlan* P);
 
 struct TableCache;
@@ -205,10 +205,11 @@ struct pimc_ctx {
     int* d_plan = nullptr;             // the plan on the device
     size_t cap_plan = 0;
     // F(q,tau) of long lattice q lists into page-locked memory: the DMA engines
-    // copy each chunk's rows out while the next chunk computes
+    // copy each piece's rows out while the next piece computes
     pimc::DmaCopies dma;
     std::vector<hipEvent_t> chunk_ev;
-    long isf_chunks = 0;               // chunks computed that way (pimc_kernel_time "isf_chunks")
+    long isf_chunks = 0;               // pieces computed that way (pimc_kernel_time "isf_chunks")
+    long isf_dma = 0;                  // those whose rows the DMA engines copied ("isf_dma")
     // staging
     double* h_stage = nullptr;    // cap_stage >= 3*M*N doubles, pinned
     size_t cap_stage = 0;

@@ -108,7 +108,9 @@ def test_pieces_into_pinned(gpu, kind):
     out = gpu.pinned_empty((len(k), M))
     out[:] = -1.0
     ctx.isf(q, out=out)
+    # a list whose order scatters the pieces' rows is copied at the end
     assert ctx.kernel_time("isf_chunks")[1] == 2
+    assert ctx.kernel_time("isf_dma")[1] == (0 if kind == "shuffled" else 2)
     assert np.array_equal(out, ctx.isf(q))
     ref = isf_from_rho(lattice_rho(b, n[k][::97], L), N)
     assert np.abs(out[::97] - ref).max() <= BOUND * M * N

@@ -46,20 +46,21 @@ def _case(orc, N, M, kind, qmax):
     f_gpu = ctx.isf(q)
     extra = {}
     if N == 256:
-        # 7.2 MB into page-locked memory: two halves, each copied out while the
-        # other computes
+        # 7.2 MB into page-locked memory: the piecewise form, one piece
         f_pin = pimc_amd.pinned_empty((q.shape[0], M))
         ctx.isf(q, out=f_pin)
         extra["chunks"] = ctx.kernel_time("isf_chunks")[1]
+        extra["dma"] = ctx.kernel_time("isf_dma")[1]
         extra["f_pin"] = [np.array(f_pin)]
     if N == 2048:
-        # into page-locked memory: the chunked form (modes and lags per chunk of
-        # q, each chunk's rows copied out while the next computes), twice in a
-        # row; then with the rho kernel timed, which keeps one launch per kernel
+        # into page-locked memory: the piecewise form (modes and lags per piece,
+        # each piece's rows copied out while the next computes), twice in a row;
+        # then with the rho kernel timed, which keeps one launch per kernel
         f_pin = [pimc_amd.pinned_empty((q.shape[0], M)) for _ in range(3)]
         ctx.isf(q, out=f_pin[0])
         ctx.isf(q, out=f_pin[1])
         extra["chunks"] = ctx.kernel_time("isf_chunks")[1]
+        extra["dma"] = ctx.kernel_time("isf_dma")[1]
         ctx.set_timing(True, kinds=["rho"])
         ctx.isf(q, out=f_pin[2])
         ctx.set_timing(False)
@@ -112,10 +113,10 @@ def test_isf_n256_m167_all_q_all_lags(walker):
     _check_values(walker)
 
 
-def test_isf_n256_m167_halves_into_pinned(walker):
-    """F(q,tau) of the 5377 q into page-locked memory runs as two halves of the
-    q list: bit-identical to the one-launch result."""
-    assert walker["chunks"] == 2
+def test_isf_n256_m167_into_pinned(walker):
+    """F(q,tau) of the 5377 q into page-locked memory (187 rows of q, 12 jobs) is one
+    piece, copied by the DMA engines: bit-identical to the pageable result."""
+    assert walker["chunks"] == 1 and walker["dma"] == 1
     assert np.array_equal(walker["f_pin"][0], walker["f_gpu"])
 
 
@@ -142,10 +143,11 @@ def test_ssf_n2048_m250_oracle_pair_sum(orc, large):
 
 
 def test_isf_n2048_m250_chunked_into_pinned(large):
-    """F(q,tau) of the 100 401 q into page-locked memory takes the chunked form
-    (3 chunks of at most 34 000 q, the last one ragged): bit-identical to the one-launch
-    result, on two calls in a row, and not taken while the rho kernel is timed."""
-    assert large["chunks"] == 2 * 3
+    """F(q,tau) of the 100 401 q into page-locked memory takes the piecewise form
+    (139 jobs, nine pieces), every piece's rows copied by the DMA engines: bit-identical to
+    the one-launch result, on two calls in a row, and not taken while the rho kernel is
+    timed."""
+    assert large["chunks"] == 2 * 9 and large["dma"] == 2 * 9
     assert large["chunks_timed"] == 0
     for f in large["f_pin"]:
         assert np.array_equal(f, large["f_gpu"])
