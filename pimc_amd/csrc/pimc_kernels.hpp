@@ -332,6 +332,8 @@ hipError_t launch_rho_matrix(hipStream_t st, const RhoMatrixArgs& A);
 // fqt (-1: none), or to row u without dst.
 hipError_t launch_isf(hipStream_t st, const double* rho, int nu, int u0, int u_end, int M, double inv_n,
                       const int* dst, double* fqt);
+// Rows {row, row it repeats} of fqt.
+hipError_t launch_isf_repeat(hipStream_t st, const int2* rep, int n, int M, double* fqt);
 // S of nq modes; done (or null): published with seq once sq (mapped) is written,
 // ticket a zeroed counter.
 hipError_t launch_ssf(hipStream_t st, const double* rho, int nq, int M, double inv_n, double* sq,

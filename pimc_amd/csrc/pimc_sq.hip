@@ -443,6 +443,14 @@ __global__ __launch_bounds__(256) void k_isf_from_rho(const double* __restrict__
     }
 }
 
+// Rows of q that a list names again: one workgroup each.
+__global__ __launch_bounds__(128) void k_isf_repeat(const int2* __restrict__ rep, int M, double* __restrict__ fqt) {
+    const int2 r = rep[blockIdx.x];
+    const double* from = fqt + (int64_t)r.y * M;
+    double* to = fqt + (int64_t)r.x * M;
+    for (int t = threadIdx.x; t < M; t += 128) to[t] = from[t];
+}
+
 // S(q) contribution = sum_m |rho_q(m)|^2 / N.  A workgroup takes 32 q (32
 // consecutive entries of rho, coalesced) with 8 lanes each: lane g adds the
 // slices [g seg, (g + 1) seg), seg = ceil(M / 8), in order, eight loads in flight,
@@ -614,6 +622,13 @@ hipError_t launch_isf(hipStream_t st, const double* rho, int nu, int u0, int u_e
         attr_set.store(true, std::memory_order_release);
     }
     hipLaunchKernelGGL(k_isf_from_rho, g, b, lds, st, rho, nu, u0, u_end, M, inv_n, dst, fqt);
+    return hipGetLastError();
+}
+
+hipError_t launch_isf_repeat(hipStream_t st, const int2* rep, int n, int M, double* fqt) {
+    (void)hipGetLastError();
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_isf_repeat, dim3(n), dim3(128), 0, st, rep, M, fqt);
     return hipGetLastError();
 }
 

@@ -94,7 +94,7 @@ def test_list_orders(gpu, kind):
     assert np.array_equal(ctx.isf(_q(n[k], L)), f[k])
 
 
-@pytest.mark.parametrize("kind", ["list", "shuffled", "repeated"])
+@pytest.mark.parametrize("kind", ["list", "shuffled", "repeated", "repeated often"])
 def test_pieces_into_pinned(gpu, kind):
     """F into page-locked memory (more than 4 MB) in several pieces: rows copied as they
     complete, whatever the list's order; the values of the pageable result."""
@@ -103,14 +103,15 @@ def test_pieces_into_pinned(gpu, kind):
     n = _box(11, 11, 11)
     rng = np.random.default_rng(3)
     k = {"list": np.arange(len(n)), "shuffled": rng.permutation(len(n)),
-         "repeated": np.concatenate([np.arange(len(n)), [5, 5, 700]])}[kind]
+         "repeated": np.concatenate([np.arange(len(n)), [5, 5, 700]]),       # copied by the host
+         "repeated often": np.concatenate([np.arange(len(n)), rng.integers(0, len(n), 900)])}[kind]   # by the device
     q = _q(n[k], L)
     out = gpu.pinned_empty((len(k), M))
     out[:] = -1.0
     ctx.isf(q, out=out)
     # a list whose order scatters the pieces' rows is copied at the end
     assert ctx.kernel_time("isf_chunks")[1] == 2
-    assert ctx.kernel_time("isf_dma")[1] == (0 if kind == "shuffled" else 2)
+    assert ctx.kernel_time("isf_dma")[1] == (2 if kind in ("list", "repeated") else 0)
     assert np.array_equal(out, ctx.isf(q))
     ref = isf_from_rho(lattice_rho(b, n[k][::97], L), N)
     assert np.abs(out[::97] - ref).max() <= BOUND * M * N
