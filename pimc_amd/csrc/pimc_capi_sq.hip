@@ -402,8 +402,22 @@ void make_rho_plan(const int* n3, int nq, int max_pieces, RhoPlan* P) {
     const int wy = 2 * h[1] + 1, wz = 2 * h[2] + 1;
     const int width = 16 * (h[2] / 16 + 1), blocks = width / 16;
     P->width = width;
-    // modes by (n_x, n_y, n_z) of the half space, rows by (n_x, n_y)
-    P->mode_at.assign((size_t)(h[0] + 1) * wy * wz, -1);
+    // modes by (n_x, n_y, n_z) of the half space, rows by (n_x, n_y): a table of the
+    // box, or, of a large box that the list leaves mostly empty, {place, mode} in an open
+    // hash table of at least two places a q (ten q at |n| <= 40, N = 16 x
+    // 125: S(q) 33.6 -> 25.3 us, F 60.5 -> 51.4)
+    const size_t box = (size_t)(h[0] + 1) * wy * wz;
+    size_t places = 0;   // of the hash table, a power of two; 0: a table of the box
+    if (box > 16384 && box / 8 > (size_t)nq)
+        for (places = 64; places < 2 * (size_t)nq;) places *= 2;
+    P->mode_at.assign(places ? 2 * places : box, -1);
+    auto mode_of = [&](size_t at) -> int& {
+        if (!places) return P->mode_at[at];
+        size_t t = (uint32_t)at * 2654435761u & (places - 1);
+        while (P->mode_at[2 * t] >= 0 && P->mode_at[2 * t] != (int)at) t = (t + 1) & (places - 1);
+        P->mode_at[2 * t] = (int)at;
+        return P->mode_at[2 * t + 1];
+    };
     P->row_at.assign((size_t)(h[0] + 1) * wy, -1);
     P->mode.resize(nq);
     P->first.resize(nq);
@@ -423,7 +437,7 @@ void make_rho_plan(const int* n3, int nq, int max_pieces, RhoPlan* P) {
             nz = -nz;
         }
         const size_t rk = (size_t)nx * wy + (ny + h[1]);
-        int& u = P->mode_at[rk * wz + (nz + h[2])];
+        int& u = mode_of(rk * wz + (nz + h[2]));
         if (u < 0) {
             u = nu++;
             P->first[u] = k;

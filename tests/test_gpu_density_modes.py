@@ -117,6 +117,22 @@ def test_pieces_into_pinned(gpu, kind):
     assert np.abs(out[::97] - ref).max() <= BOUND * M * N
 
 
+@pytest.mark.parametrize("nq", [1, 2, 33, 500, 2500])
+def test_few_q_of_a_large_box(gpu, nq):
+    """Lists that leave their box mostly empty find their modes by a hash table: q, -q and
+    repeats of either, up to a table half full, against FP64 phasors and each other."""
+    N, M = 20, 3
+    ctx, b, L = _context(gpu, N, M)
+    rng = np.random.default_rng(nq)
+    n = rng.integers(-40, 41, size=(nq, 3))
+    n[0] = (40, 40, 40)
+    s, f = _check(ctx, b, L, n, N, M)
+    k = rng.integers(0, nq, 4 * nq)
+    sign = rng.choice([-1, 1], size=(4 * nq, 1))
+    assert np.array_equal(ctx.ssf(_q(n[k] * sign, L)), s[k])
+    assert np.array_equal(ctx.isf(_q(n[k] * sign, L)), f[k])
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 7, 8, 9, 64, 126, 127, 128, 129, 511, 512])
 def test_lags_and_parts(gpu, M):
     """Lags up to M / 2 and their mirror images, and S in eight parts, at every remainder."""
