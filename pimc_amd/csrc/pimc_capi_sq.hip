@@ -381,11 +381,11 @@ int lattice_qs(const double* q, int nq, double L, std::vector<int>& n3, std::vec
 
 // A 16 x 16 block of the matrix form takes the same time whatever it holds (up to
 // 512 modes, both signs of n_z), a mode of the lane form always its own.  Random
-// parts of the 100 401 q at N = 2048 x 250: at 160 modes a block the matrix form
-// took 2.01 ms against 3.68 ms, at 73 2.01 against 1.73, at 25 1.16 against 0.83
-// ms; of the 5377 q at N = 256 x 167: at 97 31.7 against 41.0 us, at 47 29.7
-// against 29.8, at 28 29.9 against 24.8 us.  With a few blocks both are a chain of
-// stages, shorter in the matrix form (one block, 14 modes: 17.7 against 19.4 us).
+// parts of the 100 401 q at N = 2048 x 250: at 133 modes a block the matrix form
+// takes 2.01 ms against 3.40 ms, at 72 1.98 against 2.02, at 42 1.72 against 1.18;
+// of the 5377 q at N = 256 x 167: at 80 30.5 us against 30.9, at 47 30.0 against 27.3,
+// at 29 29.0 against 26.4.  With a few blocks both are a chain of stages (105 modes in
+// five blocks 24.6 us against 24.7).
 constexpr int kModesPerBlock = 72, kFewBlocks = 4;
 
 // Jobs of a piece: those of one workgroup of k_rho_matrix per slice, which at M = 250 is

@@ -141,8 +141,9 @@ __device__ __forceinline__ double2 rho_of_sums(double rc, double rs, double ic, 
 }
 
 // rho_q(m) for lattice q, one lane per q (lane t of a workgroup takes q = base +
-// t + 256 k, k < QPT): the form for short runs and for q lists too sparse for
-// the matrix form below.  q and -q are conjugates, so a q is first turned into
+// t + 256 k, k < QPT): the form for q lists too sparse for the matrix form below and,
+// a lane for every q of the list, of the callers that make no plan (pimc_ssf_noalloc and
+// the server; 4913 q, N = 256 x 167: 164 us a call).  q and -q are conjugates, so a q is first turned into
 // the half space n_x > 0, or n_x = 0 and n_y > 0, ...: the sums, their order
 // (32 beads in FP32, then FP64) and so the bits are those of the matrix form.
 template <int QPT, int H>
@@ -192,12 +193,29 @@ __global__ __launch_bounds__(kRhoThreads) void k_rho_lattice(RhoArgs A) {
         float frc[QPT], frs[QPT], fic[QPT], fis[QPT];
 #pragma unroll
         for (int k = 0; k < QPT; ++k) frc[k] = frs[k] = fic[k] = fis[k] = 0.f;
-        for (int bb = 0; bb < nb; ++bb) {
+        // byte offsets walked bead by bead, the compiler not told how far apart they are:
+        // it would read two beads at once (ds_read2_b64), which keeps the LDS busy four
+        // cycles a value where ds_read_b64 takes some two, and the kernel is bound by that
+        // (9261 q, N = 2048 x 100: 957 -> 769 us)
+        unsigned ox[QPT], oy[QPT], oz[QPT];
+#pragma unroll
+        for (int k = 0; k < QPT; ++k) {
+            ox[k] = sizeof(float2) * (T::X + ix[k]);
+            oy[k] = sizeof(float2) * (T::Y + iy[k]);
+            oz[k] = sizeof(float2) * (T::Z + iz[k]);
+        }
+        auto entry = [&](unsigned& o, unsigned step) {
+            const float2 v = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(ph) + o);
+            o += sizeof(float2) * step;
+            asm("" : "+v"(o));
+            return v;
+        };
+        auto bead = [&]() {
 #pragma unroll
             for (int k = 0; k < QPT; ++k) {
-                const float2 ex = ph[T::X + bb * T::WX + ix[k]];
-                const float2 ey = ph[T::Y + bb * T::WY + iy[k]];
-                const float2 ez = ph[T::Z + bb * T::WZ + iz[k]];
+                const float2 ex = entry(ox[k], T::WX);
+                const float2 ey = entry(oy[k], T::WY);
+                const float2 ez = entry(oz[k], T::WZ);
                 const float xr = fmaf(ex.x, ey.x, -ex.y * ey.y);
                 const float xi = fmaf(ex.x, ey.y, ex.y * ey.x);
                 frc[k] = fmaf(xr, ez.x, frc[k]);
@@ -205,7 +223,15 @@ __global__ __launch_bounds__(kRhoThreads) void k_rho_lattice(RhoArgs A) {
                 fic[k] = fmaf(xi, ez.x, fic[k]);
                 fis[k] = fmaf(xi, ez.y, fis[k]);
             }
+        };
+        int left = nb;
+        for (; left >= 4; left -= 4) {
+            bead();
+            bead();
+            bead();
+            bead();
         }
+        for (; left > 0; --left) bead();
 #pragma unroll
         for (int k = 0; k < QPT; ++k) {
             rc[k] += (double)frc[k];
@@ -240,9 +266,9 @@ __global__ __launch_bounds__(kRhoThreads) void k_rho_lattice(RhoArgs A) {
 // Bound: the FP32 matrix rate (126 TFLOP/s measured here), 128 SIMD cycles per job
 // and four beads; the unit shares the vector unit's multipliers, so the tables, the
 // X Y operands and the FP64 sums (about a third of the time) add to it.  At N = 2048
-// x 250 the 50 201 modes of 100 401 q take 2.0 ms (one lane per q, every q: 17.8
-// ms; one lane per mode 7.8 ms), at N = 256 x 167 the 2689 modes of 5377 q 32 us
-// (103 us; 72 us).  Waves that only make tables beside waves that only sum were
+// x 250 the 50 201 modes of 100 401 q take 2.0 ms (one lane per mode 8.1 ms), at N = 256
+// x 167 the 2689 modes of 5377 q 33 us (57 us).  Waves that only make tables beside
+// waves that only sum were
 // slower (2.8 ms), as were 8 waves to a workgroup (2.9 ms).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRhoWaves = 16;
@@ -549,13 +575,19 @@ __global__ void k_ssf_finish(const double* __restrict__ partial, int nq, int M, 
     sq[qi] = s * inv_n;
 }
 
-// The smallest table size that holds nmax: f(std::integral_constant<int, H>).
-template <typename F>
+// The smallest table size that holds nmax: f(std::integral_constant<int, H>).  FINE: also
+// sizes for |n| <= 20 and 24, with which six and five workgroups of k_rho_lattice fit a CU,
+// four at 32 (3000 q with |n| <= 20, N = 2048 x 100: 479 -> 381 us).
+template <bool FINE, typename F>
 static hipError_t for_table_size(const int nmax[3], F f) {
     const int h = std::max(nmax[0], std::max(nmax[1], nmax[2]));
     if (h <= 4) return f(std::integral_constant<int, 4>{});
     if (h <= 8) return f(std::integral_constant<int, 8>{});
     if (h <= 16) return f(std::integral_constant<int, 16>{});
+    if constexpr (FINE) {
+        if (h <= 20) return f(std::integral_constant<int, 20>{});
+        if (h <= 24) return f(std::integral_constant<int, 24>{});
+    }
     if (h <= 32) return f(std::integral_constant<int, 32>{});
     return f(std::integral_constant<int, 40>{});
 }
@@ -569,7 +601,7 @@ hipError_t launch_rho(bool lattice, hipStream_t st, const RhoArgs& A) {
         int qpt = 4;
         while (qpt > 1 && blocks(qpt) < 2048) qpt >>= 1;
         dim3 g((A.nq + kRhoThreads * qpt - 1) / (kRhoThreads * qpt), A.num_slices), b(kRhoThreads);
-        (void)for_table_size(A.nmax, [&](auto h) {
+        (void)for_table_size<true>(A.nmax, [&](auto h) {
             constexpr int H = decltype(h)::value;
             if (qpt == 4) hipLaunchKernelGGL((k_rho_lattice<4, H>), g, b, 0, st, A);
             else if (qpt == 2) hipLaunchKernelGGL((k_rho_lattice<2, H>), g, b, 0, st, A);
@@ -591,7 +623,7 @@ hipError_t launch_rho_matrix(hipStream_t st, const RhoMatrixArgs& A) {
     // four waves, which share the table passes however few jobs there are
     const int groups = (jobs + kRhoWaves - 1) / kRhoWaves;
     const int waves = std::max(4, (jobs + groups - 1) / groups);
-    const hipError_t e = for_table_size(A.nmax, [&](auto h) {
+    const hipError_t e = for_table_size<false>(A.nmax, [&](auto h) {
         constexpr int H = decltype(h)::value;
         const size_t lds = 3 * sizeof(float2) * Phasors<H>::kEntries;   // at most 126 KB
         static std::atomic<bool> attr_set{false};

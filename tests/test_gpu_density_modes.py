@@ -1,5 +1,5 @@
 """The density modes of a q list in the matrix form (k_rho_matrix) and in the lane
-form (k_rho_lattice) at the edges of both: table sizes (|n| <= 4, 8, 16, 32, 40) and
+form (k_rho_lattice) at the edges of both: table sizes (|n| <= 4, 8, 16, 20, 24, 32, 40) and
 the blocks of 16 rows, 16 columns and 32 beads, permuted and repeated lists, lists
 without their -q, and lists mixed with general q.
 
@@ -59,7 +59,8 @@ def test_bead_counts(gpu, N):
 
 
 @pytest.mark.parametrize("h", [(0, 0, 0), (1, 0, 0), (0, 0, 1), (2, 3, 4), (5, 4, 3), (8, 7, 9), (3, 9, 15),
-                               (2, 2, 16), (4, 2, 17), (1, 1, 31), (1, 2, 33), (40, 1, 1), (1, 40, 2), (2, 1, 40)])
+                               (2, 2, 16), (4, 2, 17), (1, 1, 31), (1, 2, 33), (2, 20, 3), (21, 2, 2),
+                               (3, 3, 24), (25, 1, 2), (40, 1, 1), (1, 40, 2), (2, 1, 40)])
 def test_table_sizes(gpu, h):
     N, M = 37, 4
     ctx, b, L = _context(gpu, N, M)
