@@ -687,12 +687,11 @@ int pimc_ctx_create(const pimc_desc* d, pimc_ctx** out) {
     if ((r = ctx_dalloc(c.get(), &c->d_slices, M))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_walker, 1))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_vslice, M))) return r;
-    if ((r = ctx_dalloc(c.get(), &c->d_out, 32))) return r;
+    if ((r = ctx_dalloc(c.get(), &c->d_ticket, 1))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_hist, 64))) return r;
     if ((r = ctx_dalloc(c.get(), &c->d_kin_partials, 1024))) return r;
     c->cap_stage = std::max<size_t>(3 * (size_t)M * N, 256);
     if ((r = ctx_halloc(c.get(), &c->h_stage, c->cap_stage))) return r;
-    if ((r = ctx_halloc(c.get(), &c->h_out, 64))) return r;
     {
         // small results are written by the kernels straight into host memory
         hipError_t e = hipHostMalloc((void**)&c->h_map,
@@ -713,7 +712,7 @@ int pimc_ctx_create(const pimc_desc* d, pimc_ctx** out) {
     }
     HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_hash, 0xff, sizeof(int) * (size_t)cells * M * N, c->stream));
     HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_numlab, 0, sizeof(int) * (size_t)cells * M, c->stream));
-    HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_out, 0, sizeof(double) * 32, c->stream));
+    HIP_OR_FAIL(c.get(), hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned), c->stream));
     build_grid_nn(c.get());
     HIP_OR_FAIL(c.get(), hipMemcpyAsync(c->d_grid_nn, c->grid_nn.data(), sizeof(int) * c->grid_nn.size(),
                                         hipMemcpyHostToDevice, c->stream));

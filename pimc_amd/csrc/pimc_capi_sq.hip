@@ -546,7 +546,7 @@ int pimc_ssf(pimc_ctx* c, const double* q, int nq, double* sq) {
         if (!mapped && (r = grow(c, &c->d_fqt, &c->cap_fqt, (size_t)P.nu))) return r;
         const unsigned long long seq = ++c->seq;
         c->timed_begin(3);
-        SHIP(c, launch_ssf(c->stream, c->d_rho, P.nu, M, inv_n, mapped ? c->d_map + pimc_ctx::kSqSlot : c->d_fqt, c->d_ticket(),
+        SHIP(c, launch_ssf(c->stream, c->d_rho, P.nu, M, inv_n, mapped ? c->d_map + pimc_ctx::kSqSlot : c->d_fqt, c->d_ticket,
                            mapped ? c->d_done() : nullptr, seq));
         c->timed_end();
         const double* got = c->h_map + pimc_ctx::kSqSlot;
@@ -554,7 +554,7 @@ int pimc_ssf(pimc_ctx* c, const double* q, int nq, double* sq) {
         if (mapped) {
             if (c->wait_done(seq) != 0) {
                 // the arrival counter may have been left part-way
-                (void)hipMemsetAsync(c->d_ticket(), 0, sizeof(unsigned), c->stream);
+                (void)hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned), c->stream);
                 return sfail(c, PIMC_E_HIP, "S(q): completion not published");
             }
         } else {

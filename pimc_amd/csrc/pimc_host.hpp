@@ -95,7 +95,7 @@ struct pimc_ctx {
     int num_cus = 256;
     int device = 0;               // the HIP device current when the context was created
     double* d_vslice = nullptr;
-    double* d_out = nullptr;
+    unsigned* d_ticket = nullptr;   // the arrival counter of the S(q) kernel (zero between calls)
     // mapped, coherent pinned host memory: 64 doubles of small results, then from
     // kSqSlot room for kMappedSq S(q) values
     static constexpr int kSqSlot = 64, kMappedSq = 8192;
@@ -106,8 +106,6 @@ struct pimc_ctx {
     static constexpr int kDoneSlot = 63;
     unsigned long long seq = 0;
     unsigned long long* d_done() { return reinterpret_cast<unsigned long long*>(d_map + kDoneSlot); }
-    // the arrival counter of the S(q) kernel (zero between calls): past d_out's 16
-    unsigned* d_ticket() { return reinterpret_cast<unsigned*>(d_out + 16); }
     int wait_done(unsigned long long s, bool packet = false);   // spin, then fall back to a stream sync
     // the direct Delta V form's per-bead results (mapped, coherent pinned block)
     pimc::VnnDirectOut* h_vdir = nullptr;
@@ -213,7 +211,6 @@ struct pimc_ctx {
     // staging
     double* h_stage = nullptr;    // cap_stage >= 3*M*N doubles, pinned
     size_t cap_stage = 0;
-    double* h_out = nullptr;      // 64 doubles, pinned
     // host mirrors
     std::vector<int> h_nbs;
     std::vector<uint8_t> h_on;

@@ -640,7 +640,8 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_window(const RowTile* __r
 // the per-walker potential action (src/action.cpp:462-469).  One workgroup of
 // 1024 lanes: the partials and the slices' item ranges are first pulled into LDS
 // with every load in flight; then each lane sums the items of one slice in item
-// order, and one wave per walker sums its slices (lanes strided, fixed shuffle
+// order (partials too many for LDS: sixteen lanes a slice, strided, and a shuffle
+// tree), and one wave per walker sums its slices (lanes strided, fixed shuffle
 // tree), so the result depends only on the work list, never on timing.  v_host (or
 // null): mapped host memory, also receives the slice sums and, after them, the
 // slices' gradVSquared.

@@ -11,9 +11,10 @@
 // (O(n_q M^2)) instead of O(n_q M^2 N^2) trigonometric pair terms.
 //
 // Lattice q = (2 pi / L) n: exp(i q.r) = prod_d exp(2 pi i n_d s_d), s_d = x_d / L.
-// Each workgroup stages per-bead axis phasors exp(2 pi i n s_d) in LDS (phase
-// reduced in FP64, FP32 sincospi) and sums X Y Z over the beads with FP32 products
-// and FP64 sums every 32 beads: as real matrix products on the matrix cores for a
+// Each workgroup stages per-bead axis phasors exp(2 pi i n s_d) in LDS (phase in
+// quarter turns reduced in FP64, sine and cosine of the rest as FP32 series, for n < 4
+// and multiples of four; the others one product of those) and sums X Y Z over the beads
+// with FP32 products and FP64 sums every 32 beads: as real matrix products on the matrix cores for a
 // list of q (k_rho_matrix), or one lane per q (k_rho_lattice).  q and -q have
 // conjugate modes and equal S and F, so a list's modes are formed once per pair.
 #include <hip/hip_runtime.h>

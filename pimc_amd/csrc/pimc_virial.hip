@@ -284,9 +284,9 @@ __global__ __launch_bounds__(256) void k_virial_chunk(VirialArgs A, AzizDev az) 
 
 // How k_virial_sym shares the slices' offsets among its workgroups: a slice has
 // `steps` of them, each of weight w (8 where T is needed, 5 elsewhere: about their
-// issue slots), and workgroup g takes the steps that start in its equal share of
-// the total weight.  Every workgroup's share is at least one step.
-// The whole numbers stay far below 2^52 and so their FP64 quotients floor exactly
+// issue slots), and workgroup g takes the steps that end in its equal share of the
+// total weight: one that straddles two shares goes to the later workgroup.  Every
+// workgroup's share is at least one step.  The whole numbers stay far below 2^52 and so their FP64 quotients floor exactly
 // (a 64-bit integer division is a hundred scalar instructions).
 struct SymShare {
     double steps, we, wo, total, wgs;
@@ -317,8 +317,9 @@ struct SymShare {
 // write different tiles of the group's LDS sums, and the rounds are separated by
 // barriers, so every sum has one fixed order.  In the last round of an even number
 // of tiles both waves of a tile pair take half of the offsets.  The groups share out
-// the offsets.  16 waves per CU (126 VGPRs), each workgroup with an equal
-// share of all slices' offsets: with half a slice with T or a whole one without it
+// the offsets; waves beyond the last whole group only help to stage the slice (5 of 8
+// waves work at five tiles, 6 of 8 at three and six, 9 of 16 at nine).  16 waves per CU
+// (126 VGPRs), each workgroup with an equal share of all slices' offsets: with half a slice with T or a whole one without it
 // as the unit, N = 256 and M = 166 took 72 us (two uneven rounds of the CUs).
 // A sum entry is nine doubles (18 banks: the 32 lanes of a half-wave hit 32 different
 // pairs of banks).
@@ -482,7 +483,7 @@ void virial_chunks(VirialArgs* A, int num_cus) {
     }
     A->tiles = std::max(1, (A->nalloc + 63) / 64);
     A->waves = A->tiles <= 8 ? 8 : 16;   // (4 for one to four tiles: no faster, twice the partials)
-    // 16 waves per CU, each at least one step
+    // 16 waves per CU, those that work with at least one step each
     const int64_t steps = (int64_t)A->num_slices * 32 * A->tiles;
     A->wgs = (int)std::max<int64_t>(
         1, std::min<int64_t>(num_cus * (16 / A->waves), steps / (2 * (A->waves / A->tiles))));
