@@ -1,6 +1,6 @@
 // oracle.cpp -- CPU FP64 restatement of pimc's all-bead-pairs hot path.
 //
-// TEST INFRASTRUCTURE ONLY: the checker for libpimc_gpu.so.  Only tests/,
+// TEST INFRASTRUCTURE ONLY: what the tests hold libpimc_gpu.so against.  Only tests/,
 // __graft_entry__.smoke() and bench.py's cpu_baseline leg load this library.
 //
 // Single-threaded FP64, built with -ffp-contract=off so every expression is

@@ -1,7 +1,7 @@
 /*
  * oracle.h -- CPU FP64 restatement of DelMaestroGroup/pimc's all-bead-pairs hot path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker: only the test suite
+ * TEST INFRASTRUCTURE ONLY.  Tests compare against this library: only the test suite
  * (tests/), __graft_entry__.smoke() and the cpu_baseline leg of bench.py may load
  * it.  The product (pimc_amd/, libpimc_gpu.so) never links or calls it, and it is
  * never the thing that is measured as the GPU result.

@@ -1,7 +1,7 @@
 """ctypes binding of the CPU oracle (oracle/_build/liboracle.so).
 
 TEST INFRASTRUCTURE ONLY.  Imported by tests/, __graft_entry__.smoke() and the
-cpu_baseline leg of bench.py, where it is the checker, never the product.
+cpu_baseline leg of bench.py, where it is the oracle, never the product.
 """
 import ctypes as C
 import os
